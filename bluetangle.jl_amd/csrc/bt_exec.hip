@@ -48,25 +48,28 @@ struct BatchArgs {
   unsigned long long* stats;  // passes, rpasses, boundary, draws, overflow, bytes_units*2
   int32_t* err;
   int64_t max_passes;
+  void* mats;         // kMatEntries per workgroup
+  PassResult* res;    // one per workgroup
 };
 
-template <typename R>
+template <typename R, typename O>
 __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_batch(BatchArgs a) {
   constexpr int NT = TileCfg<R>::NT;
   extern __shared__ __align__(16) unsigned char smem[];
   C<R>* tile = (C<R>*)smem;
   __shared__ PassGeom geom;
-  __shared__ C<R> mats[kMatEntries];
+  __shared__ __align__(16) C<R> staged[kStageEntries<R>];
   __shared__ double red[(NT / 64) * kAcc];
   __shared__ double sums[kAcc];
   __shared__ Plan plan;
-  __shared__ PassResult res;
   __shared__ int cmd;
   __shared__ unsigned long long traj_sh;
 
   const uint64_t len = 1ull << a.nbits;
   C<R>* state = (C<R>*)a.states + (uint64_t)blockIdx.x * len;
   bti::Interp* ip = a.interps + blockIdx.x;
+  C<R>* mats = (C<R>*)a.mats + (uint64_t)blockIdx.x * kMatEntries;
+  PassResult* res = a.res + blockIdx.x;  // lane 0's; out of LDS, so that two workgroups fit a CU
   const uint64_t ntiles = 1ull << (a.nbits - (a.T < a.nbits ? a.T : a.nbits));
 
   for (;;) {
@@ -88,7 +91,7 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_batch(Bat
     int fresh = 1;
     for (;;) {
       if (threadIdx.x == 0) {
-        int c = ip->step(&plan, &res);
+        int c = ip->step(&plan, res);
         if (c && ++npass > a.max_passes) {
           ip->err = BT_ERR_STATE;
           c = 0;
@@ -105,10 +108,11 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_batch(Bat
       __syncthreads();
       if (!cmd) break;
       if (threadIdx.x < kAcc) sums[threadIdx.x] = 0.0;
+      stage_ops<R>(geom, mats, staged, threadIdx.x, NT);
       __syncthreads();
-      tile_pass<R, uint32_t>(state, geom, mats, tile, 0, 1, ntiles, red, sums, fresh);
+      tile_pass<R, O>(state, GeomLds(&geom, mats), staged, tile, 0, 1, ntiles, red, sums, fresh);
       if (geom.write) fresh = 0;
-      if (threadIdx.x == 0) to_result(plan, geom.red_swap, sums, &res);
+      if (threadIdx.x == 0) to_result(plan, geom.red_swap, sums, res);
       __syncthreads();
     }
     if (threadIdx.x == 0) {
@@ -135,31 +139,19 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_batch(Bat
 // ---------------------------------------------------------------------------
 // grid pass for one large state (host-driven interpreter)
 // ---------------------------------------------------------------------------
-template <typename R>
-struct GridTable {
-  PassGeom g;
-  C<R> mats[kMatEntries];
-};
-
-// O: offset type of the tile pass (uint32_t up to 2^32 amplitudes)
+// O: type of the per-thread byte offset (narrow_io)
 template <typename R, typename O>
-__global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_grid_pass(C<R>* state, const GridTable<R>* tab, uint64_t ntiles,
+__global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_grid_pass(C<R>* state, const unsigned char* tab, uint64_t ntiles,
                                                               double* part) {
   constexpr int NT = TileCfg<R>::NT;
   extern __shared__ __align__(16) unsigned char smem[];
   C<R>* tile = (C<R>*)smem;
-  __shared__ PassGeom geom;
-  __shared__ C<R> mats[kMatEntries];
+  __shared__ __align__(16) C<R> staged[kStageEntries<R>];
   __shared__ double red[(NT / 64) * kAcc];
   __shared__ double sums[kAcc];
-  load_geom(&tab->g, &geom, threadIdx.x, NT);
-  {
-    const int nm = tab->g.nmats;
-    for (int i = threadIdx.x; i < nm; i += NT) mats[i] = tab->mats[i];
-  }
   if (threadIdx.x < kAcc) sums[threadIdx.x] = 0.0;
-  __syncthreads();
-  tile_pass<R, O>(state, geom, mats, tile, blockIdx.x, gridDim.x, ntiles, red, sums);
+  tile_pass<R, O>(state, GeomConst(tab, sizeof(C<R>)), staged, tile, blockIdx.x, gridDim.x, ntiles,
+                  red, sums);
   if (threadIdx.x < kAcc) part[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = sums[threadIdx.x];
 }
 
@@ -271,9 +263,21 @@ void free_grid_res(GridRes* g) {
   delete g;
 }
 
+static size_t table_max(int prec) { return prec == BT_C64 ? kTableMax<float> : kTableMax<double>; }
+
+static int pass_table(int prec, const Plan& plan, const QOp* slots, int nbits, unsigned char* out, size_t* bytes,
+                      TableHead* head) {
+  return prec == BT_C64 ? build_table<float>(plan, slots, nbits, out, bytes, head)
+                        : build_table<double>(plan, slots, nbits, out, bytes, head);
+}
+
+static bool pass_narrow(int prec, const TableHead& h) {
+  return prec == BT_C64 ? narrow_io<float>(h) : narrow_io<double>(h);
+}
+
 static int grid_res(bt_state_s* s, GridRes** out) {
   if (!s->grid) {
-    const size_t tabsz = s->prec == BT_C64 ? sizeof(GridTable<float>) : sizeof(GridTable<double>);
+    const size_t tabsz = table_max(s->prec);
     const int cus = ctx().cus > 0 ? ctx().cus : 256;
     auto* g = new GridRes();
     bool ok = hipHostMalloc(&g->h_ring, tabsz * kRing) == hipSuccess &&
@@ -314,10 +318,9 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
   ip->outcap = outcap;
   ip->fold = fold;
   ip->tol_exact = s->prec == BT_C64 ? 1e-6 : 1e-12;
-  const size_t tabsz = s->prec == BT_C64 ? sizeof(GridTable<float>) : sizeof(GridTable<double>);
+  const size_t tabsz = table_max(s->prec);
   const uint64_t ntiles = 1ull << (nbits - std::min(T, nbits));
   const unsigned blocks = grid_pass_blocks(ntiles);
-  const size_t lds = (size_t)(1u << std::min(T, nbits)) * s->elem();
   GridRes* gr = nullptr;
   int rc = grid_res(s, &gr);
   if (rc) return rc;
@@ -349,47 +352,21 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
     }
     char* hslot = (char*)h_ring + tabsz * slot;
     char* dslot = (char*)d_ring + tabsz * slot;
-    int grc;
-    if (s->prec == BT_C64) {
-      auto* t = (GridTable<float>*)hslot;
-      grc = build_geom<float>(plan, slots.data(), nbits, &t->g, t->mats);
-      red_swap = t->g.red_swap;
-    } else {
-      auto* t = (GridTable<double>*)hslot;
-      grc = build_geom<double>(plan, slots.data(), nbits, &t->g, t->mats);
-      red_swap = t->g.red_swap;
-    }
+    size_t bytes = 0;
+    TableHead head;
+    const int grc = pass_table(s->prec, plan, slots.data(), nbits, (unsigned char*)hslot, &bytes, &head);
     if (grc) {
       rc = fail(grc, "run_grid: pass geometry");
       break;
     }
-    if (hipMemcpyAsync(dslot, hslot, tabsz, hipMemcpyHostToDevice, s->stream) != hipSuccess) {
+    red_swap = head.red_swap;
+    if (hipMemcpyAsync(dslot, hslot, bytes, hipMemcpyHostToDevice, s->stream) != hipSuccess) {
       rc = fail(BT_ERR_HIP, "run_grid: table copy");
       break;
     }
     (void)hipEventRecord(ev[slot], s->stream);
-    // 32-bit in-tile offsets whenever every tile bit is below 32 (the tile
-    // base, which holds the outside bits, stays 64-bit)
-    const bool narrow = plan.ntile == 0 || plan.tile[plan.ntile - 1] < 32;
-    if (s->prec == BT_C64) {
-      if (narrow)
-        hipLaunchKernelGGL((k_grid_pass<float, uint32_t>), dim3(blocks), dim3(TileCfg<float>::NT), lds, s->stream,
-                           (C<float>*)s->d, (const GridTable<float>*)dslot, ntiles, d_part);
-      else
-        hipLaunchKernelGGL((k_grid_pass<float, uint64_t>), dim3(blocks), dim3(TileCfg<float>::NT), lds, s->stream,
-                           (C<float>*)s->d, (const GridTable<float>*)dslot, ntiles, d_part);
-    } else {
-      if (narrow)
-        hipLaunchKernelGGL((k_grid_pass<double, uint32_t>), dim3(blocks), dim3(TileCfg<double>::NT), lds,
-                           s->stream, (C<double>*)s->d, (const GridTable<double>*)dslot, ntiles, d_part);
-      else
-        hipLaunchKernelGGL((k_grid_pass<double, uint64_t>), dim3(blocks), dim3(TileCfg<double>::NT), lds,
-                           s->stream, (C<double>*)s->d, (const GridTable<double>*)dslot, ntiles, d_part);
-    }
-    if (hipGetLastError() != hipSuccess) {
-      rc = fail(BT_ERR_HIP, "run_grid: pass launch");
-      break;
-    }
+    rc = launch_grid_pass(s, dslot, pass_narrow(s->prec, head), T, d_part);
+    if (rc) break;
     // the host waits for a pass's sums only when a decision needs them or
     // the norm is folded into the next pass (fold = 0, a density matrix:
     // passes follow one another without a round trip)
@@ -428,8 +405,8 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
 
 // Pass tables of a circuit whose pass plan does not depend on reductions
 // (a density matrix: no sampling, no renormalisation, fold = 0), planned on
-// the host once: tables gets npass GridTable entries of tabsz bytes each,
-// narrow[i] whether pass i uses 32-bit in-tile offsets.
+// the host once: tables gets npass packed tables, *tabsz bytes apart,
+// narrow[i] whether pass i's per-thread byte offsets fit 32 bits.
 int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::vector<unsigned char>* tables,
                        std::vector<uint8_t>* narrow, size_t* tabsz) {
   const int nbits = s->nbits;
@@ -438,9 +415,11 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
   bti::Program prog{ch.ops.data(), ch.ntop, ch.pool.data(), ch.chan.data(), ch.chanw.data(), nbits};
   ip->init(prog, slots.data(), T, coalesce_bits(s->prec));
   ip->fold = 0;
-  *tabsz = s->prec == BT_C64 ? sizeof(GridTable<float>) : sizeof(GridTable<double>);
   tables->clear();
   narrow->clear();
+  std::vector<unsigned char> packed, one(table_max(s->prec));
+  std::vector<size_t> size;
+  *tabsz = 16;
   Plan plan;
   PassResult res;
   memset(&res, 0, sizeof res);
@@ -449,18 +428,20 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
   while (ip->step(&plan, &res)) {
     if (plan.red != bti::RED_NONE) return fail(BT_ERR_UNSUPPORTED, "plan_static_passes: a pass needs a reduction");
     if (++npass > max_passes) return fail(BT_ERR_STATE, "plan_static_passes: pass limit exceeded");
-    tables->resize(tables->size() + *tabsz);
-    unsigned char* t = tables->data() + tables->size() - *tabsz;
-    memset(t, 0, *tabsz);
-    const int grc = s->prec == BT_C64
-                        ? build_geom<float>(plan, slots.data(), nbits, &((GridTable<float>*)t)->g, ((GridTable<float>*)t)->mats)
-                        : build_geom<double>(plan, slots.data(), nbits, &((GridTable<double>*)t)->g,
-                                             ((GridTable<double>*)t)->mats);
+    size_t bytes = 0;
+    TableHead head;
+    const int grc = pass_table(s->prec, plan, slots.data(), nbits, one.data(), &bytes, &head);
     if (grc) return fail(grc, "plan_static_passes: pass geometry");
-    narrow->push_back(plan.ntile == 0 || plan.tile[plan.ntile - 1] < 32 ? 1 : 0);
+    packed.insert(packed.end(), one.begin(), one.begin() + (long)bytes);
+    size.push_back(bytes);
+    *tabsz = std::max(*tabsz, (bytes + 15) / 16 * 16);
+    narrow->push_back(pass_narrow(s->prec, head) ? 1 : 0);
     memset(&res, 0, sizeof res);
   }
   if (ip->err) return fail(ip->err, "plan_static_passes: interpreter error (" + std::to_string(ip->err) + ")");
+  tables->assign(*tabsz * size.size(), 0);
+  for (size_t i = 0, at = 0; i < size.size(); at += size[i], i++)
+    memcpy(tables->data() + i * *tabsz, packed.data() + at, size[i]);
   return BT_OK;
 }
 
@@ -474,17 +455,17 @@ int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double
   if (s->prec == BT_C64) {
     if (narrow)
       hipLaunchKernelGGL((k_grid_pass<float, uint32_t>), dim3(blocks), dim3(TileCfg<float>::NT), lds, s->stream,
-                         (C<float>*)s->d, (const GridTable<float>*)dtab, ntiles, d_part);
+                         (C<float>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
     else
       hipLaunchKernelGGL((k_grid_pass<float, uint64_t>), dim3(blocks), dim3(TileCfg<float>::NT), lds, s->stream,
-                         (C<float>*)s->d, (const GridTable<float>*)dtab, ntiles, d_part);
+                         (C<float>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
   } else {
     if (narrow)
       hipLaunchKernelGGL((k_grid_pass<double, uint32_t>), dim3(blocks), dim3(TileCfg<double>::NT), lds, s->stream,
-                         (C<double>*)s->d, (const GridTable<double>*)dtab, ntiles, d_part);
+                         (C<double>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
     else
       hipLaunchKernelGGL((k_grid_pass<double, uint64_t>), dim3(blocks), dim3(TileCfg<double>::NT), lds, s->stream,
-                         (C<double>*)s->d, (const GridTable<double>*)dtab, ntiles, d_part);
+                         (C<double>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
   }
   BT_HIP(hipGetLastError());
   return BT_OK;
@@ -694,6 +675,8 @@ int bt_run_batch_persistent(bt_circuit c, int prec, uint64_t seed, int64_t traj0
   int32_t* d_outs = nullptr;
   int64_t* d_nouts = nullptr;
   double* d_final = nullptr;
+  void* d_mats = nullptr;
+  PassResult* d_res = nullptr;
   hipStream_t st = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   auto cleanup = [&]() {
@@ -706,6 +689,8 @@ int bt_run_batch_persistent(bt_circuit c, int prec, uint64_t seed, int64_t traj0
     if (d_outs) (void)hipFree(d_outs);
     if (d_nouts) (void)hipFree(d_nouts);
     if (d_final) (void)hipFree(d_final);
+    if (d_mats) (void)hipFree(d_mats);
+    if (d_res) (void)hipFree(d_res);
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     if (st) (void)hipStreamDestroy(st);
@@ -719,6 +704,8 @@ int bt_run_batch_persistent(bt_circuit c, int prec, uint64_t seed, int64_t traj0
       hipMalloc((void**)&d_err, sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void**)&d_outs, outs_bytes) != hipSuccess ||
       hipMalloc((void**)&d_nouts, sizeof(int64_t) * ntraj) != hipSuccess ||
+      hipMalloc(&d_mats, elem * kMatEntries * nwg) != hipSuccess ||
+      hipMalloc((void**)&d_res, sizeof(PassResult) * nwg) != hipSuccess ||
       (final_states && hipMalloc((void**)&d_final, sizeof(double) * 2 * len * ntraj) != hipSuccess)) {
     cleanup();
     (void)hipGetLastError();
@@ -752,15 +739,19 @@ int bt_run_batch_persistent(bt_circuit c, int prec, uint64_t seed, int64_t traj0
   a.tol_exact = prec == BT_C64 ? 1e-6 : 1e-12;
   a.stats = d_stats;
   a.err = d_err;
+  a.mats = d_mats;
+  a.res = d_res;
   a.max_passes = 64 + 8 * (int64_t)c->h.ops.size();
   const size_t lds = (size_t)(1u << T) * elem;
   (void)hipEventRecord(e0, st);
   if (prec == BT_C64) {
-    (void)hipFuncSetAttribute((const void*)k_batch<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((k_batch<float>), dim3((unsigned)nwg), dim3(TileCfg<float>::NT), lds, st, a);
+    auto* k = narrow_state<float>(nbits) ? k_batch<float, uint32_t> : k_batch<float, uint64_t>;
+    (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(k, dim3((unsigned)nwg), dim3(TileCfg<float>::NT), lds, st, a);
   } else {
-    (void)hipFuncSetAttribute((const void*)k_batch<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((k_batch<double>), dim3((unsigned)nwg), dim3(TileCfg<double>::NT), lds, st, a);
+    auto* k = narrow_state<double>(nbits) ? k_batch<double, uint32_t> : k_batch<double, uint64_t>;
+    (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(k, dim3((unsigned)nwg), dim3(TileCfg<double>::NT), lds, st, a);
   }
   hipError_t le = hipGetLastError();
   (void)hipEventRecord(e1, st);

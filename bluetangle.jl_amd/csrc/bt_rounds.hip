@@ -51,24 +51,19 @@ struct RoundItem {
   int32_t pad;
 };
 
-// table layout: PassGeom, then int32 nmats (padded to 16 B), then nmats matrix entries
-constexpr size_t kGeomBytes = (sizeof(PassGeom) + 15) / 16 * 16;
-
-
 // One workgroup per `tpb` consecutive tiles of one item (tpb per item, from
 // the item's own size: an item's reductions, summed per workgroup and then
 // over its workgroups in a fixed order, do not depend on what else the
 // launch holds).  nb_uniform != 0: every item has that many workgroups (the
 // block -> item map is a division), else a binary search over the items'
 // first blocks.
-template <typename R>
+template <typename R, typename O>
 __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_round(const RoundItem* items, int nitems, uint32_t nb_uniform,
                                                           const unsigned char* blob, double* part) {
   constexpr int NT = TileCfg<R>::NT;
   extern __shared__ __align__(16) unsigned char smem[];
   C<R>* tile = (C<R>*)smem;
-  __shared__ PassGeom geom;
-  __shared__ C<R> mats[kMatEntries];
+  __shared__ __align__(16) C<R> staged[kStageEntries<R>];
   __shared__ double red[(NT / 64) * kAcc];
   __shared__ double sums[kAcc];
   __shared__ int item_sh;
@@ -90,18 +85,11 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_round(con
   }
   const RoundItem it = items[item];
   const unsigned char* tab = blob + it.table;
-  load_geom((const PassGeom*)tab, &geom, threadIdx.x, NT);
-  {
-    const int nm = *(const int*)(tab + kGeomBytes);
-    const C<R>* m = (const C<R>*)(tab + kGeomBytes + 16);
-    for (int i = threadIdx.x; i < nm; i += NT) mats[i] = m[i];
-  }
   if (threadIdx.x < kAcc) sums[threadIdx.x] = 0.0;
-  __syncthreads();
   const uint32_t local = blockIdx.x - it.block0;
   const uint64_t t0 = (uint64_t)local * it.tpb;
   const uint64_t tend = std::min<uint64_t>((uint64_t)it.ntiles, t0 + it.tpb);
-  tile_pass<R, uint32_t>((C<R>*)it.state, geom, mats, tile, t0, 1, tend, red, sums, it.fresh);
+  tile_pass<R, O>((C<R>*)it.state, GeomConst(tab, sizeof(C<R>)), staged, tile, t0, 1, tend, red, sums, it.fresh);
   if (threadIdx.x < kAcc) part[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = sums[threadIdx.x];
 }
 
@@ -332,27 +320,20 @@ class RoundEngine {
         return;
       }
       j->has_plan = 1;
-      const size_t need = kGeomBytes + 16 + sizeof(C<double>) * kMatEntries;
-      j->table.resize(need);
-      PassGeom* g = (PassGeom*)j->table.data();
-      int nm = 0, grc;
-      if (prec_ == BT_C64) {
-        C<float>* m = (C<float>*)(j->table.data() + kGeomBytes + 16);
-        grc = build_geom<float>(j->plan, j->slots.data(), j->nbits, g, m);
-      } else {
-        C<double>* m = (C<double>*)(j->table.data() + kGeomBytes + 16);
-        grc = build_geom<double>(j->plan, j->slots.data(), j->nbits, g, m);
-      }
+      j->table.resize(prec_ == BT_C64 ? kTableMax<float> : kTableMax<double>);
+      size_t bytes = 0;
+      TableHead head{};
+      const int grc = prec_ == BT_C64
+                          ? build_table<float>(j->plan, j->slots.data(), j->nbits, j->table.data(), &bytes, &head)
+                          : build_table<double>(j->plan, j->slots.data(), j->nbits, j->table.data(), &bytes, &head);
       if (grc) {
         j->err = grc;
         j->done = 1;
         j->has_plan = 0;
         return;
       }
-      j->red_swap = g->red_swap;
-      nm = g->nmats;
-      *(int*)(j->table.data() + kGeomBytes) = nm;
-      j->table.resize(kGeomBytes + 16 + elem() * nm);
+      j->red_swap = head.red_swap;
+      j->table.resize(bytes);
     });
     // 2. pack
     act_.clear();
@@ -390,6 +371,9 @@ class RoundEngine {
       blob += (j->table.size() + 15) / 16 * 16;
     }
     nacc_ = kAccSmall;
+    // one kernel for the whole round: 64-bit offsets if any state needs them
+    bool narrow = true;
+    for (Job* j : act) narrow = narrow && (prec_ == BT_C64 ? narrow_state<float>(j->nbits) : narrow_state<double>(j->nbits));
     for (Job* j : act)
       if (j->plan.red == bti::RED_RHO && j->plan.red_k == 3) nacc_ = kAcc;
     int rc = reserve(blob, act.size(), (uint64_t)blocks * (uint64_t)kAcc);
@@ -404,12 +388,14 @@ class RoundEngine {
     const size_t lds = (size_t)(1ull << maxT) * elem();
     BT_HIP(hipEventRecord(ev_a_, stream_));
     if (prec_ == BT_C64) {
-      (void)hipFuncSetAttribute((const void*)k_round<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      hipLaunchKernelGGL((k_round<float>), dim3(blocks), dim3(TileCfg<float>::NT), lds, stream_, d_items_,
+      auto* k = narrow ? k_round<float, uint32_t> : k_round<float, uint64_t>;
+      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipLaunchKernelGGL(k, dim3(blocks), dim3(TileCfg<float>::NT), lds, stream_, d_items_,
                          (int)items.size(), nb_uniform, (const unsigned char*)d_blob_, d_part_);
     } else {
-      (void)hipFuncSetAttribute((const void*)k_round<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      hipLaunchKernelGGL((k_round<double>), dim3(blocks), dim3(TileCfg<double>::NT), lds, stream_, d_items_,
+      auto* k = narrow ? k_round<double, uint32_t> : k_round<double, uint64_t>;
+      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      hipLaunchKernelGGL(k, dim3(blocks), dim3(TileCfg<double>::NT), lds, stream_, d_items_,
                          (int)items.size(), nb_uniform, (const unsigned char*)d_blob_, d_part_);
     }
     BT_HIP(hipGetLastError());

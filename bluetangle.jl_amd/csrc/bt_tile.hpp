@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <cstring>
 
 #include "bt_internal.hpp"
 #include "bt_interp.hpp"
@@ -35,16 +36,19 @@ constexpr int kMatEntries = bti::Interp::kPassMatEntries;
 // doubles over 2 bits, 64 over 3)
 constexpr int kAcc = 65;
 constexpr int kAccSmall = 17;  // enough unless a pass reduces rho over 3 bits
-constexpr int kRB = 5;     // register bits (most): 32 amplitudes per thread
+constexpr int kRB = 5;     // register bits (most)
+constexpr int kTB = 8;     // thread bits (most)
 constexpr int kMaxPh = 28;
 
-// 256 threads per workgroup; complex64 keeps 32 amplitudes per thread (T =
-// 13), complex128 16 (T = 12): 64 KiB tiles, registers <= 256 per lane.
+// 256 threads per workgroup; complex64 takes 32 amplitudes per thread in a
+// phase (T = 13), complex128 16 (T = 12): 64 KiB tiles, registers <= 256 per
+// lane, two workgroups per CU.  Measured at 2^22 amplitudes x 256 noisy
+// trajectories (32 layers): this 320 ms; 512 threads x 16 amplitudes at 128
+// registers 341 ms; 512 x 32 on 2^14-amplitude tiles (one workgroup per CU)
+// 314 ms there but 22.0 ms against 19.6 on a 2^30-amplitude circuit.
 template <typename R>
 struct TileCfg;
-// WAVES: waves per SIMD the kernels are compiled for (launch-bounds
-// minimum): complex64 runs two 64 KiB-tile workgroups per CU (registers
-// <= 256), complex128 one (its tile + matrices exceed half the LDS).
+// WAVES: waves per SIMD the kernels are compiled for (launch-bounds minimum).
 template <>
 struct TileCfg<float> {
   static constexpr int NT = 256;
@@ -57,7 +61,7 @@ struct TileCfg<double> {
   static constexpr int NT = 256;
   static constexpr int LOGNT = 8;
   static constexpr int RB = 4;
-  static constexpr int WAVES = 1;
+  static constexpr int WAVES = 2;
 };
 
 // An operator of a pass.  k <= 2: applied in registers, `mask` = register
@@ -69,6 +73,7 @@ struct ROp {
   int32_t k;
   int32_t mask;
   int32_t moff;
+  int32_t stage;       // offset in the workgroup's staged operators (complex entries)
   int32_t lsorted[4];  // k >= 3: ascending local bits
   uint32_t loff[16];   // k >= 3: local offset of each matrix index
   uint64_t gctrl;      // control bits outside the tile (global positions)
@@ -78,7 +83,7 @@ struct ROp {
 // a swizzled local index and the swizzle is XOR-linear, so the slot of
 // (thread base | register offset) is the XOR of the slots of its bits.
 struct LSlots {
-  uint16_t ts[8];    // slot of thread-index bit i (0 where the thread bit is unused)
+  uint16_t ts[kTB];  // slot of thread-index bit i (0 where the thread bit is unused)
   uint16_t rs[kRB];  // slot of register position j (0 for phantoms)
   uint16_t pad[3];
 };
@@ -102,14 +107,16 @@ struct PhaseTemplate {
 };
 constexpr PhaseTemplate kPhaseTemplates[] = {
     {0, {0, 0, 0, 0}},
+    {3, {0x0c, 0x03, 0x06, 0}},
     {2, {0x0c, 0x03, 0, 0}},
+    {1, {0x03, 0, 0, 0}},
 };
 constexpr int kNumPhaseTemplates = (int)(sizeof(kPhaseTemplates) / sizeof(kPhaseTemplates[0]));
 
 constexpr int kLayIn = kMaxPh, kLayOut = kMaxPh + 1;  // slot tables of the load / store layouts
 
 struct PassGeom {
-  int32_t T, nrb, tb, ncomp, write, need_norm, red, red_k, red_swap, nph, nops, nmats;
+  int32_t T, nrb, tb, ncomp, write, need_norm, red, red_k, red_swap, nph, nops, nmats, nstage;
   int32_t hist_fast;         // RED_HIST with no histogram bit in the store layout's registers
   int32_t tile[bti::kMaxT];  // local bit -> global bit
   int32_t comp[40];          // global bits outside the tile, ascending
@@ -118,12 +125,20 @@ struct PassGeom {
   int32_t red_bits[4];       // RED_HIST: global bits; RED_RHO: register positions (last phase), ascending
   int8_t io_in[kRB], io_out[kRB];
   int8_t pad[6];
-  uint32_t red_loff[8];      // RED_RHO over 3 bits: local offset of each index (red_bits[0] = MSB)
-  int32_t red_ls[4];         // RED_RHO over 3 bits: the three local bits, ascending
+  // the load / store layouts in global bits: thread-index bit i (0 where
+  // unused: that bit of the thread index is never set), register position j
+  // (63 for a phantom: it shifts out of a byte offset)
+  uint8_t thr_in[12], thr_out[12], reg_in[8], reg_out[8];
+  int32_t in_direct, out_direct;  // first phase reads / last phase stores in its own layout
+  int32_t top_thr;                // highest global bit on a thread in either layout
+  int32_t pad2;
+  uint64_t outside;               // global bits outside the tile
+  uint32_t red_loff[8];      // RED_RHO: local offset of each packed index
+  int32_t red_ls[4];         // RED_RHO: the local bits, ascending; RED_HIST: local bit of bin bit j (-1: outside)
   LSlots lay[kMaxPh + 2];    // slot tables: phases, then kLayIn, kLayOut
   double scale;
   RPhase ph[kMaxPh];
-  ROp ops[bti::kPMax];
+  ROp ops[bti::kPMax];  // last: a packed table holds only the used ones
 };
 
 // ---------------------------------------------------------------------------
@@ -161,10 +176,47 @@ __host__ __device__ inline void make_slots(const int8_t* rb, int T, LSlots* s) {
     s->rs[j] = rb[j] >= 0 ? (uint16_t)swz<R>(1u << rb[j]) : (uint16_t)0;
   }
   int i = 0;
-  for (int b = 0; b < T && i < 8; b++)
+  for (int b = 0; b < T && i < kTB; b++)
     if (!((regm >> b) & 1)) s->ts[i++] = (uint16_t)swz<R>(1u << b);
-  for (; i < 8; i++) s->ts[i] = 0;
+  for (; i < kTB; i++) s->ts[i] = 0;
   s->pad[0] = s->pad[1] = s->pad[2] = 0;
+}
+
+// Operators as the workgroup holds them in LDS: a complex64 operator of one or
+// two bits in the lane order of the matrix cores (see op_lane: 16 or 64
+// floats), k >= 3 as complex entries; complex128 reads its k <= 2 matrices
+// from the pass table instead.  Entries are complex numbers of the pass's
+// precision; the most a pass can need follows from its operator and matrix
+// limits (kPMax operators, kMatEntries entries: 20 two-bit, one four-bit and
+// three three-bit operators).
+template <typename R>
+__host__ __device__ constexpr int stage_entries(int k) {
+  return k >= 3 ? 1 << (2 * k) : sizeof(R) == 4 ? 2 << (2 * k) : 0;
+}
+template <typename R>
+constexpr int kStageEntries = sizeof(R) == 4 ? 1088 : kMatEntries;
+
+// Fill the staged form of a pass's operators (entries t, t + step, ... by
+// worker t of `step`).
+template <typename R>
+__host__ __device__ inline void stage_ops(const PassGeom& g, const C<R>* mats, C<R>* out, int t, int step) {
+  for (int o = 0; o < g.nops; o++) {
+    const ROp& op = g.ops[o];
+    const int n = stage_entries<R>(op.k), D = 1 << op.k;
+    for (int e = t; e < n; e += step) {
+      C<R> x;
+      if (op.k >= 3) {
+        x = mats[op.moff + e];
+      } else {
+        // lane i holds, per 4-row slice h, the coefficients of (Re x_c, Im x_c)
+        // in output row 2h + (i >> 1), real part if i is even
+        const int i = e / (n / 4), h = (e % (n / 4)) / D, c = e % D;
+        const C<R> m = mats[op.moff + 2 * h + (i >> 1) + c * D];
+        x = (i & 1) ? cmake<C<R>>(m.y, m.x) : cmake<C<R>>(m.x, -m.y);
+      }
+      out[op.stage + e] = x;
+    }
+  }
 }
 
 template <typename R>
@@ -316,9 +368,8 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     // Register order: a phase with the same bits as the one before keeps its
     // order (no relayout between them).  Otherwise a relayout enters it
     // anyway, so the order is free: an opening pair of disjoint two-bit
-    // operators goes to positions (2,3) then (0,1), the straight-line
-    // template, and a lone opening pair to (1,2), which the per-operator
-    // dispatch tests first.
+    // operators goes to positions (2,3) then (0,1) and a lone opening pair to
+    // (0,1): the straight-line templates.
     if (p > 0 && ph_mask[p] == ph_mask[p - 1]) {
       for (int j = 0; j < kRB; j++) g->ph[p].rb[j] = g->ph[p - 1].rb[j];
       continue;
@@ -341,8 +392,7 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
       put(opm[first[1]]);  // positions 0, 1
       put(opm[first[0]]);  // positions 2, 3
     } else {
-      put(ph_mask[p] & ~opm[first[0]] & (0u - (ph_mask[p] & ~opm[first[0]])));  // lowest other bit: position 0
-      put(opm[first[0]]);                                                       // positions 1, 2
+      put(opm[first[0]]);  // positions 0, 1
     }
     put(ph_mask[p]);  // the rest, ascending
     if (cnt == n) set_layout(g->ph[p].rb, order, n);
@@ -394,7 +444,7 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
   // 4. operators in execution order, in register positions, matrices
   //    permuted to the ascending position convention (index bit j <-> j-th
   //    lowest position)
-  int moff = 0;
+  int moff = 0, nstage = 0;
   g->nops = plan.nops;
   for (int e = 0; e < plan.nops; e++) {
     const int o = exec[e];
@@ -443,6 +493,8 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     const int D = 1 << q.k;
     if (moff + D2 * D2 > kMatEntries) return BT_ERR_UNSUPPORTED;
     r.moff = moff;
+    r.stage = nstage;
+    nstage += stage_entries<R>(k2);
     for (int nr = 0; nr < D2; nr++)
       for (int ncl = 0; ncl < D2; ncl++) {
         // operand-order indices (operand 0 = MSB) of the new indices
@@ -468,6 +520,7 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     moff += D2 * D2;
   }
   g->nmats = moff;
+  g->nstage = nstage;
   // straight-line phase templates
   for (int p = 0; p < nph; p++) {
     RPhase& ph = g->ph[p];
@@ -502,6 +555,33 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     }
     g->scale = 1.0;
   }
+  auto io_bits = [&](const int8_t* rb, uint8_t* thr, uint8_t* reg) {
+    uint32_t regm = 0;
+    for (int j = 0; j < 8; j++) {
+      const bool real = j < kRB && rb[j] >= 0;
+      reg[j] = real ? (uint8_t)plan.tile[rb[j]] : (uint8_t)63;
+      if (real) regm |= 1u << rb[j];
+    }
+    int i = 0;
+    for (int b = 0; b < T && i < 12; b++)
+      if (!((regm >> b) & 1)) thr[i++] = (uint8_t)plan.tile[b];
+    for (; i < 12; i++) thr[i] = 0;
+  };
+  io_bits(g->io_in, g->thr_in, g->reg_in);
+  io_bits(g->io_out, g->thr_out, g->reg_out);
+  g->top_thr = 0;
+  for (int i = 0; i < g->tb && i < 12; i++) {
+    if (g->thr_in[i] > g->top_thr) g->top_thr = g->thr_in[i];
+    if (g->thr_out[i] > g->top_thr) g->top_thr = g->thr_out[i];
+  }
+  g->in_direct = g->out_direct = 1;
+  const int8_t* first_rb = nph > 0 ? g->ph[0].rb : g->io_in;
+  const int8_t* last_rb = nph > 0 ? g->ph[nph - 1].rb : g->io_in;
+  for (int j = 0; j < kRB; j++) {
+    if (g->io_in[j] != first_rb[j]) g->in_direct = 0;
+    if (g->io_out[j] != last_rb[j]) g->out_direct = 0;
+  }
+  g->outside = (nbits < 64 ? (1ull << nbits) - 1ull : ~0ull) & ~tmask;
   for (int p = 0; p < nph; p++) make_slots<R>(g->ph[p].rb, T, &g->lay[p]);
   make_slots<R>(g->io_in, T, &g->lay[kLayIn]);
   make_slots<R>(g->io_out, T, &g->lay[kLayOut]);
@@ -515,17 +595,6 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
         if ((a >> (2 - i)) & 1) off |= 1u << rank[plan.red_bits[i]];
       g->red_loff[a] = off;
     }
-    int ls[3];
-    for (int i = 0; i < 3; i++) ls[i] = rank[plan.red_bits[i]];
-    for (int i = 0; i < 3; i++)
-      for (int j = i + 1; j < 3; j++)
-        if (ls[j] < ls[i]) {
-          const int t = ls[i];
-          ls[i] = ls[j];
-          ls[j] = t;
-        }
-    for (int i = 0; i < 3; i++) g->red_ls[i] = ls[i];
-    g->red_ls[3] = 0;
   } else if (plan.red == bti::RED_RHO) {
     const RPhase& ph = g->ph[nph - 1];
     int p[2] = {0, 0};
@@ -541,8 +610,68 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
       // position); the plan wants red_bits[0] as the MSB
       g->red_swap = p[0] < p[1] ? 1 : 0;
     }
+    for (int a = 0; a < (1 << plan.red_k); a++) {
+      uint32_t off = 0;
+      for (int j = 0; j < plan.red_k; j++)
+        if ((a >> j) & 1) off |= 1u << ph.rb[g->red_bits[j]];
+      g->red_loff[a] = off;
+    }
+  }
+  if (plan.red == bti::RED_RHO) {
+    int n = 0;
+    for (int b = 0; b < T; b++)
+      for (int i = 0; i < plan.red_k; i++)
+        if (rank[plan.red_bits[i]] == b) g->red_ls[n++] = b;
+  } else if (plan.red == bti::RED_HIST) {  // local bits (-1: outside the tile)
+    for (int i = 0; i < plan.red_k; i++) g->red_ls[i] = rank[plan.red_bits[i]];
   }
   return BT_OK;
+}
+
+// A pass's table as the launched executors read it: the geometry up to its
+// last used operator, the staged operators, and in complex128 the matrices
+// (complex64 needs them in staged form only).
+inline size_t geom_bytes(int nops) { return (offsetof(PassGeom, ops) + (size_t)nops * sizeof(ROp) + 15) / 16 * 16; }
+template <typename R>
+constexpr size_t kTableMax =
+    (sizeof(PassGeom) + 15) / 16 * 16 + sizeof(C<R>) * (kStageEntries<R> + (sizeof(R) == 8 ? kMatEntries : 0));
+
+// Build a pass's table in `out` (kTableMax<R> bytes, 16-byte aligned);
+// *bytes: its size.  *head (nullable): a copy of what the host needs of it.
+struct TableHead {
+  int32_t red_swap, top_thr;
+};
+template <typename R>
+inline int build_table(const Plan& plan, const QOp* slots, int nbits, unsigned char* out, size_t* bytes,
+                       TableHead* head) {
+  C<R> mats[kMatEntries];
+  PassGeom* g = (PassGeom*)out;
+  const int rc = build_geom<R>(plan, slots, nbits, g, mats);
+  if (rc) return rc;
+  size_t n = geom_bytes(g->nops);
+  C<R> staged[kStageEntries<R>];
+  stage_ops<R>(*g, mats, staged, 0, 1);
+  memcpy(out + n, staged, sizeof(C<R>) * (size_t)g->nstage);
+  n += sizeof(C<R>) * (size_t)g->nstage;
+  if (sizeof(R) == 8) {
+    memcpy(out + n, mats, sizeof(C<R>) * (size_t)g->nmats);
+    n += sizeof(C<R>) * (size_t)g->nmats;
+  }
+  *bytes = n;
+  if (head) *head = TableHead{g->red_swap, g->top_thr};
+  return BT_OK;
+}
+
+// Whether a pass's per-thread byte offsets fit 32 bits (then every access is a
+// scalar base plus a 32-bit offset per lane), and whether every pass of a
+// state of nbits index bits does.
+template <typename R>
+inline bool narrow_io(const TableHead& h) {
+  return h.top_thr + (sizeof(C<R>) == 8 ? 3 : 4) < 32;
+}
+template <typename R>
+inline bool narrow_state(int nbits) {
+  return nbits + (sizeof(C<R>) == 8 ? 3 : 4) <= 32;
 }
 
 // ---------------------------------------------------------------------------
@@ -586,110 +715,14 @@ __host__ __device__ __forceinline__ void apply_reg(C<R>* v, const C<R>* mats) {
   }
 }
 
-#if defined(__HIP_DEVICE_COMPILE__)
-typedef float floatx4_t __attribute__((ext_vector_type(4)));
-
-// The same operator on a complex64 tile, on the FP32 matrix cores.
-// v_mfma_f32_4x4x1f32 is 16 blocks of 4 x 4 x 1 products: lane l (block
-// b = l / 4) gets D[i] += A(lane 4b + i) * B(lane l), i = 0..3.  With B = one
-// real input of lane l's own group and A(lane 4b + i) = the operator's real
-// form at output row i of a 4-row slice, every lane computes 4 real outputs
-// of its own group from its own inputs: nothing moves between lanes, and the
-// 2^K x 2^K complex product (2^(K+1) real inputs) costs 2^(K+1) instructions
-// per 4 outputs, at twice the FP32 rate of the vector FMAs and beside them.
-// Output slice h holds rows 2h, 2h + 1 of the complex matrix as
-// (Re y_2h, Im y_2h, Re y_2h+1, Im y_2h+1); the lane with l % 4 = i holds
-// the slice's row 2h + (i >> 1), real part if i is even, else imaginary,
-// against the inputs (Re x_c, Im x_c): (Mr, -Mi) for a real part, (Mi, Mr)
-// for an imaginary one.
-template <int MASK>
-__device__ __forceinline__ void apply_reg_mfma(C<float>* v, const C<float>* mats) {
-  constexpr int K = __builtin_popcount(MASK);
-  static_assert(K == 1 || K == 2, "matrix-core register operators cover one and two bits");
-  constexpr int D = 1 << K, NS = D / 2;
-  constexpr int NR = 1 << kRB;
-  int P[K];
-  {
-    int c = 0;
-#pragma unroll
-    for (int j = 0; j < kRB; j++)
-      if ((MASK >> j) & 1) P[c++] = j;
-  }
-  const int i = threadIdx.x & 3;
-  const bool imag = (i & 1) != 0;
-  float a[NS][2 * D];
-#pragma unroll
-  for (int h = 0; h < NS; h++) {
-    const int r = 2 * h + (i >> 1);
-#pragma unroll
-    for (int c = 0; c < D; c++) {
-      const C<float> m = mats[r + c * D];
-      a[h][2 * c] = imag ? m.y : m.x;
-      a[h][2 * c + 1] = imag ? m.x : -m.y;
-    }
-  }
-#pragma unroll
-  for (int base = 0; base < NR; base++) {
-    if (base & MASK) continue;
-    C<float> x[D];
-    int idx[D];
-#pragma unroll
-    for (int l = 0; l < D; l++) {
-      idx[l] = base;
-#pragma unroll
-      for (int j = 0; j < K; j++)
-        if ((l >> j) & 1) idx[l] |= 1 << P[j];
-      x[l] = v[idx[l]];
-    }
-#pragma unroll
-    for (int h = 0; h < NS; h++) {
-      floatx4_t d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int c = 0; c < D; c++) {
-        d = __builtin_amdgcn_mfma_f32_4x4x1f32(a[h][2 * c], x[c].x, d, 0, 0, 0);
-        d = __builtin_amdgcn_mfma_f32_4x4x1f32(a[h][2 * c + 1], x[c].y, d, 0, 0, 0);
-      }
-      v[idx[2 * h]] = cmake<C<float>>(d[0], d[1]);
-      v[idx[2 * h + 1]] = cmake<C<float>>(d[2], d[3]);
-    }
-  }
-}
-#endif
-
-// Register operator with the mask a compile-time constant: complex64 on the
-// device runs on the matrix cores, everything else (complex128, the host
-// emulation) as vector FMAs.
-template <typename R, int MASK>
-__host__ __device__ __forceinline__ void apply_regk(C<R>* v, const C<R>* m) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (sizeof(R) == 4) {
-    apply_reg_mfma<MASK>(v, m);
-    return;
-  }
-#endif
-  apply_reg<R, MASK>(v, m);
-}
-
 template <typename R>
 __host__ __device__ __forceinline__ void apply_mask(int mask, C<R>* v, const C<R>* m) {
-  // adjacent register pairs are the common case (brickwork pairs after the
-  // phase planner): test them first, every level of the dispatch costs moves
-  if (__builtin_expect(mask == 0x06, 1)) {
-    apply_regk<R, 0x06>(v, m);
-    return;
-  }
-  if constexpr (TileCfg<R>::RB == 5) {
-    if (__builtin_expect(mask == 0x18, 1)) {
-      apply_regk<R, 0x18>(v, m);
-      return;
-    }
-  }
   switch (mask) {
 #define BT_CASE(M) \
-  case M: apply_regk<R, M>(v, m); break;
+  case M: apply_reg<R, M>(v, m); break;
 #define BT_CASE5(M)                                   \
   case M:                                             \
-    if constexpr (TileCfg<R>::RB == 5) apply_regk<R, M>(v, m); \
+    if constexpr (TileCfg<R>::RB == 5) apply_reg<R, M>(v, m); \
     break;
     BT_CASE(1) BT_CASE(2) BT_CASE(4) BT_CASE(8) BT_CASE(3) BT_CASE(5) BT_CASE(6) BT_CASE(9) BT_CASE(10) BT_CASE(12)
     BT_CASE5(16) BT_CASE5(17) BT_CASE5(18) BT_CASE5(20) BT_CASE5(24)
@@ -701,24 +734,24 @@ __host__ __device__ __forceinline__ void apply_mask(int mask, C<R>* v, const C<R
 
 // A matched phase template: the operators' register applications in order,
 // straight-line (the masks are compile-time constants of each case).
-// Keeps the next operator's matrix loads from being hoisted above this
-// operator (all of a template's matrices live at once would spill).
-__host__ __device__ __forceinline__ void op_fence() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("" ::: "memory");
-#endif
-}
-
-// A matched phase template: the operators' register applications in order,
-// straight-line (the masks are compile-time constants of each case).
 template <typename R>
 __host__ __device__ __forceinline__ void apply_template(int tm, C<R>* v, const C<R>* mats, const ROp* ops) {
-#define BT_A(M, I)                              \
-  apply_regk<R, M>(v, mats + ops[I].moff); \
-  op_fence();
-  if (tm == 1) {
-    BT_A(0x0c, 0)
-    BT_A(0x03, 1)
+#define BT_A(M, I) apply_reg<R, M>(v, mats + ops[I].moff);
+  switch (tm) {
+    case 1:
+      BT_A(0x0c, 0)
+      BT_A(0x03, 1)
+      BT_A(0x06, 2)
+      break;
+    case 2:
+      BT_A(0x0c, 0)
+      BT_A(0x03, 1)
+      break;
+    case 3:
+      BT_A(0x03, 0)
+      break;
+    default:
+      break;
   }
 #undef BT_A
 }
@@ -808,41 +841,53 @@ __host__ __device__ __forceinline__ void apply_lds(C<R>* lds, int T, const ROp& 
   }
 }
 
-// Reduced rho over three tile bits, read from the tile image in LDS
-// (swizzled): thread tid takes packed entry e = tid / 4 (the 8 diagonal
-// entries, then the 28 pairs a < b in order (0,1), (0,2), ..., (6,7)) and the
-// index groups tid % 4, tid % 4 + 4, ...; returns e (-1: no entry) and the
-// thread's partial sum of Re (xr) and Im (xi) of rho[a, b].
-template <typename R>
-__host__ __device__ __forceinline__ int rho3_partial(const C<R>* lds, const PassGeom& g, uint32_t tid, double* xr,
-                                                     double* xi) {
-  const int e = (int)(tid >> 2), s = (int)(tid & 3);
-  *xr = 0.0;
-  *xi = 0.0;
-  if (e >= 36) return -1;
-  int a = e, b = e;
-  if (e >= 8) {
-    int p = e - 8;
-    a = 0;
-    while (p >= 7 - a) {
-      p -= 7 - a;
-      a++;
-    }
-    b = a + 1 + p;
+// Indices a <= b of packed entry e < 36 of a reduced rho over three bits: the 8
+// diagonal entries, then the 28 pairs a < b in order (0,1), (0,2), ..., (6,7).
+__host__ __device__ __forceinline__ void rho3_pair(int e, int* a, int* b) {
+  *a = *b = e;
+  if (e < 8) return;
+  int p = e - 8, x = 0;
+  while (p >= 7 - x) {
+    p -= 7 - x;
+    x++;
   }
-  const uint32_t oa = g.red_loff[a], ob = g.red_loff[b];
-  const uint32_t ng = 1u << (g.T - 3);
+  *a = x;
+  *b = x + 1 + p;
+}
+
+// Sum over the index groups s, s + 4, ... of the tile image in LDS
+// (swizzled): Re (xr) and Im (xi) of rho[a, b], oa / ob the local offsets of
+// indices a and b, ls the three local bits, ascending.
+template <typename R>
+__host__ __device__ __forceinline__ void rho3_sum(const C<R>* lds, int T, uint32_t oa, uint32_t ob, const int* ls,
+                                                  uint32_t s, double* xr, double* xi) {
+  const uint32_t ng = 1u << (T - 3);
   double sr = 0.0, si = 0.0;
-  for (uint32_t grp = (uint32_t)s; grp < ng; grp += 4) {
+  for (uint32_t grp = s; grp < ng; grp += 4) {
     uint32_t lb = grp;
 #pragma unroll
-    for (int i = 0; i < 3; i++) lb = ((lb >> g.red_ls[i]) << (g.red_ls[i] + 1)) | (lb & ((1u << g.red_ls[i]) - 1u));
+    for (int i = 0; i < 3; i++) lb = ins0(lb, ls[i]);
     const C<R> va = lds[swz<R>(lb + oa)], vb = lds[swz<R>(lb + ob)];
     sr += (double)va.x * (double)vb.x + (double)va.y * (double)vb.y;
     si += (double)va.y * (double)vb.x - (double)va.x * (double)vb.y;
   }
   *xr = sr;
   *xi = si;
+}
+
+// Reduced rho over three tile bits: thread tid takes packed entry e = tid / 4
+// and the index groups tid % 4, tid % 4 + 4, ...; returns e (-1: no entry)
+// and the thread's partial sums.
+template <typename R>
+__host__ __device__ __forceinline__ int rho3_partial(const C<R>* lds, const PassGeom& g, uint32_t tid, double* xr,
+                                                     double* xi) {
+  const int e = (int)(tid >> 2);
+  *xr = 0.0;
+  *xi = 0.0;
+  if (e >= 36) return -1;
+  int a, b;
+  rho3_pair(e, &a, &b);
+  rho3_sum<R>(lds, g.T, g.red_loff[a], g.red_loff[b], g.red_ls, tid & 3, xr, xi);
   return e;
 }
 
@@ -879,37 +924,12 @@ __device__ __forceinline__ double wave_sum(double x) {
   return (readlane_f64(x, 0) + readlane_f64(x, 16)) + (readlane_f64(x, 32) + readlane_f64(x, 48));
 }
 
-// The quad's four partials of a 3-bit reduced-rho entry, summed in a fixed
-// order ((s0 + s1) + (s2 + s3)), added by the quad's first lane to its
-// wavefront's packed-rho slots (wrho: LDS; each entry has one writer).
-template <typename R>
-__device__ __forceinline__ void rho3_accumulate_t(const C<R>* lds, const PassGeom& g, double* wrho) {
-  double xr, xi;
-  const int e = rho3_partial<R>(lds, g, threadIdx.x, &xr, &xi);
-  xr += dpp_f64<0xb1>(xr);
-  xr += dpp_f64<0x4e>(xr);
-  xi += dpp_f64<0xb1>(xi);
-  xi += dpp_f64<0x4e>(xi);
-  if (e >= 0 && (threadIdx.x & 3) == 0) {
-    const int sl = rho3_slot(e);
-    wrho[sl] += xr;
-    if (e >= 8) wrho[sl + 1] += xi;
-  }
-}
-
-// Add M per-thread values into this wavefront's accumulator slots
-// (wred[0..M), LDS): one writer lane, tiles in order, no barrier.
-template <int M>
-__device__ __forceinline__ void wave_accumulate(const double* v, double* wred) {
-  const bool lead = (threadIdx.x & 63) == 0;
-#pragma unroll
-  for (int j = 0; j < M; j++) {
-    const double t = wave_sum(v[j]);
-    if (lead) wred[j] += t;
-  }
-}
 #endif
 
+// ---------------------------------------------------------------------------
+// One thread's part of a pass, as the host emulation steps through it; the
+// device's own forms of these steps are in the "device pass" section below.
+// ---------------------------------------------------------------------------
 // Local index of thread t's register r under a layout: thread bits are the
 // local bits not in registers, ascending, holding t's bits in order.
 __host__ __device__ __forceinline__ uint32_t thread_base(const int8_t* rb, int T, uint32_t t) {
@@ -927,22 +947,12 @@ __host__ __device__ __forceinline__ uint32_t thread_base(const int8_t* rb, int T
   return base;
 }
 
-// A value the whole workgroup holds in common, moved to a scalar register
-// on the device (identity on the host).
-__host__ __device__ __forceinline__ uint32_t uni32(uint32_t x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_readfirstlane(x);
-#else
-  return x;
-#endif
-}
-
 // Slot of thread tid's register 0 under a layout (XOR of its bits' slots).
 __host__ __device__ __forceinline__ uint32_t slot_base(const LSlots& s, uint32_t tid) {
   uint32_t b = 0;
 #pragma unroll
-  for (int i = 0; i < 8; i++)
-    if ((tid >> i) & 1) b ^= uni32(s.ts[i]);
+  for (int i = 0; i < kTB; i++)
+    if ((tid >> i) & 1) b ^= s.ts[i];
   return b;
 }
 
@@ -951,7 +961,7 @@ __host__ __device__ __forceinline__ uint32_t reg_slot(const LSlots& s, int r) {
   uint32_t u = 0;
 #pragma unroll
   for (int j = 0; j < kRB; j++)
-    if ((r >> j) & 1) u ^= uni32(s.rs[j]);
+    if ((r >> j) & 1) u ^= s.rs[j];
   return u;
 }
 
@@ -1028,75 +1038,6 @@ __host__ __device__ __forceinline__ void opaque(T& x) {
 #endif
 }
 
-// The same for a value that is equal in every lane, kept in a scalar
-// register (moved there first: a lane-uniform value the compiler cannot
-// prove uniform would otherwise occupy a vector register per lane).
-template <typename T>
-__host__ __device__ __forceinline__ void opaque_uniform(T& x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (sizeof(T) == 8) {
-    const uint64_t u = (uint64_t)x;
-    x = (T)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32) |
-            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u));
-  } else {
-    x = (T)__builtin_amdgcn_readfirstlane((int)x);
-  }
-  asm volatile("" : "+s"(x));
-#else
-  (void)x;
-#endif
-}
-
-// gin / gout are the same in every lane (pass geometry); gthr_* are per thread.
-template <typename O>
-__host__ __device__ __forceinline__ void opaque_io(ThreadIO<O>& io) {
-#pragma unroll
-  for (int j = 0; j < kRB; j++) {
-    opaque_uniform(io.gin[j]);
-    opaque_uniform(io.gout[j]);
-  }
-  opaque(io.gthr_in);
-  opaque(io.gthr_out);
-}
-
-// State loads and stores on the device go through the global address space
-// (global_load / global_store, counted by vmcnt alone).  Through a generic
-// pointer they compile to flat_* accesses, which also count against lgkmcnt,
-// so every LDS or scalar-load wait in the pass would also wait for the
-// in-flight prefetch of the next tile and the stores of the last one.
-template <typename R>
-__host__ __device__ __forceinline__ C<R> gload(const C<R>* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef R v2 __attribute__((ext_vector_type(2)));  // a builtin vector: no struct copy through a generic pointer
-  const v2 x = *(const __attribute__((address_space(1))) v2*)p;
-  return cmake<C<R>>(x.x, x.y);
-#else
-  return *p;
-#endif
-}
-template <typename R>
-__host__ __device__ __forceinline__ void gstore(C<R>* p, const C<R>& v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef R v2 __attribute__((ext_vector_type(2)));
-  v2 x;
-  x.x = v.x;
-  x.y = v.y;
-  *(__attribute__((address_space(1))) v2*)p = x;
-#else
-  *p = v;
-#endif
-}
-
-// A flag that is the same in every lane (a pass-geometry field), moved to a
-// scalar register so branches on it are scalar branches.
-__host__ __device__ __forceinline__ bool uflag(bool x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_readfirstlane((int)x) != 0;
-#else
-  return x;
-#endif
-}
-
 // Wait until every vector-memory access this wave issued has completed
 // (s_waitcnt vmcnt(0), the LDS and export counters left alone).
 __host__ __device__ __forceinline__ void vm_wait_all() {
@@ -1131,7 +1072,7 @@ __host__ __device__ __forceinline__ void fetch_regs(C<R>* raw, const C<R>* __res
 #pragma unroll
     for (int j = 0; j < kRB; j++)
       if ((r >> j) & 1) off |= io.gin[j];
-    raw[r] = gload<R>(tp + off);
+    raw[r] = tp[off];
   }
 }
 
@@ -1173,8 +1114,8 @@ __host__ __device__ __forceinline__ void store_regs(const C<R>* v, C<R>* __restr
                                                     const ThreadIO<O>& io, uint64_t base, double* acc) {
   constexpr int NR = 1 << TileCfg<R>::RB;
   C<R>* __restrict__ tp = state + base;
-  const bool slow_hist = uflag(g.red == bti::RED_HIST && !g.hist_fast);
-  const bool write = uflag(g.write), need_norm = uflag(g.need_norm);
+  const bool slow_hist = g.red == bti::RED_HIST && !g.hist_fast;
+  const bool write = g.write, need_norm = g.need_norm;
   double s = 0.0;
   if (io.active && io.nvalid_mask == 0 && !slow_hist) {  // every register real: no masks
     if (write) {
@@ -1184,7 +1125,7 @@ __host__ __device__ __forceinline__ void store_regs(const C<R>* v, C<R>* __restr
 #pragma unroll
         for (int j = 0; j < kRB; j++)
           if ((r >> j) & 1) off |= io.gout[j];
-        gstore<R>(tp + off, v[r]);
+        tp[off] = v[r];
       }
     }
     if (need_norm) {
@@ -1202,7 +1143,7 @@ __host__ __device__ __forceinline__ void store_regs(const C<R>* v, C<R>* __restr
     for (int j = 0; j < kRB; j++)
       if ((r >> j) & 1) off |= io.gout[j];
     if (io.active && !(r & io.nvalid_mask)) {
-      if (g.write) gstore<R>(tp + off, v[r]);
+      if (g.write) tp[off] = v[r];
       if (g.need_norm) {
         const double w = (double)v[r].x * (double)v[r].x + (double)v[r].y * (double)v[r].y;
         s += w;
@@ -1233,25 +1174,11 @@ __host__ __device__ __forceinline__ int rho_reg_mask(const PassGeom& g) {
 
 #if defined(__HIPCC__)
 // A value the whole workgroup holds in common, moved to scalar registers.
-__device__ __forceinline__ int uniform_i32(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 __device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
   return ((uint64_t)hi << 32) | lo;
-}
-
-// Copy a pass geometry into LDS: the header, the used phases and operators.
-__device__ __forceinline__ void load_geom(const PassGeom* __restrict__ src, PassGeom* dst, int tid, int nt) {
-  constexpr int hdr = (int)(offsetof(PassGeom, ph) / 4);
-  const int nph = src->nph, nops = src->nops;
-  const int* s = (const int*)src;
-  int* d = (int*)dst;
-  const int ph_end = hdr + nph * (int)(sizeof(RPhase) / 4);
-  constexpr int ops0 = (int)(offsetof(PassGeom, ops) / 4);
-  const int ops_end = ops0 + nops * (int)(sizeof(ROp) / 4);
-  for (int i = tid; i < ph_end; i += nt) d[i] = s[i];
-  for (int i = ops0 + tid; i < ops_end; i += nt) d[i] = s[i];
 }
 
 // Fixed-order sum of per-workgroup partials laid out accumulator-major
@@ -1269,133 +1196,708 @@ __device__ __forceinline__ double sum_blocks(const double* __restrict__ p, uint3
   return sh[0];
 }
 
+// ---------------------------------------------------------------------------
+// device pass
+// ---------------------------------------------------------------------------
+// Where a pass's table (geometry, matrices) lives.  In the launched executors
+// it is read-only global memory: every field is the same in all lanes, so it
+// is read through the constant address space into scalar registers, costing
+// neither vector instructions nor LDS.  The persistent executor builds its
+// tables on the device, in LDS.
+typedef const __attribute__((address_space(4))) uint32_t* const_words;
+
+struct GeomConst {
+  const_words g, m;
+  const unsigned char* staged;  // the staged operators, 16-byte aligned
+  // a packed table (build_table) of element size `elem`
+  __device__ GeomConst(const unsigned char* tab, int elem) : g((const_words)(uintptr_t)tab) {
+    const uint32_t nops = w(offsetof(PassGeom, nops)), nstage = w(offsetof(PassGeom, nstage));
+    staged = tab + (offsetof(PassGeom, ops) + nops * sizeof(ROp) + 15) / 16 * 16;
+    m = (const_words)(uintptr_t)(staged + nstage * (uint32_t)elem);
+  }
+  __device__ __forceinline__ uint32_t w(size_t byte) const { return g[byte / 4]; }
+  // Touch every 64-byte line of what the pass reads through the scalar cache,
+  // 16 loads in flight at a time, so that no phase waits for memory on its
+  // first use of a line (a complex128 operator's matrix alone is 4 lines: a
+  // one-tile circuit of 120 two-bit operators ran at 328 us without it,
+  // 303 with it).
+  template <typename R>
+  __device__ __forceinline__ void warm() const {
+    const uint32_t head = (uint32_t)(offsetof(PassGeom, ops) + w(offsetof(PassGeom, nops)) * sizeof(ROp));
+    const uint32_t nmat = sizeof(R) == 8 ? w(offsetof(PassGeom, nmats)) * (uint32_t)sizeof(C<R>) : 0u;
+    touch(g, head);
+    touch(m, nmat);
+  }
+  static __device__ __forceinline__ void touch(const_words p, uint32_t bytes) {
+    uint32_t at = 0;
+    for (; at + 1024 <= bytes; at += 1024) {
+      uint32_t x[16];
+#pragma unroll
+      for (int i = 0; i < 16; i++) x[i] = p[at / 4 + 16 * i];
+#pragma unroll
+      for (int i = 0; i < 16; i++) asm volatile("" ::"s"(x[i]));
+    }
+    if (at < bytes) {  // the rest: lines past the end repeat the first one
+      uint32_t x[16];
+#pragma unroll
+      for (int i = 0; i < 16; i++) x[i] = p[at + 64 * i < bytes ? at / 4 + 16 * i : at / 4];
+#pragma unroll
+      for (int i = 0; i < 16; i++) asm volatile("" ::"s"(x[i]));
+    }
+  }
+  __device__ __forceinline__ uint32_t lane_w(size_t byte) const { return g[byte / 4]; }  // a word of each lane's own
+  // The same table through a pointer whose origin is hidden from the
+  // optimiser: what is read through it is not hoisted out of a loop (dozens of
+  // live scalar registers otherwise).
+  __device__ __forceinline__ GeomConst again() const {
+    GeomConst c = *this;
+    uint64_t x = (uint64_t)(uintptr_t)c.g, y = (uint64_t)(uintptr_t)c.m;
+    asm volatile("" : "+s"(x), "+s"(y));
+    c.g = (const_words)(uintptr_t)x;
+    c.m = (const_words)(uintptr_t)y;
+    return c;
+  }
+  template <typename R>
+  __device__ __forceinline__ C<R> mat(int i) const {
+    const auto* p = (const __attribute__((address_space(4))) R*)m;
+    return cmake<C<R>>(p[2 * i], p[2 * i + 1]);
+  }
+};
+
+struct GeomLds {
+  const uint32_t* g;
+  const void* m;
+  const unsigned char* staged = nullptr;  // the caller has filled the staged operators
+  __device__ GeomLds(const PassGeom* geom, const void* mats) : g((const uint32_t*)geom), m(mats) {}
+  __device__ __forceinline__ uint32_t w(size_t byte) const {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)g[byte / 4]);
+  }
+  __device__ __forceinline__ uint32_t lane_w(size_t byte) const { return g[byte / 4]; }
+  __device__ __forceinline__ GeomLds again() const { return *this; }
+  template <typename R>
+  __device__ __forceinline__ void warm() const {}
+  template <typename R>
+  __device__ __forceinline__ C<R> mat(int i) const {
+    return ((const C<R>*)m)[i];
+  }
+};
+
+#define BT_G(field) ((int)geo.w(offsetof(PassGeom, field)))
+#define BT_GOP(o, field) ((int)geo.w(offsetof(PassGeom, ops) + (size_t)(o) * sizeof(ROp) + offsetof(ROp, field)))
+
+static_assert(sizeof(LSlots) == 32 && offsetof(PassGeom, lay) % 4 == 0 && offsetof(PassGeom, thr_in) % 4 == 0 &&
+                  offsetof(PassGeom, ph) % 4 == 0 && offsetof(RPhase, op0) == 8 && sizeof(RPhase) == 16,
+              "the pass reads its table in words");
+
+// A lane-uniform value whose origin is hidden from the optimiser (what is
+// computed from it stays where it is used).
+__device__ __forceinline__ int hide(int x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+
+// A layout's slots in bytes: thread base (per lane) and register positions.
+template <typename R, typename G>
+struct SlotRegs {
+  uint32_t base;      // byte address of this thread's register 0 in the tile image
+  uint32_t rs[TileCfg<R>::RB];
+  __device__ __forceinline__ SlotRegs(const G& geo, int lay, uint32_t tid) {
+    const size_t at = offsetof(PassGeom, lay) + (size_t)lay * sizeof(LSlots);
+    uint32_t w[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) w[i] = geo.w(at + 4 * i);
+    auto half = [&](int i) { return (w[i >> 1] >> (16 * (i & 1))) & 0xffffu; };
+    uint32_t b = 0;
+#pragma unroll
+    for (int i = 0; i < TileCfg<R>::LOGNT; i++) b ^= (0u - ((tid >> i) & 1u)) & half(i);
+    base = b * (uint32_t)sizeof(C<R>);
+#pragma unroll
+    for (int j = 0; j < TileCfg<R>::RB; j++) rs[j] = half(kTB + j) * (uint32_t)sizeof(C<R>);
+  }
+  __device__ __forceinline__ uint32_t at(int r) const {
+    uint32_t u = 0;
+#pragma unroll
+    for (int j = 0; j < TileCfg<R>::RB; j++)
+      if ((r >> j) & 1) u ^= rs[j];
+    return base ^ u;
+  }
+};
+
+template <typename R, typename G>
+__device__ __forceinline__ void image_write(const C<R>* v, C<R>* lds, const G& geo, int lay, uint32_t tid, bool active,
+                                            int nvalid_mask) {
+  constexpr int NR = 1 << TileCfg<R>::RB;
+  const SlotRegs<R, G> S(geo, lay, tid);
+  if (nvalid_mask == 0) {  // every register real
+    if (active) {
+#pragma unroll
+      for (int r = 0; r < NR; r++) *(C<R>*)((char*)lds + S.at(r)) = v[r];
+    }
+  } else {
+    const int nm = hide(nvalid_mask);
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+      if (active && !(r & nm)) *(C<R>*)((char*)lds + S.at(r)) = v[r];
+  }
+}
+
+template <typename R, typename G>
+__device__ __forceinline__ void image_read(C<R>* v, const C<R>* lds, const G& geo, int lay, uint32_t ltid) {
+  constexpr int NR = 1 << TileCfg<R>::RB;
+  const SlotRegs<R, G> S(geo, lay, ltid);
+#pragma unroll
+  for (int r = 0; r < NR; r++) v[r] = *(const C<R>*)((const char*)lds + S.at(r));
+}
+
+// Offsets of a load / store layout: register positions (the same in every
+// lane) and the thread's own part.  O = uint32_t: the thread's byte offset
+// fits 32 bits (every thread bit of the tile below 2^32 bytes), and an access
+// is a scalar base plus that offset.
+template <typename R, typename O>
+struct IoRegs {
+  uint32_t reg[TileCfg<R>::RB];  // global bit of register position j
+  O thr;                         // byte offset of this thread
+  template <typename G>
+  __device__ __forceinline__ IoRegs(const G& geo, size_t thr_at, size_t reg_at, uint32_t tid) {
+    uint32_t w[3], r[2];
+#pragma unroll
+    for (int i = 0; i < 3; i++) w[i] = geo.w(thr_at + 4 * i);
+#pragma unroll
+    for (int i = 0; i < 2; i++) r[i] = geo.w(reg_at + 4 * i);
+#pragma unroll
+    for (int j = 0; j < TileCfg<R>::RB; j++) reg[j] = (r[j >> 2] >> (8 * (j & 3))) & 63u;
+    thr = 0;
+#pragma unroll
+    for (int i = 0; i < TileCfg<R>::LOGNT; i++) {
+      const uint32_t b = (w[i >> 2] >> (8 * (i & 3))) & 63u;
+      thr |= (O)((tid >> i) & 1u) << (b + (sizeof(C<R>) == 8 ? 3 : 4));
+    }
+  }
+  // keep the per-register offsets from being hoisted out of the tile loop
+  __device__ __forceinline__ void again() {
+#pragma unroll
+    for (int j = 0; j < TileCfg<R>::RB; j++) asm volatile("" : "+s"(reg[j]));
+    opaque(thr);
+  }
+  // byte offset of register r: 0 for a phantom position (its bit is 63, which
+  // the shift to bytes drops)
+  __device__ __forceinline__ uint64_t at(int r) const {
+    uint64_t u = 0;
+#pragma unroll
+    for (int j = 0; j < TileCfg<R>::RB; j++)
+      if ((r >> j) & 1) u |= (1ull << reg[j]) * sizeof(C<R>);
+    return u;
+  }
+};
+
+// Address of register r's element: a scalar base (state, tile, register) plus
+// the thread's offset.  The scalar part is hidden from the optimiser, which
+// would otherwise add the thread's offset first and keep a 64-bit vector
+// address per register.
+template <typename R, typename O>
+__device__ __forceinline__ __attribute__((address_space(1))) char* io_addr(const C<R>* tile0, const IoRegs<R, O>& io,
+                                                                          int r) {
+  uint64_t b = (uint64_t)(uintptr_t)tile0 + io.at(r);
+  asm volatile("" : "+s"(b));
+  return (__attribute__((address_space(1))) char*)(uintptr_t)b + io.thr;
+}
+
+// Loads are unconditional and straight-line (phantom registers alias a valid
+// address, inactive threads mirror an active one), so all are in flight at once.
+template <typename R, typename O>
+__device__ __forceinline__ void pass_fetch(C<R>* raw, const C<R>* __restrict__ state, const IoRegs<R, O>& io,
+                                           uint64_t base) {
+  constexpr int NR = 1 << TileCfg<R>::RB;
+  typedef R v2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int r = 0; r < NR; r++) {
+    const v2 x = *(const __attribute__((address_space(1))) v2*)io_addr<R, O>(state + base, io, r);
+    raw[r] = cmake<C<R>>(x.x, x.y);
+  }
+}
+
+template <typename R, typename O>
+__device__ __forceinline__ void pass_store(const C<R>* v, C<R>* __restrict__ state, const IoRegs<R, O>& io,
+                                           uint64_t base, bool active, int nvalid_mask) {
+  constexpr int NR = 1 << TileCfg<R>::RB;
+  typedef R v2 __attribute__((ext_vector_type(2)));
+  auto put = [&](int r) {
+    v2 x;
+    x.x = v[r].x;
+    x.y = v[r].y;
+    *(__attribute__((address_space(1))) v2*)io_addr<R, O>(state + base, io, r) = x;
+  };
+  if (nvalid_mask == 0) {
+    if (active) {
+#pragma unroll
+      for (int r = 0; r < NR; r++) put(r);
+    }
+  } else {
+    const int nm = hide(nvalid_mask);
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+      if (active && !(r & nm)) put(r);
+  }
+}
+
+// ---- operators ------------------------------------------------------------
+// complex64: the FP32 matrix cores.  v_mfma_f32_4x4x1f32 is 16 blocks of
+// 4 x 4 x 1 products: lane l (block b = l / 4) gets D[i] += A(lane 4b + i) *
+// B(lane l), i = 0..3.  With B = one real input of lane l's own group and
+// A(lane 4b + i) = the operator's real form at output row i of a 4-row slice,
+// every lane computes 4 real outputs of its own group from its own inputs:
+// nothing moves between lanes, and the 2^K x 2^K complex product (2^(K+1)
+// real inputs) costs 2^(K+1) instructions per 4 outputs, at twice the FP32
+// rate of the vector FMAs and beside them.  Output slice h holds rows 2h,
+// 2h + 1 of the complex matrix as (Re y_2h, Im y_2h, Re y_2h+1, Im y_2h+1);
+// the lane with l % 4 = i holds the slice's row 2h + (i >> 1), real part if i
+// is even, else imaginary, against the inputs (Re x_c, Im x_c): (Mr, -Mi)
+// for a real part, (Mi, Mr) for an imaginary one.  The operators are staged in
+// LDS in that lane order (stage_ops), so a lane reads its 16 coefficients
+// with four 16-byte LDS reads.
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+
+template <int MASK>
+__device__ __forceinline__ void op_lane(C<float>* v, const C<float>* staged) {
+  constexpr int K = __builtin_popcount(MASK);
+  static_assert(K == 1 || K == 2, "matrix-core register operators cover one and two bits");
+  constexpr int D = 1 << K, NS = D / 2;
+  constexpr int NR = 1 << TileCfg<float>::RB;
+  int P[K];
+  {
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < kRB; j++)
+      if ((MASK >> j) & 1) P[c++] = j;
+  }
+  const float4* ap = (const float4*)(staged + 2 * D * NS / 2 * (threadIdx.x & 3));
+  float a[NS][2 * D];
+#pragma unroll
+  for (int h = 0; h < NS; h++)
+#pragma unroll
+    for (int q = 0; q < D / 2; q++) {
+      const float4 w = ap[2 * h + q];
+      a[h][4 * q] = w.x;
+      a[h][4 * q + 1] = w.y;
+      a[h][4 * q + 2] = w.z;
+      a[h][4 * q + 3] = w.w;
+    }
+#pragma unroll
+  for (int base = 0; base < NR; base++) {
+    if (base & MASK) continue;
+    C<float> x[D];
+    int idx[D];
+#pragma unroll
+    for (int l = 0; l < D; l++) {
+      idx[l] = base;
+#pragma unroll
+      for (int j = 0; j < K; j++)
+        if ((l >> j) & 1) idx[l] |= 1 << P[j];
+      x[l] = v[idx[l]];
+    }
+#pragma unroll
+    for (int h = 0; h < NS; h++) {
+      floatx4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < D; c++) {
+        d = __builtin_amdgcn_mfma_f32_4x4x1f32(a[h][2 * c], x[c].x, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_4x4x1f32(a[h][2 * c + 1], x[c].y, d, 0, 0, 0);
+      }
+      v[idx[2 * h]] = cmake<C<float>>(d[0], d[1]);
+      v[idx[2 * h + 1]] = cmake<C<float>>(d[2], d[3]);
+    }
+  }
+}
+
+// complex128: vector FMAs, the matrix entries from the pass table (scalar
+// registers where the table is in the constant address space).
+template <int MASK, typename G>
+__device__ __forceinline__ void op_fma(C<double>* v, const G& geo, int moff) {
+  constexpr int K = __builtin_popcount(MASK);
+  constexpr int D = 1 << K;
+  constexpr int NR = 1 << TileCfg<double>::RB;
+  int P[K];
+  {
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < kRB; j++)
+      if ((MASK >> j) & 1) P[c++] = j;
+  }
+  C<double> m[D * D];
+#pragma unroll
+  for (int i = 0; i < D * D; i++) m[i] = geo.template mat<double>(moff + i);
+#pragma unroll
+  for (int base = 0; base < NR; base++) {
+    if (base & MASK) continue;
+    C<double> x[D];
+    int idx[D];
+#pragma unroll
+    for (int l = 0; l < D; l++) {
+      idx[l] = base;
+#pragma unroll
+      for (int j = 0; j < K; j++)
+        if ((l >> j) & 1) idx[l] |= 1 << P[j];
+      x[l] = v[idx[l]];
+    }
+#pragma unroll
+    for (int r = 0; r < D; r++) {
+      C<double> acc = cmake<C<double>>(0, 0);
+#pragma unroll
+      for (int c = 0; c < D; c++) acc = cfma(acc, m[r + c * D], x[c]);
+      v[idx[r]] = acc;
+    }
+  }
+}
+
+// Operator o of the pass on the register positions MASK.
+template <typename R, int MASK, typename G>
+__device__ __forceinline__ void op_reg(C<R>* v, const G& geo, int o, const C<R>* staged) {
+  if constexpr (sizeof(R) == 4) {
+    op_lane<MASK>(v, staged + BT_GOP(o, stage));
+  } else {
+    op_fma<MASK>(v, geo, BT_GOP(o, moff));
+  }
+}
+
+template <typename R, typename G>
+__device__ __forceinline__ void op_any(int mask, C<R>* v, const G& geo, int o, const C<R>* staged) {
+  switch (mask) {
+#define BT_CASE(M) \
+  case M: op_reg<R, M>(v, geo, o, staged); break;
+#define BT_CASE5(M)                                                               \
+  case M:                                                                         \
+    if constexpr (TileCfg<R>::RB == 5) op_reg<R, M>(v, geo, o, staged); \
+    break;
+    BT_CASE(1) BT_CASE(2) BT_CASE(4) BT_CASE(8) BT_CASE(3) BT_CASE(5) BT_CASE(6) BT_CASE(9) BT_CASE(10) BT_CASE(12)
+    BT_CASE5(16) BT_CASE5(17) BT_CASE5(18) BT_CASE5(20) BT_CASE5(24)
+#undef BT_CASE5
+#undef BT_CASE
+    default: break;
+  }
+}
+
+// k >= 3 operator on the tile image, thread tid of the block.
+template <typename R, int K, typename G>
+__device__ __forceinline__ void op_image(C<R>* lds, int T, const G& geo, int o, const C<R>* staged, uint32_t tid) {
+  constexpr int NT = TileCfg<R>::NT;
+  constexpr int D = 1 << K;
+  const uint32_t ng = 1u << (T - K);
+  const C<R>* m = staged + BT_GOP(o, stage);
+  uint32_t srt[K];
+#pragma unroll
+  for (int i = 0; i < K; i++) srt[i] = (uint32_t)BT_GOP(o, lsorted[i]);
+  for (uint32_t g = tid; g < ng; g += NT) {
+    uint32_t lb = g;
+#pragma unroll
+    for (int i = 0; i < K; i++) lb = ((lb >> srt[i]) << (srt[i] + 1)) | (lb & ((1u << srt[i]) - 1u));
+    C<R> x[D];
+#pragma unroll
+    for (int l = 0; l < D; l++) x[l] = lds[swz<R>(lb + (uint32_t)BT_GOP(o, loff[l]))];
+#pragma unroll 1
+    for (int r = 0; r < D; r++) {  // rows one at a time
+      C<R> acc = cmake<C<R>>(0, 0);
+#pragma unroll
+      for (int c = 0; c < D; c++) acc = cfma(acc, m[r + c * D], x[c]);
+      lds[swz<R>(lb + (uint32_t)BT_GOP(o, loff[r]))] = acc;
+    }
+  }
+}
+
+// ---- reductions -----------------------------------------------------------
+// Norm^2 of register r.
+template <typename R>
+__device__ __forceinline__ double reg_norm(const C<R>& v) {
+  return (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+}
+
+// Add one value per thread to slot j of this wavefront's accumulators.
+__device__ __forceinline__ void wave_add(double x, double* wred, int j, bool lead) {
+  const double t = wave_sum(x);
+  if (lead) wred[j] += t;
+}
+
+// Reduced rho over K = 1 or 2 tile bits from the tile image: thread t takes
+// the index groups t, t + NT, ... and all entries, packed as rho_reg packs
+// them (the tile is in LDS at this point anyway, and its registers are free).
+template <typename R, int K, typename G>
+__device__ __forceinline__ void rho_add(const C<R>* lds, int T, const G& geo, double* wred, bool lead) {
+  constexpr int D = 1 << K;
+  uint32_t ls[K], off[D];
+#pragma unroll
+  for (int i = 0; i < K; i++) ls[i] = (uint32_t)BT_G(red_ls[i]);
+#pragma unroll
+  for (int a = 0; a < D; a++) off[a] = swz<R>((uint32_t)BT_G(red_loff[a]));  // the swizzle is linear over XOR
+  double acc[D * D];
+#pragma unroll
+  for (int j = 0; j < D * D; j++) acc[j] = 0.0;
+  const uint32_t ng = 1u << (T - K);
+#pragma unroll 1
+  for (uint32_t g = threadIdx.x; g < ng; g += TileCfg<R>::NT) {
+    uint32_t lb = g;
+#pragma unroll
+    for (int i = 0; i < K; i++) lb = ((lb >> ls[i]) << (ls[i] + 1)) | (lb & ((1u << ls[i]) - 1u));
+    const uint32_t sb = swz<R>(lb);
+    double vr[D], vi[D];
+#pragma unroll
+    for (int a = 0; a < D; a++) {
+      const C<R> x = lds[sb ^ off[a]];
+      vr[a] = (double)x.x;
+      vi[a] = (double)x.y;
+    }
+    int p = D;
+#pragma unroll
+    for (int a = 0; a < D; a++) {
+      acc[a] += vr[a] * vr[a] + vi[a] * vi[a];
+#pragma unroll
+      for (int b = a + 1; b < D; b++) {
+        acc[p] += vr[a] * vr[b] + vi[a] * vi[b];
+        acc[p + 1] += vi[a] * vr[b] - vr[a] * vi[b];
+        p += 2;
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < D * D; j++) wave_add(acc[j], wred, 1 + j, lead);
+}
+
+// The quad's four partials of a 3-bit reduced-rho entry, summed in a fixed
+// order ((s0 + s1) + (s2 + s3)), added by the quad's first lane to its
+// wavefront's packed-rho slots (LDS; each entry has one writer).
+template <typename R, typename G>
+__device__ __forceinline__ void rho3_add(const C<R>* lds, int T, const G& geo, double* wred) {
+  const int e = (int)(threadIdx.x >> 2);
+  double xr = 0.0, xi = 0.0;
+  if (e < 36) {
+    int a, b, ls[3];
+    rho3_pair(e, &a, &b);
+#pragma unroll
+    for (int i = 0; i < 3; i++) ls[i] = BT_G(red_ls[i]);
+    rho3_sum<R>(lds, T, geo.lane_w(offsetof(PassGeom, red_loff) + 4 * (size_t)a),
+                geo.lane_w(offsetof(PassGeom, red_loff) + 4 * (size_t)b), ls, threadIdx.x & 3, &xr, &xi);
+  }
+  xr += dpp_f64<0xb1>(xr);
+  xr += dpp_f64<0x4e>(xr);
+  xi += dpp_f64<0xb1>(xi);
+  xi += dpp_f64<0x4e>(xi);
+  if (e < 36 && (threadIdx.x & 3) == 0) {
+    const int sl = 1 + rho3_slot(e);
+    wred[sl] += xr;
+    if (e >= 8) wred[sl + 1] += xi;
+  }
+}
+
+// Bits of t deposited on the set bits of m, ascending.
+__device__ __forceinline__ uint64_t deposit(uint64_t t, uint64_t m) {
+  uint64_t r = 0;
+  while (m) {
+    const int lo = __builtin_ctzll(m);
+    const uint64_t up = ~(m >> lo);
+    const int len = up ? __builtin_ctzll(up) : 64 - lo;
+    const uint64_t ones = len < 64 ? (1ull << len) - 1ull : ~0ull;
+    r |= (t & ones) << lo;
+    t = len < 64 ? t >> len : 0;
+    m &= ~(ones << lo);
+  }
+  return r;
+}
+
 // One pass over tiles t = t0, t0 + tstep, ... < tend.  Reductions are added
 // to sums[0..kAcc) (LDS, zeroed by the caller): [0] norm^2, [1..16]
 // histogram, [17..32] packed rho; each wavefront accumulates its tiles in
 // red[wave * kAcc + j] (LDS, NT/64 * kAcc doubles) and the waves are summed
-// in order at the end.  lds holds 2^T elements.
+// in order at the end.  lds holds 2^T elements; staged holds kStageEntries
+// elements, filled from geo.staged (null: already filled).
 // fresh != 0: the state is |0...0> and is not read (its first pass).
-// The host emulation of this loop (tests/emu) follows it step for step.
-template <typename R, typename O>
-__device__ __forceinline__ void tile_pass(C<R>* __restrict__ state, const PassGeom& g, const C<R>* mats, C<R>* lds,
-                                          uint64_t t0, uint64_t tstep, uint64_t tend, double* red, double* sums,
-                                          int fresh = 0) {
+//
+// Between phases the tile lives in its LDS image, not in registers: a phase
+// reads its slots, applies its operators and writes the same slots back (no
+// other thread owns them in this layout), so one barrier separates phases
+// and no register array is live across the phase loop.
+// What bounds it: with neither operators nor relayouts the same loads and
+// stores move a 2^30-amplitude complex64 state at 4.8 TB/s (256 resident
+// states of 2^22: 5.2 TB/s); operators and relayouts add a third to that,
+// as dependency chains of two workgroups per CU.  With the tile held in
+// registers across phases (two barriers per relayout, geometry in LDS) a
+// 2^30 pass took 4.96 ms on average, this way 4.5 ms.
+// The host emulation (tests/emu) follows the same phases.
+template <typename R, typename O, typename G>
+__device__ __forceinline__ void tile_pass(C<R>* __restrict__ state, const G& geo0, C<R>* staged, C<R>* lds,
+                                          uint64_t t0, uint64_t tstep, uint64_t tend, double* red,
+                                          double* sums, int fresh = 0) {
   constexpr int NT = TileCfg<R>::NT;
   constexpr int NR = 1 << TileCfg<R>::RB;
-  const int T = g.T;
-  const R scale = (R)g.scale;
-  double* wred = red + (threadIdx.x >> 6) * kAcc;
-  for (int i = threadIdx.x; i < (NT / 64) * kAcc; i += NT) red[i] = 0.0;
-  __syncthreads();
-  ThreadIO<O> io;
-  thread_io<R, O>(g, threadIdx.x, io);
-  C<R> v[NR], nx[NR];
+  const G& geo = geo0;
+  const int T = BT_G(T), tb = BT_G(tb), nrb = BT_G(nrb), nph = BT_G(nph), redk = BT_G(red_k), redt = BT_G(red);
+  const bool write = BT_G(write) != 0, need_norm = BT_G(need_norm) != 0;
+  const bool in_direct = BT_G(in_direct) != 0, out_direct = BT_G(out_direct) != 0;
+  const bool hist_fast = BT_G(hist_fast) != 0;
+  const R scale = (R)__builtin_bit_cast(
+      double, ((uint64_t)geo.w(offsetof(PassGeom, scale) + 4) << 32) | (uint64_t)geo.w(offsetof(PassGeom, scale)));
+  const uint64_t M = ((uint64_t)geo.w(offsetof(PassGeom, outside) + 4) << 32) | geo.w(offsetof(PassGeom, outside));
+  const uint32_t tid = threadIdx.x, ltid = tid & ((1u << tb) - 1u);
+  const bool active = tid < (1u << tb), lead = (tid & 63) == 0;
+  const int nvalid_mask = (NR - 1) & ~((1 << nrb) - 1);
+  double* wred = red + (tid >> 6) * kAcc;
+  IoRegs<R, O> in(geo, offsetof(PassGeom, thr_in), offsetof(PassGeom, reg_in), ltid);
   // tile t's base is t's bits deposited on the outside bits M (ascending), so
   // the next tile's base is a masked add: ((base | ~M) + deposit(tstep)) & M
-  const uint64_t M = uniform_u64(tile_base(g, ~0ull)), S = uniform_u64(tile_base(g, tstep));
-  uint64_t base = uniform_u64(tile_base(g, t0));
+  const uint64_t S = uniform_u64(deposit(tstep, M));
+  uint64_t base = uniform_u64(deposit(t0, M));
+  C<R> nx[NR];
+  if (t0 < tend && !fresh) pass_fetch<R, O>(nx, state, in, base);
+  geo.template warm<R>();
+  for (int i = tid; i < (NT / 64) * kAcc; i += NT) red[i] = 0.0;
+  if (geo.staged) {
+    const int n = BT_G(nstage) * (int)sizeof(C<R>) / 16;
+    for (int e = tid; e < n; e += NT) ((float4*)staged)[e] = ((const float4*)geo.staged)[e];
+  }
+  IoRegs<R, O> out(geo, offsetof(PassGeom, thr_out), offsetof(PassGeom, reg_out), ltid);
+  __syncthreads();
   // Software pipeline over the tiles (disjoint): tile t's operators run while
   // the loads of tile t+1 and the stores of tile t-1 are in flight.  The wait
   // for tile t+1's loads is placed before tile t's stores are issued: the
   // vector-memory counter does not order loads against stores, so a wait for
   // loads issued before stores also waits for the stores; waiting first lets
   // tile t's stores complete under tile t+1's operators instead.
-  if (t0 < tend) {
-    if (!fresh) fetch_regs<R, O>(nx, state, io, base);
-    take_regs<R, O>(v, nx, io, base, scale, fresh);
-    if (!fresh && t0 + tstep < tend) fetch_regs<R, O>(nx, state, io, ((base | ~M) + S) & M);
-  }
+  const int np = nph > 0 ? nph : 1;
   for (uint64_t t = t0; t < tend; t += tstep) {
-    opaque_io(io);
     const uint64_t nbase = ((base | ~M) + S) & M;
     const bool more = t + tstep < tend;
-    int8_t cur[kRB];
+    for (int p = 0; p < np; p++) {
+      const G geo = geo0.again();
+      C<R> v[NR];
+      const int lay = nph > 0 ? p : kLayIn;
+      if (p == 0) {
+        if (!fresh && active && nvalid_mask == 0) {
 #pragma unroll
-    for (int j = 0; j < kRB; j++) cur[j] = g.io_in[j];
-    int ci = kLayIn;
-    for (int p = 0; p <= g.nph; p++) {
-      int8_t want[kRB];
-      const int wi = p < g.nph ? p : kLayOut;
-#pragma unroll
-      for (int j = 0; j < kRB; j++) want[j] = p < g.nph ? g.ph[p].rb[j] : g.io_out[j];
-      bool same = true;
-#pragma unroll
-      for (int j = 0; j < kRB; j++) same = same && (cur[j] == want[j]);
-      if (!same) {
-        regs_to_lds<R>(v, lds, g.lay[ci], io.tid, io.active, io.nvalid_mask);
-        __syncthreads();
-        lds_to_regs<R>(v, lds, g.lay[wi], io.ltid);
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kRB; j++) cur[j] = want[j];
-        ci = wi;
-      }
-      if (p == g.nph) break;
-      const int op0 = g.ph[p].op0, op1 = op0 + g.ph[p].nops;
-      const int tm = uniform_i32(g.ph[p].tmpl);
-      if (tm > 0) apply_template<R>(tm, v, mats, g.ops + op0);
-      for (int o = op0 + (tm > 0 ? 2 : 0); o < op1; o++) {  // every template covers two operators
-        const ROp& op = g.ops[o];
-        if ((base & op.gctrl) != op.gctrl) continue;
-        if (op.k <= 2) {
-          apply_mask<R>(op.mask, v, mats + op.moff);
+          for (int r = 0; r < NR; r++) v[r] = cmake<C<R>>(nx[r].x * scale, nx[r].y * scale);
         } else {
-          regs_to_lds<R>(v, lds, g.lay[ci], io.tid, io.active, io.nvalid_mask);
-          __syncthreads();
-          if (op.k == 3) apply_lds<R, 3>(lds, T, op, mats + op.moff, io.tid);
-          else apply_lds<R, 4>(lds, T, op, mats + op.moff, io.tid);
-          __syncthreads();
-          lds_to_regs<R>(v, lds, g.lay[ci], io.ltid);
+          const int nm = hide(nvalid_mask);
+#pragma unroll
+          for (int r = 0; r < NR; r++) {
+            const bool ok = active && !(r & nm);
+            if (fresh) {
+              v[r] = cmake<C<R>>(ok && r == 0 && base == 0 && in.thr == 0 ? scale : (R)0, (R)0);
+            } else {
+              v[r] = cmake<C<R>>(ok ? nx[r].x * scale : (R)0, ok ? nx[r].y * scale : (R)0);
+            }
+          }
+        }
+        if (!fresh && more) {
+          in.again();
+          pass_fetch<R, O>(nx, state, in, nbase);
+        }
+        if (!in_direct) {
+          image_write<R>(v, lds, geo, kLayIn, tid, active, nvalid_mask);
           __syncthreads();
         }
       }
-      if (p == g.nph - 1 && g.red == bti::RED_RHO) {
-        if (uflag(g.red_k == 3)) {
-          regs_to_lds<R>(v, lds, g.lay[ci], io.tid, io.active, io.nvalid_mask);
-          __syncthreads();
-          rho3_accumulate_t<R>(lds, g, wred + 1);
-          __syncthreads();
-        } else {
-          double racc[16];
-#pragma unroll
-          for (int j = 0; j < 16; j++) racc[j] = 0.0;
-          if (io.active) rho_mask<R>(rho_reg_mask(g), v, io.nvalid_mask, racc);
-          wave_accumulate<16>(racc, wred + 1);
+      if (p > 0 || !in_direct) image_read<R>(v, lds, geo, lay, ltid);
+      if (nph > 0) {
+        const size_t pa = offsetof(PassGeom, ph) + (size_t)p * sizeof(RPhase);
+        const int op0 = (int)geo.w(pa + offsetof(RPhase, op0)), op1 = op0 + (int)geo.w(pa + offsetof(RPhase, nops));
+        const int tm = (int)((geo.w(pa + 4) >> 8) & 0xffu);
+        int o = op0;
+        switch (tm) {  // the openings of kPhaseTemplates, straight-line
+          case 1:
+            op_reg<R, 0x0c>(v, geo, o, staged);
+            op_reg<R, 0x03>(v, geo, o + 1, staged);
+            op_reg<R, 0x06>(v, geo, o + 2, staged);
+            o += 3;
+            break;
+          case 2:
+            op_reg<R, 0x0c>(v, geo, o, staged);
+            op_reg<R, 0x03>(v, geo, o + 1, staged);
+            o += 2;
+            break;
+          case 3:
+            op_reg<R, 0x03>(v, geo, o, staged);
+            o += 1;
+            break;
+          default: break;
+        }
+        for (; o < op1; o++) {
+          const uint64_t gctrl = ((uint64_t)geo.w(offsetof(PassGeom, ops) + (size_t)o * sizeof(ROp) + offsetof(ROp, gctrl) + 4) << 32) |
+                                 (uint32_t)BT_GOP(o, gctrl);
+          if ((base & gctrl) != gctrl) continue;
+          const int k = BT_GOP(o, k);
+          if (k <= 2) {
+            op_any<R>(BT_GOP(o, mask), v, geo, o, staged);
+          } else {
+            image_write<R>(v, lds, geo, lay, tid, active, nvalid_mask);
+            __syncthreads();
+            if (k == 3) op_image<R, 3>(lds, T, geo, o, staged, tid);
+            else op_image<R, 4>(lds, T, geo, o, staged, tid);
+            __syncthreads();
+            image_read<R>(v, lds, geo, lay, ltid);
+          }
         }
       }
-    }
-    double acc[17];
-#pragma unroll
-    for (int j = 0; j < 17; j++) acc[j] = 0.0;
-    {
-      // tile t+1's loads (and tile t-1's stores) are done; prefetched values
-      // the register allocator parked in scratch come back here, before the
-      // stores, so that reloading them does not wait for the stores.  On
-      // every path (also the last tile, or when nothing was fetched): the
-      // compiler's wait bookkeeping merges paths, and one without this wait
-      // would make it wait at the take below, after the stores.
+      if (p + 1 < np || !out_direct || redt == bti::RED_RHO) {
+        image_write<R>(v, lds, geo, lay, tid, active, nvalid_mask);
+        __syncthreads();
+        if (p + 1 < np) continue;
+        if (redt == bti::RED_RHO) {
+          if (redk == 1) rho_add<R, 1>(lds, T, geo, wred, lead);
+          else if (redk == 2) rho_add<R, 2>(lds, T, geo, wred, lead);
+          else rho3_add<R>(lds, T, geo, wred);
+        }
+        image_read<R>(v, lds, geo, kLayOut, ltid);
+      }
+      // tile t+1's loads (and tile t-1's stores) are done before tile t's
+      // stores are issued, on every path
 #pragma unroll
       for (int r = 0; r < NR; r++) {
         opaque(nx[r].x);
         opaque(nx[r].y);
       }
       vm_wait_all();
-    }
-    store_regs<R, O>(v, state, g, io, base, acc);
-    if (g.red == bti::RED_HIST) {
-      switch (g.red_k) {  // norm + 2^red_k bins
-        case 1: wave_accumulate<3>(acc, wred); break;
-        case 2: wave_accumulate<5>(acc, wred); break;
-        case 3: wave_accumulate<9>(acc, wred); break;
-        default: wave_accumulate<17>(acc, wred); break;
+      out.again();
+      if (write) pass_store<R, O>(v, state, out, base, active, nvalid_mask);
+      if (need_norm) {
+        double s = 0.0;
+        if (nvalid_mask == 0) {
+#pragma unroll
+          for (int r = 0; r < NR; r++) s += reg_norm<R>(v[r]);
+        } else {
+          const int nm = hide(nvalid_mask);
+#pragma unroll
+          for (int r = 0; r < NR; r++) s += (r & nm) ? 0.0 : reg_norm<R>(v[r]);
+        }
+        s = active ? s : 0.0;
+        wave_add(s, wred, 0, lead);
+        if (redt == bti::RED_HIST) {
+          const int nb = 1 << redk;
+          if (hist_fast) {  // one bin for all of this thread's amplitudes
+            const uint64_t gi = base | (uint64_t)out.thr / sizeof(C<R>);
+            int bin = 0;
+#pragma unroll
+            for (int j = 0; j < bti::kGroupMax; j++)
+              if (j < redk) bin |= (int)((gi >> BT_G(red_bits[j])) & 1ull) << j;
+#pragma unroll 1
+            for (int b = 0; b < nb; b++) wave_add(bin == b ? s : 0.0, wred, 1 + b, lead);
+          } else {  // tiles too small to keep every bin bit off the registers: from the image, bin by bin
+            image_write<R>(v, lds, geo, kLayOut, tid, active, nvalid_mask);
+            __syncthreads();
+#pragma unroll 1
+            for (int b = 0; b < nb; b++) {
+              double x = 0.0;
+              for (uint32_t e = tid; e < (1u << T); e += NT) {
+                int bin = 0;
+                for (int j = 0; j < redk; j++) {
+                  const int lb = BT_G(red_ls[j]);
+                  bin |= (int)(lb >= 0 ? (e >> lb) & 1u : (uint32_t)(base >> BT_G(red_bits[j])) & 1u) << j;
+                }
+                x += bin == b ? reg_norm<R>(lds[swz<R>(e)]) : 0.0;
+              }
+              wave_add(x, wred, 1 + b, lead);
+            }
+          }
+        }
       }
-    } else if (g.need_norm) {
-      wave_accumulate<1>(acc, wred);
     }
-    if (more) {  // tile t+1 into registers, tile t+2's loads in flight
-      take_regs<R, O>(v, nx, io, nbase, scale, fresh);
-      if (!fresh && t + 2 * tstep < tend) fetch_regs<R, O>(nx, state, io, ((nbase | ~M) + S) & M);
-    }
+    // the next tile's first write to the image waits for this tile's last reads
+    if (more) __syncthreads();
     base = nbase;
   }
   __syncthreads();
