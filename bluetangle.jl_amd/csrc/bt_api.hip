@@ -10,6 +10,7 @@
 #include <string>
 #include <vector>
 
+#include "bt_circuit.hpp"
 #include "bt_internal.hpp"
 #include "bt_interp.hpp"
 
@@ -456,32 +457,37 @@ int bt_apply_kraus_dm(bt_state s, int k, int nkraus, const double* kraus, const 
   if (rc) return rc;
   if (s->kind != BT_DM) return fail(BT_ERR_UNSUPPORTED, "bt_apply_kraus_dm needs a density matrix");
   if (k < 1 || k > 2 || nkraus < 1 || !kraus || !bits) return fail(BT_ERR_ARG, "bad channel arguments");
-  const int D = 1 << k, S = D * D;
+  const int D = 1 << k;
   for (int i = 0; i < k; i++)
     if (bits[i] < 0 || bits[i] >= s->n) return fail(BT_ERR_ARG, "bit position out of range");
   // superoperator sum_i K_i (x) conj(K_i) on [row bits, column bits]
-  std::vector<double> sup(2 * S * S, 0.0);
+  std::vector<std::vector<cd>> A((size_t)nkraus);
   for (int i = 0; i < nkraus; i++) {
     const double* K = kraus + (size_t)i * 2 * D * D;
-    for (int r1 = 0; r1 < D; r1++)
-      for (int c1 = 0; c1 < D; c1++)
-        for (int r0 = 0; r0 < D; r0++)
-          for (int c0 = 0; c0 < D; c0++) {
-            cd v = mget(K, D, r1, r0) * std::conj(mget(K, D, c1, c0));
-            int row = (r1 << k) | c1, col = (r0 << k) | c0;
-            sup[2 * (row + col * S)] += v.real();
-            sup[2 * (row + col * S) + 1] += v.imag();
-          }
+    for (int e = 0; e < D * D; e++) A[(size_t)i].push_back(cd(K[2 * e], K[2 * e + 1]));
+  }
+  const std::vector<cd> sup = btc::superoperator(k, A);
+  Placement pl;
+  std::vector<cd> f[2];
+  if (k == 2 && bits[0] != bits[1] && btc::split_superoperator(sup, &f[0], &f[1])) {
+    // independent noise on the two qubits: one 4 x 4 operator each, in the
+    // kernel arguments, instead of a 16 x 16 one staged in device memory
+    for (int q = 0; q < 2; q++) {
+      const int rc2[2] = {bits[q], bits[q] + s->n};
+      rc = make_placement(s->nbits, 2, rc2, 0, &pl);
+      if (rc == BT_OK) rc = launch_apply(s, s->nbits, 2, (const double*)f[q].data(), pl, 1.0, false);
+      if (rc) return rc;
+    }
+    return BT_OK;
   }
   int sb[2 * 3];
   for (int i = 0; i < k; i++) {
     sb[i] = bits[i];
     sb[k + i] = bits[i] + s->n;
   }
-  Placement pl;
   rc = make_placement(s->nbits, 2 * k, sb, 0, &pl);
   if (rc) return rc;
-  return launch_apply(s, s->nbits, 2 * k, sup.data(), pl, 1.0, false);
+  return launch_apply(s, s->nbits, 2 * k, (const double*)sup.data(), pl, 1.0, false);
 }
 
 // ---- measurement -------------------------------------------------------------

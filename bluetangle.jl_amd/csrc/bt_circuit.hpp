@@ -249,11 +249,64 @@ inline int analyze(int nbits, const bt_ir_op* ops, int nops, int ntop, const dou
 
 using cd = std::complex<double>;
 
+// sum_i K_i (x) conj(K_i) of k-bit Kraus operators (column-major), a matrix
+// over [row bits, column bits] of vec(rho), column-major.
+inline std::vector<cd> superoperator(int k, const std::vector<std::vector<cd>>& A) {
+  const int D = 1 << k, S = D * D;
+  std::vector<cd> sup((size_t)S * S, cd(0, 0));
+  for (const auto& K : A)
+    for (int r1 = 0; r1 < D; r1++)
+      for (int c1 = 0; c1 < D; c1++)
+        for (int r0 = 0; r0 < D; r0++)
+          for (int c0 = 0; c0 < D; c0++) {
+            const cd v = K[r1 + r0 * D] * std::conj(K[c1 + c0 * D]);
+            sup[((r1 << k) | c1) + ((r0 << k) | c0) * S] += v;
+          }
+  return sup;
+}
+
+// A two-qubit superoperator over [row a, row b, column a, column b] that is
+// the product of one on qubit a and one on qubit b (independent noise on the
+// two: the 2-qubit model noise_model builds) as those factors, each over
+// [row, column].  Two 4 x 4 operators cost half the products of the 16 x 16
+// one and fit the matrix-core form.  False unless the product gives every
+// entry back to rounding.
+inline bool split_superoperator(const std::vector<cd>& s16, std::vector<cd>* sa, std::vector<cd>* sb) {
+  // S[(ra rb ca cb), (ra' rb' ca' cb')] = A[(ra ca), (ra' ca')] B[(rb cb), (rb' cb')]
+  auto at16 = [&](int a, int b) -> const cd& {  // a, b: row * 4 + column of A, B
+    const int ar = a >> 2, ac = a & 3, br = b >> 2, bc = b & 3;
+    auto mix = [](int x, int y) { return ((x >> 1) << 3) | ((y >> 1) << 2) | ((x & 1) << 1) | (y & 1); };
+    return s16[(size_t)mix(ar, br) + 16 * (size_t)mix(ac, bc)];
+  };
+  int pa = 0, pb = 0;
+  double top = 0;
+  for (int a = 0; a < 16; a++)
+    for (int b = 0; b < 16; b++)
+      if (std::abs(at16(a, b)) > top) {
+        top = std::abs(at16(a, b));
+        pa = a;
+        pb = b;
+      }
+  if (!(top > 0) || !std::isfinite(top)) return false;
+  std::vector<cd> A(16), B(16);
+  const cd pivot = at16(pa, pb);  // the largest entry: the division is well conditioned
+  for (int a = 0; a < 16; a++) A[(a >> 2) + 4 * (a & 3)] = at16(a, pb);
+  for (int b = 0; b < 16; b++) B[(b >> 2) + 4 * (b & 3)] = at16(pa, b) / pivot;
+  for (int a = 0; a < 16; a++)
+    for (int b = 0; b < 16; b++)
+      if (!(std::abs(A[(a >> 2) + 4 * (a & 3)] * B[(b >> 2) + 4 * (b & 3)] - at16(a, b)) <= 8 * 2.3e-16 * top)) return false;
+  *sa = A;
+  *sb = B;
+  return true;
+}
+
 // Density-matrix lowering: every op becomes superoperators on vec(rho)
-// (row bit b at b, column bit b at b + N).  A gate followed by its noise
-// channel on the same bits becomes one superoperator sum_i (K_i U) (x)
-// conj(K_i U); other gates become U on the row bits and conj(U) on the column
-// bits (controls on both sides).
+// (row bit b at b, column bit b at b + N).  A gate becomes U on the row bits
+// and conj(U) on the column bits (controls on both sides).  A one-qubit gate
+// followed by its noise channel becomes one superoperator sum_i (K_i U) (x)
+// conj(K_i U); a two-qubit channel whose superoperator is a product becomes
+// one superoperator per qubit; any other two-qubit channel is fused with the
+// gate before it on the same bits.
 inline int lower_dm(const CircuitHost& c, CircuitHost* out, std::string* msg) {
   const int N = c.n;
   out->n = 2 * N;
@@ -275,16 +328,7 @@ inline int lower_dm(const CircuitHost& c, CircuitHost* out, std::string* msg) {
     out->ops.push_back(o);
   };
   auto superop = [&](int k, const std::vector<std::vector<cd>>& A, const int32_t* bits) {
-    const int D = 1 << k, S = D * D;
-    std::vector<cd> sup(S * S, cd(0, 0));
-    for (const auto& K : A)
-      for (int r1 = 0; r1 < D; r1++)
-        for (int c1 = 0; c1 < D; c1++)
-          for (int r0 = 0; r0 < D; r0++)
-            for (int c0 = 0; c0 < D; c0++) {
-              cd v = K[r1 + r0 * D] * std::conj(K[c1 + c0 * D]);
-              sup[((r1 << k) | c1) + ((r0 << k) | c0) * S] += v;
-            }
+    const std::vector<cd> sup = superoperator(k, A);
     int32_t sb[4];
     for (int i = 0; i < k; i++) {
       sb[i] = bits[i];
@@ -298,6 +342,27 @@ inline int lower_dm(const CircuitHost& c, CircuitHost* out, std::string* msg) {
     const double* p = c.pool.data() + 2 * (op.mat + (int64_t)idx * D * D);
     for (int i = 0; i < D * D; i++) m[i] = cd(p[2 * i], p[2 * i + 1]);
     return m;
+  };
+  // the factors of a two-qubit channel (empty: not a product); a noise model
+  // repeats one channel, so the last answer is kept with its matrices
+  std::vector<double> last_k;
+  std::vector<cd> last_f[2];
+  auto factors = [&](const bt_ir_op& op) {
+    const double* p = c.pool.data() + 2 * op.mat;
+    const size_t n = (size_t)2 * 16 * op.nkraus;
+    if (last_k.size() == n && std::equal(last_k.begin(), last_k.end(), p)) return !last_f[0].empty();
+    last_k.assign(p, p + n);
+    last_f[0].clear();
+    std::vector<std::vector<cd>> A;
+    for (int j = 0; j < op.nkraus; j++) A.push_back(mat(op, j));
+    if (!split_superoperator(superoperator(2, A), &last_f[0], &last_f[1])) last_f[0].clear();
+    return !last_f[0].empty();
+  };
+  auto add_factors = [&](const int32_t* bits) {
+    for (int q = 0; q < 2; q++) {
+      const int32_t rc[2] = {bits[q], bits[q] + N};
+      add_gate(2, rc, 0, last_f[q]);
+    }
   };
   for (int i = 0; i < c.ntop; i++) {
     const bt_ir_op& op = c.ops[i];
@@ -315,6 +380,10 @@ inline int lower_dm(const CircuitHost& c, CircuitHost* out, std::string* msg) {
         *msg = "3-qubit channels have no density-matrix method";
         return BT_ERR_UNSUPPORTED;
       }
+      if (op.k == 2 && factors(op)) {
+        add_factors(op.bits);
+        continue;
+      }
       std::vector<std::vector<cd>> A;
       for (int j = 0; j < op.nkraus; j++) A.push_back(mat(op, j));
       superop(op.k, A, op.bits);
@@ -327,9 +396,23 @@ inline int lower_dm(const CircuitHost& c, CircuitHost* out, std::string* msg) {
     }
     const std::vector<cd> U = mat(op, 0);
     const int D = 1 << op.k;
+    auto both_sides = [&] {
+      std::vector<cd> Uc(U.size());
+      for (size_t j = 0; j < U.size(); j++) Uc[j] = std::conj(U[j]);
+      int32_t cb[4];
+      for (int j = 0; j < op.k; j++) cb[j] = op.bits[j] + N;
+      add_gate(op.k, op.bits, op.ctrl_mask, U);
+      add_gate(op.k, cb, op.ctrl_mask << N, Uc);
+    };
     if (op.ctrl_mask == 0 && i + 1 < c.ntop && c.ops[i + 1].kind == BT_OP_CHANNEL && c.ops[i + 1].k == op.k &&
         std::equal(op.bits, op.bits + op.k, c.ops[i + 1].bits)) {
       const bt_ir_op& ch = c.ops[i + 1];
+      if (op.k == 2 && factors(ch)) {
+        both_sides();
+        add_factors(ch.bits);
+        i++;
+        continue;
+      }
       std::vector<std::vector<cd>> A;
       for (int j = 0; j < ch.nkraus; j++) {
         std::vector<cd> K = mat(ch, j), KU(D * D, cd(0, 0));
@@ -342,12 +425,7 @@ inline int lower_dm(const CircuitHost& c, CircuitHost* out, std::string* msg) {
       i++;
       continue;
     }
-    std::vector<cd> Uc(U.size());
-    for (size_t j = 0; j < U.size(); j++) Uc[j] = std::conj(U[j]);
-    int32_t cb[4];
-    for (int j = 0; j < op.k; j++) cb[j] = op.bits[j] + N;
-    add_gate(op.k, op.bits, op.ctrl_mask, U);
-    add_gate(op.k, cb, op.ctrl_mask << N, Uc);
+    both_sides();
   }
   out->ntop = (int)out->ops.size();
   out->chan.assign(out->ops.size(), bti::ChanDesc{1, 0, 0});  // no renormalisation bookkeeping
