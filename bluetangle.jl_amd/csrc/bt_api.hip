@@ -192,13 +192,14 @@ int bt_state_create(int nqubits, int kind, int prec, bt_state* out) {
       return fail(BT_ERR_NOMEM, "hipMalloc of the state failed (out of HBM)");
     }
   }
-  if (hipMalloc(&s->d_part, sizeof(double) * kRedBlocks * kRedMax) != hipSuccess ||
-      hipMalloc(&s->d_out, sizeof(double) * kRedMax) != hipSuccess ||
+  const size_t part = sizeof(double) * kRedBlocks * kRedMax;
+  if (hipMalloc(&s->d_part, part + 16) != hipSuccess || hipMemset((char*)s->d_part + part, 0, 16) != hipSuccess ||
       hipHostMalloc(&s->h_out, sizeof(double) * kRedMax) != hipSuccess ||
       hipStreamCreate(&s->stream) != hipSuccess) {
     bt_state_destroy(s);
     return fail(BT_ERR_NOMEM, "allocation of state scratch failed");
   }
+  s->d_count = (unsigned*)((char*)s->d_part + part);
   rc = launch_set_basis(s, 0);
   if (rc) {
     bt_state_destroy(s);
@@ -213,7 +214,6 @@ int bt_state_destroy(bt_state s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   if (s->d) (void)hipFree(s->d);
   if (s->d_part) (void)hipFree(s->d_part);
-  if (s->d_out) (void)hipFree(s->d_out);
   if (s->d_mat) (void)hipFree(s->d_mat);
   if (s->h_out) (void)hipHostFree(s->h_out);
   if (s->grid) bt::free_grid_res(s->grid);
@@ -608,6 +608,15 @@ int bt_expect(bt_state s, int k, const double* mat, const int* bits, uint64_t xm
   if (!re || !im) return fail(BT_ERR_ARG, "null output");
   if (k > 0 && (!mat || !bits)) return fail(BT_ERR_ARG, "bt_expect: null block");
   return launch_expect(s, k, mat, bits, xmask, zmask, re, im);
+}
+
+int bt_expect_each(bt_state s, int pauli, double* out) {
+  int rc = check_state(s);
+  if (rc) return rc;
+  if (!out) return fail(BT_ERR_ARG, "null output");
+  if (s->kind != BT_SV) return fail(BT_ERR_UNSUPPORTED, "bt_expect_each: state vectors only (use bt_expect)");
+  if (pauli < 1 || pauli > 3) return fail(BT_ERR_ARG, "bt_expect_each: pauli must be 1 (X), 2 (Y) or 3 (Z)");
+  return launch_expect_each(s, pauli, out);
 }
 
 int bt_trace_purity(bt_state s, double* trace, double* purity) {

@@ -142,8 +142,8 @@ struct bt_state_s {
   uint64_t len = 0;  // 2^nbits complex entries
   void* d = nullptr; // device entries
   double* d_part = nullptr;  // reduction partials (device)
-  double* d_out = nullptr;   // reduction result (device)
-  double* h_out = nullptr;   // pinned host copy of the result
+  unsigned* d_count = nullptr;  // workgroups of the running reduction that have finished (behind the partials)
+  double* h_out = nullptr;   // reduction result (pinned host memory, written by the reduction's last workgroup)
   void* d_mat = nullptr;     // device matrix staging (k >= 4 blocks)
   bt::GridRes* grid = nullptr;  // circuit executor staging, made on the first run, kept with the state
   hipStream_t stream = nullptr;
@@ -180,6 +180,8 @@ struct ExpectArgs {
 };
 int launch_expect(bt_state_s* s, int k, const double* mat, const int* bits, uint64_t xmask, uint64_t zmask,
                   double* re, double* im);
+// <P_b> of every index bit b of a state vector (out[b]), P = X (1), Y (2) or Z (3).
+int launch_expect_each(bt_state_s* s, int pauli, double* out);
 // Shot sampling of a state vector (bt_sample.hip): shot s takes the smallest i
 // with u_s T < C_i (FP64 cumulative sums in index order, T the total);
 // d_u null -> every shot takes u0.  d_flag[s] = 1 when u_s T lies within 1e-12 T

@@ -7,6 +7,7 @@
 // FP64 and finish in a fixed order, so they are bit-reproducible.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -166,11 +167,9 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Block-level reduction of M per-thread values; thread j < M writes the
-// block sum of slot j to out[j].
+// Per-wavefront sums of M per-thread values (blockDim.x == 256: 4 waves).
 template <int M>
-__device__ __forceinline__ void block_reduce_store(double (&acc)[M], double* out) {
-  __shared__ double red[4][M];  // blockDim.x == 256 -> 4 waves
+__device__ __forceinline__ void block_sums(const double (&acc)[M], double (*red)[M]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int j = 0; j < M; j++) {
@@ -178,7 +177,79 @@ __device__ __forceinline__ void block_reduce_store(double (&acc)[M], double* out
     if (lane == 0) red[wave][j] = v;
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < M; j += blockDim.x) out[j] = red[0][j] + red[1][j] + red[2][j] + red[3][j];
+}
+
+// Where a reduction's M sums go: per-workgroup partials (part[b * M + j]),
+// then, by the last workgroup to finish, the totals.  part and count are
+// the state's, out its pinned host buffer: a reduction is one launch and one
+// wait, where a second launch for the totals and a copy of them cost another
+// 10 us of every call.
+struct ReduceOut {
+  double* part;
+  unsigned* count;  // 0 between launches
+  double* out;
+};
+
+// Store this workgroup's sums (red: [4][M] of block_sums) and, in the last
+// workgroup to finish, add up all workgroups' in a fixed order: 256 / M2
+// threads per sum (M2: M rounded up to a power of two), each over a fixed
+// stride of workgroups, then a fixed tree.  The partials cross the XCDs' L2
+// caches: agent-scope stores, complete before the count is raised, and
+// agent-scope loads after it.  Returns true in the last workgroup, with the
+// totals in sh[0..M).
+template <int M>
+__device__ __forceinline__ bool reduce_finish(const double (*red)[M], const ReduceOut& o, double* sh) {
+  __shared__ int last;
+  constexpr int M2 = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 16 ? 16 : 64;
+  constexpr unsigned G = 256 / M2;  // threads per sum
+  const unsigned nb = gridDim.x;
+  const int j = threadIdx.x & (M2 - 1);
+  const unsigned q = threadIdx.x / M2;
+  if (nb == 1) {
+    if (q == 0 && j < M) sh[j] = red[0][j] + red[1][j] + red[2][j] + red[3][j];
+    __syncthreads();
+    return true;
+  }
+  if (q == 0 && j < M)
+    __hip_atomic_store(o.part + (size_t)blockIdx.x * M + j, red[0][j] + red[1][j] + red[2][j] + red[3][j],
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials have reached the point of coherence
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(o.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+  __syncthreads();
+  if (!last) return false;
+  if (threadIdx.x == 0) __hip_atomic_store(o.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  double t = 0.0;
+  if (j < M) {
+    unsigned b = q;
+    for (; b + 7 * G < nb; b += 8 * G) {  // eight loads in flight
+      double x[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        x[i] = __hip_atomic_load(o.part + (size_t)(b + i * G) * M + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int i = 0; i < 8; i++) t += x[i];
+    }
+    for (; b < nb; b += G)
+      t += __hip_atomic_load(o.part + (size_t)b * M + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  sh[threadIdx.x] = t;  // slot j + M2 q
+  __syncthreads();
+  for (unsigned w = G / 2; w > 0; w >>= 1) {
+    if (q < w) sh[threadIdx.x] += sh[threadIdx.x + w * M2];
+    __syncthreads();
+  }
+  return true;
+}
+
+// Finish a reduction of M sums per thread: the totals go to o.out[0..M).
+template <int M>
+__device__ __forceinline__ void reduce_out(const double (&acc)[M], const ReduceOut& o) {
+  __shared__ double red[4][M];
+  __shared__ double sh[256];
+  block_sums<M>(acc, red);
+  if (reduce_finish<M>(red, o, sh) && threadIdx.x < M) o.out[threadIdx.x] = sh[threadIdx.x];
 }
 
 template <typename R, int K>
@@ -189,7 +260,7 @@ struct ReduceArgs {
   uint64_t off[D];
   int nfixed;
   int fixed[kMaxFixed];
-  double* part;
+  ReduceOut out;
 };
 
 // Packed layout of a reduced rho (D*D reals): [0, D) diagonal, then for
@@ -260,29 +331,12 @@ __global__ void __launch_bounds__(256) k_reduce(ReduceArgs<R, K> a) {
       }
     }
   }
-  block_reduce_store<M>(acc, a.part + (size_t)blockIdx.x * M);
+  reduce_out<M>(acc, a.out);
 }
 
-// out[j] = sum over blocks of part[b * M + j], one workgroup per j: each
-// thread sums a fixed stride of blocks, then a fixed tree (bit-reproducible).
-__global__ void __launch_bounds__(256) k_finalize(const double* part, int nblocks, int M, double* out) {
-  __shared__ double sh[256];
-  const int j = blockIdx.x;
-  double t = 0.0;
-  for (int b = threadIdx.x; b < nblocks; b += 256) t += part[(size_t)b * M + j];
-  sh[threadIdx.x] = t;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[j] = sh[0];
-}
-
-// <a|b> = sum conj(a_i) b_i in FP64 (either precision on either side):
-// per-workgroup partials (re, im)
+// <a|b> = sum conj(a_i) b_i in FP64 (either precision on either side): (re, im)
 template <typename RA, typename RB>
-__global__ void __launch_bounds__(256) k_inner(const C<RA>* a, const C<RB>* b, uint64_t n, double* part) {
+__global__ void __launch_bounds__(256) k_inner(const C<RA>* a, const C<RB>* b, uint64_t n, ReduceOut o) {
   constexpr int U = 4;
   double acc[2] = {0.0, 0.0};
   uint64_t lo, hi;
@@ -304,7 +358,7 @@ __global__ void __launch_bounds__(256) k_inner(const C<RA>* a, const C<RB>* b, u
       acc[1] = fma((double)x[u].x, (double)y[u].y, fma(-(double)x[u].y, (double)y[u].x, acc[1]));
     }
   }
-  block_reduce_store<2>(acc, part + (size_t)blockIdx.x * 2);
+  reduce_out<2>(acc, o);
 }
 
 // Expectation of O = P(x, z) G(B): P(x, z)[a, b] = (-1)^popcount(a & z) when
@@ -314,7 +368,7 @@ __global__ void __launch_bounds__(256) k_inner(const C<RA>* a, const C<RB>* b, u
 //   SV: conj(psi_a) O[a, b] psi_b       DM: O[a, b] rho[b + a 2^n]
 // On a state vector with x != 0, a0 also has the top bit of x clear and the
 // item takes both a0 and a0 ^ x, so each amplitude is read once.
-// Per-workgroup FP64 partials (re, im).
+// FP64 sums (re, im).
 template <typename R, int D>
 __device__ __forceinline__ void expect_quad(const C<R> (&u)[D], const C<R> (&v)[D], const double* g, double& sr,
                                             double& si) {
@@ -333,7 +387,7 @@ __device__ __forceinline__ void expect_quad(const C<R> (&u)[D], const C<R> (&v)[
 }
 
 template <typename R, int K, bool DM>
-__global__ void __launch_bounds__(256) k_expect(const C<R>* s, ExpectArgs a, double* part) {
+__global__ void __launch_bounds__(256) k_expect(const C<R>* s, ExpectArgs a, ReduceOut o) {
   constexpr int D = 1 << K;
   constexpr int U = DM ? 1 : red_unroll<K>();
   double acc[2] = {0.0, 0.0};
@@ -398,17 +452,155 @@ __global__ void __launch_bounds__(256) k_expect(const C<R>* s, ExpectArgs a, dou
       acc[1] += neg ? -si : si;
     }
   }
-  block_reduce_store<2>(acc, part + (size_t)blockIdx.x * 2);
+  reduce_out<2>(acc, o);
+}
+
+// ---------------------------------------------------------------------------
+// <X_b>, <Y_b> or <Z_b> of every index bit b at once
+// ---------------------------------------------------------------------------
+// One read of the state gives <Z_b> for all bits (each amplitude's weight
+// enters every sum with a sign), and a tile of 2^12 amplitudes gives <X_b> or
+// <Y_b> for its 12 bits, where a reduction per bit reads the state once per
+// bit: 25 bits of a 2^25-amplitude complex64 state are 1 read instead of 25
+// for Z and 3 for X.
+constexpr int kEachT = 12;  // tile: 256 threads x 16 amplitudes
+constexpr int kEachJ = 14;  // most bits of the tile number inside a workgroup's range
+
+// Rows of part / out: [0, 12) the tile's bits, [12, 12 + J) the tile
+// number's low bits (its range within a workgroup), then the total, whose
+// signed sums over workgroups give the bits above.
+constexpr int kEachZRows = kEachT + kEachJ + 1;
+
+template <typename R>
+__global__ void __launch_bounds__(256) k_expect_z(const C<R>* s, int nbits, int J, ReduceOut o) {
+  const uint64_t n = 1ull << nbits;
+  double acc[kEachZRows];
+#pragma unroll
+  for (int j = 0; j < kEachZRows; j++) acc[j] = 0.0;
+  const uint64_t t0 = (uint64_t)blockIdx.x << J;
+  double tot = 0.0;
+  for (uint32_t t = 0; t < (1u << J); t++) {
+    const uint64_t base = (t0 + t) << kEachT;
+    double w[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const uint64_t i = base + 256u * r + threadIdx.x;
+      C<R> v = cmake<C<R>>(0, 0);
+      if (i < n) v = s[i];
+      w[r] = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+    }
+    // the four register bits by halving: sums of pairs go on, differences are the signed sums
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+#pragma unroll
+      for (int r = 0; r < (8 >> b); r++) {
+        acc[8 + b] += w[2 * r] - w[2 * r + 1];
+        w[r] = w[2 * r] + w[2 * r + 1];
+      }
+    }
+    tot += w[0];
+#pragma unroll
+    for (int j = 0; j < kEachJ; j++)
+      if (j < J) acc[kEachT + j] += ((t >> j) & 1u) ? -w[0] : w[0];
+  }
+#pragma unroll
+  for (int b = 0; b < 8; b++) acc[b] = ((threadIdx.x >> b) & 1u) ? -tot : tot;
+  acc[kEachZRows - 1] = tot;
+  __shared__ double red[4][kEachZRows];
+  block_sums<kEachZRows>(acc, red);
+  // every workgroup's sums, row-major, for k_each_finish
+  if (threadIdx.x < kEachZRows) {
+    const int j = threadIdx.x;
+    o.part[(size_t)j * gridDim.x + blockIdx.x] = red[0][j] + red[1][j] + red[2][j] + red[3][j];
+  }
+}
+
+// Tile bits 0..3 are index bits 0..3, tile bits 4..11 the index bits
+// hi0..hi0 + 7 (hi0 >= 4); tile t's base is t deposited on the other bits.
+// imag: <Y> (2 Im conj(psi_0) psi_1) instead of <X> (2 Re).
+template <typename R>
+__global__ void __launch_bounds__(256) k_expect_xy(const C<R>* s, int nbits, int hi0, int imag, uint64_t ntiles,
+                                                   ReduceOut o) {
+  __shared__ C<R> tile[1 << kEachT];
+  const uint64_t n = 1ull << nbits;
+  const uint32_t tid = threadIdx.x;
+  double acc[kEachT];
+#pragma unroll
+  for (int j = 0; j < kEachT; j++) acc[j] = 0.0;
+  // one slot per 16-byte bank group: XOR the low bits with the ones above them
+  auto slot = [](uint32_t l) { return l ^ ((l >> 4) & 15u) ^ ((l >> 8) & 15u); };
+  auto pairs = [&](const C<R>* v, double* a) {  // the four register bits
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        if ((r >> b) & 1) continue;
+        const C<R> x = v[r], y = v[r | (1 << b)];
+        if (imag) a[b] = fma((double)x.x, (double)y.y, fma(-(double)x.y, (double)y.x, a[b]));
+        else a[b] = fma((double)x.x, (double)y.x, fma((double)x.y, (double)y.y, a[b]));
+      }
+  };
+  const bool low = hi0 == 4;  // the first call also takes bits 0..3
+  // thread t, register r: tile index r * 256 + t; index bits of t and r
+  const uint64_t thr = (tid & 15u) | ((uint64_t)(tid >> 4) << hi0);
+  const uint64_t per = (ntiles + gridDim.x - 1) / gridDim.x;
+  const uint64_t t1 = std::min<uint64_t>(ntiles, ((uint64_t)blockIdx.x + 1) * per);
+  for (uint64_t t = (uint64_t)blockIdx.x * per; t < t1; t++) {
+    // bits 4..hi0-1 below the window, the rest above it
+    const uint64_t lo = t & ((1ull << (hi0 - 4)) - 1ull), up = t >> (hi0 - 4);
+    const uint64_t base = (lo << 4) | (up << (hi0 + 8)) | thr;
+    C<R> v[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const uint64_t i = base | ((uint64_t)r << (hi0 + 4));
+      v[r] = cmake<C<R>>(0, 0);
+      if (i < n) v[r] = s[i];
+    }
+    pairs(v, acc + 8);
+    __syncthreads();  // the last tile's reads are done
+#pragma unroll
+    for (int r = 0; r < 16; r++) tile[slot(tid | (r << 8))] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; r++) v[r] = tile[slot((tid & 15u) | (r << 4) | ((tid >> 4) << 8))];
+    pairs(v, acc + 4);
+    if (low) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) v[r] = tile[slot((uint32_t)r | (tid << 4))];
+      pairs(v, acc);
+    }
+  }
+  __shared__ double red[4][kEachT];
+  block_sums<kEachT>(acc, red);
+  if (tid < kEachT) o.part[(size_t)tid * gridDim.x + blockIdx.x] = 2.0 * (red[0][tid] + red[1][tid] + red[2][tid] + red[3][tid]);
+}
+
+// out[b]: row b's sum over the nb workgroups; for b >= rows, the last row
+// (total) signed by bit b - rows of the workgroup number.  One workgroup per
+// output, fixed order.
+__global__ void __launch_bounds__(256) k_each_finish(const double* part, int nb, int rows, int total, double* out) {
+  __shared__ double sh[256];
+  const int b = blockIdx.x;
+  const double* p = part + (size_t)(b < rows ? b : total) * nb;
+  double t = 0.0;
+  for (int i = threadIdx.x; i < nb; i += 256) t += b < rows || !((i >> (b - rows)) & 1) ? p[i] : -p[i];
+  sh[threadIdx.x] = t;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) out[b] = sh[0];
 }
 
 // sum over i of Re(s[i * step]) for i < count (trace of vec(rho): step = D+1)
 template <typename R>
-__global__ void __launch_bounds__(256) k_strided_re_sum(const C<R>* s, uint64_t count, uint64_t step, double* part) {
+__global__ void __launch_bounds__(256) k_strided_re_sum(const C<R>* s, uint64_t count, uint64_t step, ReduceOut o) {
   double acc[1] = {0.0};
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride)
     acc[0] += (double)s[i * step].x;
-  block_reduce_store<1>(acc, part + blockIdx.x);
+  reduce_out<1>(acc, o);
 }
 
 template <typename R>
@@ -455,13 +647,21 @@ __global__ void k_gather(const C<R>* s, uint64_t len, const uint64_t* idx, uint6
 // Workgroups of a reduction with M partial values each over `work` items:
 // 16384 for large states (each a contiguous range, see red_range: 6.2 TB/s
 // against 6.1 at 4096 and 6.0 at 2048 for one read of 2^30 complex64
-// amplitudes); kRedBlocks below 2^26 items, where the launch and the final
-// sum of the partials dominate; always within the partial buffer of
-// kRedBlocks * kRedMax values.
+// amplitudes), 4096 below 2^28 items, kRedBlocks below 2^26, where the launch
+// and the final sum of the partials dominate; always within the partial
+// buffer of kRedBlocks * kRedMax values.
 static uint64_t red_cap(int M, uint64_t work) {
   const uint64_t c = (uint64_t)kRedBlocks * kRedMax / (uint64_t)M;
-  const uint64_t want = work >= (1ull << 26) ? 16384 : kRedBlocks;
+  const uint64_t want = work >= (1ull << 28) ? 16384 : work >= (1ull << 26) ? 4096 : kRedBlocks;
   return c < want ? c : want;
+}
+
+static ReduceOut reduce_to(bt_state_s* s) { return ReduceOut{s->d_part, s->d_count, s->h_out}; }
+
+static int reduce_wait(bt_state_s* s) {
+  BT_HIP(hipGetLastError());
+  BT_HIP(hipStreamSynchronize(s->stream));
+  return BT_OK;
 }
 
 static unsigned grid_for(uint64_t work, unsigned block = 256, uint64_t cap = (1ull << 20)) {
@@ -578,15 +778,10 @@ static int reduce_t(bt_state_s* s, const Placement& p) {
   for (int l = 0; l < D; l++) a.off[l] = p.off[l];
   a.nfixed = p.nfixed;
   for (int i = 0; i < p.nfixed; i++) a.fixed[i] = p.fixed[i];
-  a.part = s->d_part;
+  a.out = reduce_to(s);
   const unsigned blocks = grid_for(a.ngroups, 256, red_cap(M, a.ngroups));
   hipLaunchKernelGGL((k_reduce<R, K>), dim3(blocks), dim3(256), 0, s->stream, a);
-  BT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_finalize, dim3(M), dim3(256), 0, s->stream, (const double*)s->d_part, (int)blocks, M, s->d_out);
-  BT_HIP(hipGetLastError());
-  BT_HIP(hipMemcpyAsync(s->h_out, s->d_out, sizeof(double) * M, hipMemcpyDeviceToHost, s->stream));
-  BT_HIP(hipStreamSynchronize(s->stream));
-  return BT_OK;
+  return reduce_wait(s);
 }
 
 int launch_inner(bt_state_s* a, bt_state_s* b, double* re, double* im) {
@@ -595,21 +790,18 @@ int launch_inner(bt_state_s* a, bt_state_s* b, double* re, double* im) {
   const bool fa = a->prec == BT_C64, fb = b->prec == BT_C64;
   if (fa && fb)
     hipLaunchKernelGGL((k_inner<float, float>), dim3(blocks), dim3(256), 0, a->stream, (const C<float>*)a->d,
-                       (const C<float>*)b->d, n, a->d_part);
+                       (const C<float>*)b->d, n, reduce_to(a));
   else if (fa)
     hipLaunchKernelGGL((k_inner<float, double>), dim3(blocks), dim3(256), 0, a->stream, (const C<float>*)a->d,
-                       (const C<double>*)b->d, n, a->d_part);
+                       (const C<double>*)b->d, n, reduce_to(a));
   else if (fb)
     hipLaunchKernelGGL((k_inner<double, float>), dim3(blocks), dim3(256), 0, a->stream, (const C<double>*)a->d,
-                       (const C<float>*)b->d, n, a->d_part);
+                       (const C<float>*)b->d, n, reduce_to(a));
   else
     hipLaunchKernelGGL((k_inner<double, double>), dim3(blocks), dim3(256), 0, a->stream, (const C<double>*)a->d,
-                       (const C<double>*)b->d, n, a->d_part);
-  BT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_finalize, dim3(2), dim3(256), 0, a->stream, (const double*)a->d_part, (int)blocks, 2, a->d_out);
-  BT_HIP(hipGetLastError());
-  BT_HIP(hipMemcpyAsync(a->h_out, a->d_out, sizeof(double) * 2, hipMemcpyDeviceToHost, a->stream));
-  BT_HIP(hipStreamSynchronize(a->stream));
+                       (const C<double>*)b->d, n, reduce_to(a));
+  const int rc = reduce_wait(a);
+  if (rc) return rc;
   *re = a->h_out[0];
   *im = a->h_out[1];
   return BT_OK;
@@ -657,15 +849,12 @@ int launch_trace(bt_state_s* s, double* out) {
   const unsigned blocks = grid_for(D, 256, kRedBlocks);
   if (s->prec == BT_C64)
     hipLaunchKernelGGL(k_strided_re_sum<float>, dim3(blocks), dim3(256), 0, s->stream, (const C<float>*)s->d, D, D + 1,
-                       s->d_part);
+                       reduce_to(s));
   else
     hipLaunchKernelGGL(k_strided_re_sum<double>, dim3(blocks), dim3(256), 0, s->stream, (const C<double>*)s->d, D,
-                       D + 1, s->d_part);
-  BT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, s->stream, (const double*)s->d_part, (int)blocks, 1, s->d_out);
-  BT_HIP(hipGetLastError());
-  BT_HIP(hipMemcpyAsync(s->h_out, s->d_out, sizeof(double), hipMemcpyDeviceToHost, s->stream));
-  BT_HIP(hipStreamSynchronize(s->stream));
+                       D + 1, reduce_to(s));
+  const int rc = reduce_wait(s);
+  if (rc) return rc;
   *out = s->h_out[0];
   return BT_OK;
 }
@@ -718,10 +907,11 @@ int launch_gather(bt_state_s* s, const uint64_t* d_idx, uint64_t n, double* d_ou
 template <typename R, int K>
 static void expect_t(bt_state_s* s, const ExpectArgs& a, unsigned blocks) {
   if (s->kind == BT_DM)
-    hipLaunchKernelGGL((k_expect<R, K, true>), dim3(blocks), dim3(256), 0, s->stream, (const C<R>*)s->d, a, s->d_part);
+    hipLaunchKernelGGL((k_expect<R, K, true>), dim3(blocks), dim3(256), 0, s->stream, (const C<R>*)s->d, a,
+                       reduce_to(s));
   else
     hipLaunchKernelGGL((k_expect<R, K, false>), dim3(blocks), dim3(256), 0, s->stream, (const C<R>*)s->d, a,
-                       s->d_part);
+                       reduce_to(s));
 }
 
 int launch_expect(bt_state_s* s, int k, const double* mat, const int* bits, uint64_t xmask, uint64_t zmask,
@@ -770,14 +960,54 @@ int launch_expect(bt_state_s* s, int k, const double* mat, const int* bits, uint
     case 2: f ? expect_t<float, 2>(s, a, blocks) : expect_t<double, 2>(s, a, blocks); break;
     default: f ? expect_t<float, 3>(s, a, blocks) : expect_t<double, 3>(s, a, blocks); break;
   }
-  BT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_finalize, dim3(2), dim3(256), 0, s->stream, (const double*)s->d_part, (int)blocks, 2, s->d_out);
-  BT_HIP(hipGetLastError());
-  BT_HIP(hipMemcpyAsync(s->h_out, s->d_out, sizeof(double) * 2, hipMemcpyDeviceToHost, s->stream));
-  BT_HIP(hipStreamSynchronize(s->stream));
+  const int rc = reduce_wait(s);
+  if (rc) return rc;
   *re = s->h_out[0];
   *im = s->h_out[1];
   return BT_OK;
+}
+
+// <P_b> of every bit b of a state vector, P = X (1), Y (2) or Z (3).
+template <typename R>
+static int expect_each_t(bt_state_s* s, int pauli, double* out) {
+  const int N = s->n;
+  const uint64_t ntiles = N > kEachT ? 1ull << (N - kEachT) : 1;
+  if (pauli == 3) {
+    // at most 2048 workgroups of at most 2^kEachJ tiles (N <= 36: 2^24 tiles)
+    const int tb = N > kEachT ? N - kEachT : 0, J = std::max(0, tb - 11);
+    if (J > kEachJ) return fail(BT_ERR_ARG, "expectation of every qubit: state too large");
+    const int nb = (int)(ntiles >> J);
+    hipLaunchKernelGGL(k_expect_z<R>, dim3((unsigned)nb), dim3(256), 0, s->stream, (const C<R>*)s->d, N, J,
+                       reduce_to(s));
+    BT_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_each_finish, dim3((unsigned)N), dim3(256), 0, s->stream, (const double*)s->d_part, nb,
+                       kEachT + J, kEachZRows - 1, s->h_out);
+    const int rc = reduce_wait(s);
+    if (rc) return rc;
+    for (int b = 0; b < N; b++) out[b] = s->h_out[b];
+    return BT_OK;
+  }
+  // windows of 8 bits above the low 4; the last one ends at the top bit
+  const unsigned nb = (unsigned)std::min<uint64_t>(ntiles, 2048);
+  for (int b = 4; b < std::max(N, 5); b += 8) {
+    const int hi0 = b == 4 ? 4 : std::min(b, N - 8);
+    hipLaunchKernelGGL(k_expect_xy<R>, dim3(nb), dim3(256), 0, s->stream, (const C<R>*)s->d, N, hi0, pauli == 2 ? 1 : 0,
+                       ntiles, reduce_to(s));
+    BT_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_each_finish, dim3(kEachT), dim3(256), 0, s->stream, (const double*)s->d_part, (int)nb, kEachT,
+                       0, s->h_out);
+    const int rc = reduce_wait(s);
+    if (rc) return rc;
+    for (int j = hi0 == 4 ? 0 : 4; j < kEachT; j++) {
+      const int bit = j < 4 ? j : hi0 + j - 4;
+      if (bit < N) out[bit] = s->h_out[j];
+    }
+  }
+  return BT_OK;
+}
+
+int launch_expect_each(bt_state_s* s, int pauli, double* out) {
+  return s->prec == BT_C64 ? expect_each_t<float>(s, pauli, out) : expect_each_t<double>(s, pauli, out);
 }
 
 }  // namespace bt

@@ -192,6 +192,11 @@ def expect(state: DeviceState, what=None, qubit: Union[int, None] = None, pars=N
         m = gates(what)
         if qubit is not None:
             return _expect_product(state, {_bit(N, qubit): m}).real
+        pf = _pauli_form(m) if m.shape == (2, 2) and isinstance(state, StateVector) else None
+        if pf is not None and pf[0] != "I":  # a Pauli on every qubit: bt_expect_each, a few reads of the state
+            each = np.empty(N, dtype=np.float64)
+            L.check(L.lib().bt_expect_each(state.handle, "XYZ".index(pf[0]) + 1, L.dptr(each)))
+            return (pf[1] * each[::-1]).real  # qubit q on bit N - q
         return np.array([_expect_product(state, {_bit(N, q): m}).real for q in range(1, N + 1)])
     return _expect_complex(state, what, pars).real
 

@@ -129,6 +129,11 @@ int bt_inner(bt_state a, bt_state b, double* re, double* im);
  * and correlation(state, qubits) (func.jl:17-23: a Z string). */
 int bt_expect(bt_state s, int k, const double* mat, const int* bits, uint64_t xmask, uint64_t zmask, double* re,
               double* im);
+/* <psi|P_b|psi> of every index bit b (out[b], n doubles), P = X (1), Y (2) or
+ * Z (3), in FP64: expect(state, op_str) over all qubits (func.jl:91-100) in
+ * one read of the state for Z and one per 8 bits above the low 12 for X and
+ * Y, where bt_expect reads it once per bit.  State vectors only. */
+int bt_expect_each(bt_state s, int pauli, double* out);
 /* Shot sampling of a state vector: shot s returns the smallest basis index i
  * with u[s] * T < C_i, C_i the FP64 cumulative sum of |psi_j|^2 over j <= i in
  * index order and T the total (the state need not be normalised).  u: shots
