@@ -132,6 +132,8 @@ int dm_tile_bits_for(int prec, int nbits);      // the same for vec(rho) of nbit
 namespace bt {
 struct GridRes;  // the circuit executor's staging of a state (bt_exec.hip)
 void free_grid_res(GridRes* g);
+struct SampleBuffers;  // bt_sample's buffers of a state (bt_sample.hip)
+void free_sample_res(SampleBuffers* b);
 }  // namespace bt
 
 struct bt_state_s {
@@ -146,6 +148,7 @@ struct bt_state_s {
   double* h_out = nullptr;   // reduction result (pinned host memory, written by the reduction's last workgroup)
   void* d_mat = nullptr;     // device matrix staging (k >= 4 blocks)
   bt::GridRes* grid = nullptr;  // circuit executor staging, made on the first run, kept with the state
+  bt::SampleBuffers* sample = nullptr;  // bt_sample's buffers, made on the first call, kept with the state
   hipStream_t stream = nullptr;
   size_t elem() const { return prec == BT_C64 ? 8 : 16; }
 };

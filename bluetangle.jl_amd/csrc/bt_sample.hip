@@ -6,16 +6,16 @@
 //
 // Three kernels on the caller's stream:
 //   k_chunk_sums   FP64 sum of each chunk of 2048 probabilities;
-//   k_chunk_scan   exclusive prefix of the chunk sums (one workgroup, fixed
-//                  order), prefix[nchunks] = T;
+//   k_chunk_scan   exclusive prefix of the chunk sums, one workgroup per 2048
+//                  chunks, whose last one to finish adds up the workgroups;
 //   k_sample_find  one wavefront per shot: binary search of the chunk prefix,
-//                  then a wavefront scan of the chunk's probabilities (32
-//                  consecutive entries per lane).
+//                  then the chunk's rows in order (one 1 KiB row per load).
 // Sums are formed in a different order than a sequential cumsum; a shot whose
 // u_s T lies within 1e-12 T of a cumulative boundary is flagged.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -24,29 +24,51 @@
 namespace bt {
 
 constexpr int kChunk = 2048;       // probabilities per chunk
-constexpr int kLaneRun = kChunk / 64;  // consecutive entries per lane in the search
+constexpr int kScanRun = 2048;     // chunks per workgroup of the scan
 constexpr double kBoundaryTol = 1e-12;
 
 template <typename R>
-__device__ __forceinline__ double prob(const C<R>* s, uint64_t i) {
-  const C<R> v = s[i];
-  return (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+__device__ __forceinline__ double weight(R x, R y) {
+  return (double)x * (double)x + (double)y * (double)y;
 }
 
-// One wavefront per chunk (no workgroup barriers): lane l sums entries
-// l, l + 64, ... of the chunk in order, then a fixed butterfly over the
-// lanes.  The workgroup's four wavefronts take four consecutive chunks.
+// Entries of a row: the consecutive probabilities one wavefront load covers
+// (16 bytes per lane: two complex64 or one complex128 amplitude).
 template <typename R>
-__global__ void __launch_bounds__(256) k_chunk_sums(const C<R>* s, uint64_t n, uint64_t nchunks, double* sums) {
+constexpr int kRowEntries = 64 * 16 / (2 * sizeof(R));
+
+// The lane's probabilities of row r of the chunk at `base` (0 past n).
+template <typename R, int E>
+__device__ __forceinline__ void row_weights(const C<R>* s, uint64_t n, uint64_t base, int r, int lane, double (&p)[E]) {
+  const uint64_t i = base + (uint64_t)r * kRowEntries<R> + (uint64_t)(E * lane);
+  typedef R vec __attribute__((ext_vector_type(2 * E)));
+  if (i + E <= n) {
+    const vec v = *(const vec*)(s + i);
+#pragma unroll
+    for (int e = 0; e < E; e++) p[e] = weight<R>(v[2 * e], v[2 * e + 1]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; e++) p[e] = i + e < n ? weight<R>(s[i + e].x, s[i + e].y) : 0.0;
+  }
+}
+
+// One wavefront per chunk (no workgroup barriers): the rows in order, then a
+// fixed butterfly over the lanes.  Also clears the scan's counter.
+template <typename R>
+__global__ void __launch_bounds__(256) k_chunk_sums(const C<R>* s, uint64_t n, uint64_t nchunks, double* sums,
+                                                    unsigned* count) {
+  constexpr int E = kRowEntries<R> / 64, ROWS = kChunk / kRowEntries<R>;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;
   const int lane = threadIdx.x & 63;
   const uint64_t nw = (uint64_t)gridDim.x * 4;
   for (uint64_t c = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6); c < nchunks; c += nw) {
-    const uint64_t base = c * kChunk + (uint64_t)lane;
     double t = 0.0;
 #pragma unroll
-    for (int j = 0; j < kChunk / 64; j++) {
-      const uint64_t i = base + 64u * j;
-      if (i < n) t += prob<R>(s, i);
+    for (int r = 0; r < ROWS; r++) {
+      double p[E];
+      row_weights<R, E>(s, n, c * kChunk, r, lane, p);
+#pragma unroll
+      for (int e = 0; e < E; e++) t += p[e];
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
@@ -54,136 +76,308 @@ __global__ void __launch_bounds__(256) k_chunk_sums(const C<R>* s, uint64_t n, u
   }
 }
 
-// prefix[k] = sum of sums[0..k) for k <= nchunks; one workgroup of 1024 threads,
-// thread t owns a contiguous run of chunks.
-__global__ void __launch_bounds__(1024) k_chunk_scan(const double* sums, uint64_t nchunks, double* prefix) {
-  __shared__ double part[1024];
-  const uint64_t per = (nchunks + 1023) / 1024;
-  const uint64_t b = threadIdx.x * per, e = std::min<uint64_t>(b + per, nchunks);
-  double t = 0.0;
-  for (uint64_t k = b; k < e; k++) t += sums[k];
-  part[threadIdx.x] = t;
-  __syncthreads();
-  if (threadIdx.x == 0) {  // exclusive scan of the 1024 run totals, in order
-    double run = 0.0;
-    for (int i = 0; i < 1024; i++) {
-      const double v = part[i];
-      part[i] = run;
-      run += v;
-    }
-    prefix[nchunks] = run;
+// Inclusive scan of x over the workgroup's 256 threads, fixed order; *total
+// gets the sum.
+__device__ __forceinline__ double block_scan(double x, double* total) {
+  __shared__ double wsum[4];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double v = __shfl_up(x, o, 64);
+    if (lane >= o) x += v;
   }
   __syncthreads();
-  double run = part[threadIdx.x];
-  for (uint64_t k = b; k < e; k++) {
-    prefix[k] = run;
-    run += sums[k];
-  }
+  if (lane == 63) wsum[w] = x;
+  __syncthreads();
+  double before = 0.0;
+  for (int i = 0; i < w; i++) before += wsum[i];
+  *total = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+  return before + x;
 }
 
-// One wavefront per shot.  u: device uniforms (or null: every shot takes u0).
+// pre[k]: sum of this workgroup's chunks before k (in place of the sums);
+// off[b]: sum of the workgroups before b, off[gridDim.x] = T.  One workgroup
+// over all chunks took 20 us at 8192 chunks and grew with them.
+__global__ void __launch_bounds__(256) k_chunk_scan(double* pre, uint64_t nchunks, double* off, unsigned* count) {
+  __shared__ int last;
+  const uint64_t b0 = (uint64_t)blockIdx.x * kScanRun;
+  constexpr int P = kScanRun / 256;  // consecutive chunks per thread
+  double x[P], mine = 0.0, total;
+#pragma unroll
+  for (int i = 0; i < P; i++) {
+    const uint64_t k = b0 + (uint64_t)threadIdx.x * P + i;
+    x[i] = k < nchunks ? pre[k] : 0.0;
+    mine += x[i];
+  }
+  double run = block_scan(mine, &total) - mine;
+#pragma unroll
+  for (int i = 0; i < P; i++) {
+    const uint64_t k = b0 + (uint64_t)threadIdx.x * P + i;
+    if (k < nchunks) pre[k] = run;
+    run += x[i];
+  }
+  if (threadIdx.x == 0) {
+    // the totals cross the XCDs' caches: complete before the count is raised
+    __hip_atomic_store(off + blockIdx.x, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  double base = 0.0;
+  for (unsigned b = 0; b < gridDim.x; b += 256) {
+    const unsigned k = b + threadIdx.x;
+    const double v =
+        k < gridDim.x ? __hip_atomic_load(off + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+    double sum;
+    const double incl = block_scan(v, &sum);
+    __syncthreads();
+    if (k < gridDim.x) off[k] = base + (incl - v);
+    base += sum;
+  }
+  if (threadIdx.x == 0) off[gridDim.x] = base;
+}
+
+// Where a shot's uniform comes from: the caller's array, one value for all
+// (u null), or the counter stream u(seed, traj, draw0 + shot).
+struct Uniforms {
+  const double* u;
+  double u0;
+  uint64_t seed, traj, draw0;
+  int stream;
+};
+
+// One wavefront per shot.
 template <typename R>
-__global__ void __launch_bounds__(256) k_sample_find(const C<R>* s, uint64_t n, const double* prefix,
-                                                     uint64_t nchunks, const double* u, double u0, int64_t shots,
-                                                     uint64_t* out, uint8_t* flag) {
+__global__ void __launch_bounds__(256) k_sample_find(const C<R>* s, uint64_t n, const double* pre, const double* off,
+                                                     uint64_t nchunks, Uniforms un, int64_t shots, uint64_t* out,
+                                                     uint8_t* flag) {
+  constexpr int E = kRowEntries<R> / 64, ROWS = kChunk / kRowEntries<R>;
   const int lane = threadIdx.x & 63;
   const int64_t shot = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (shot >= shots) return;  // whole wavefronts leave together
-  const double T = prefix[nchunks];
-  const double tgt = (u ? u[shot] : u0) * T;
-  // largest k < nchunks with prefix[k] <= tgt
-  uint64_t lo = 0, hi = nchunks;
+  const uint64_t nrun = (nchunks + kScanRun - 1) / kScanRun;
+  const double T = off[nrun];
+  const double u = un.stream ? uniform(un.seed, un.traj, un.draw0 + (uint64_t)shot) : un.u ? un.u[shot] : un.u0;
+  const double tgt = u * T;
+  // largest run, then largest chunk in it, that starts at or below the target
+  uint64_t lo = 0, hi = nrun;
   while (hi - lo > 1) {
     const uint64_t mid = lo + (hi - lo) / 2;
-    if (prefix[mid] <= tgt) lo = mid;
+    if (off[mid] <= tgt) lo = mid;
     else hi = mid;
   }
-  const uint64_t base = lo * kChunk + (uint64_t)lane * kLaneRun;
-  double p[kLaneRun];
-  double mine = 0.0;
-#pragma unroll
-  for (int j = 0; j < kLaneRun; j++) {
-    const uint64_t i = base + j;
-    p[j] = i < n ? prob<R>(s, i) : 0.0;
-    mine += p[j];
+  const double o0 = off[lo];
+  lo *= kScanRun;
+  hi = std::min<uint64_t>(lo + kScanRun, nchunks);
+  while (hi - lo > 1) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    if (o0 + pre[mid] <= tgt) lo = mid;
+    else hi = mid;
   }
-  // inclusive scan of the lane totals in lane order (Hillis-Steele)
+  const uint64_t base = lo * kChunk;
+  double p[ROWS][E];
+#pragma unroll
+  for (int r = 0; r < ROWS; r++) row_weights<R, E>(s, n, base, r, lane, p[r]);
+  // the first row that ends past the target; if rounding leaves none, the
+  // last entry holding probability
+  double c = o0 + pre[lo], before = c;
+  int row = -1, last_row = -1;
+  double last_before = c;
+#pragma unroll
+  for (int r = 0; r < ROWS; r++) {
+    if (row >= 0) continue;  // the same in every lane
+    double q = p[r][0];
+    if (E > 1) q += p[r][E - 1];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
+    if (q > 0.0) {
+      last_row = r;
+      last_before = c;
+    }
+    if (q > 0.0 && c + q > tgt) {
+      row = r;
+      before = c;
+    }
+    c += q;
+  }
+  const bool past = row < 0;
+  if (past) {
+    row = last_row;
+    before = last_before;
+  }
+  if (row < 0) {  // a chunk without probability (a state of zeros or NaN)
+    if (lane == 0) {
+      out[shot] = 0;
+      flag[shot] = 1;
+    }
+    return;
+  }
+  double w[E];
+#pragma unroll
+  for (int e = 0; e < E; e++) w[e] = 0.0;
+#pragma unroll
+  for (int r = 0; r < ROWS; r++)
+    if (r == row)
+#pragma unroll
+      for (int e = 0; e < E; e++) w[e] = p[r][e];
+  double mine = w[0];
+  if (E > 1) mine += w[E - 1];
   double incl = mine;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const double v = __shfl_up(incl, o, 64);
     if (lane >= o) incl += v;
   }
-  const double excl = incl - mine;
-  const double c0 = prefix[lo];
-  // first lane whose run ends past the target; if rounding leaves none, the
-  // last lane holding probability
-  const uint64_t hit = __ballot(c0 + incl > tgt && mine > 0.0);
+  const uint64_t hit = past ? 0 : __ballot(before + incl > tgt && mine > 0.0);
   const uint64_t nz = __ballot(mine > 0.0);
-  int src;
-  if (hit) src = __builtin_ctzll(hit);
-  else if (nz) src = 63 - __builtin_clzll(nz);
-  else src = -1;
-  if (lane == (src < 0 ? 0 : src)) {
-    uint64_t idx = 0;
-    double lo_c = c0 + excl, hi_c = lo_c;
-    if (src >= 0) {
-      int pick = -1, last = -1;
-      double run = c0 + excl, last_lo = run, last_hi = run;
+  const int src = hit ? __builtin_ctzll(hit) : 63 - __builtin_clzll(nz);
+  if (lane == src) {
+    const double l0 = before + (incl - mine);
+    int pick = -1, fall = 0;
+    double run = l0, lo_c = l0, hi_c = l0, fall_lo = l0, fall_hi = l0;
 #pragma unroll
-      for (int j = 0; j < kLaneRun; j++) {
-        const double nxt = run + p[j];
-        if (p[j] > 0.0) {
-          last = j;
-          last_lo = run;
-          last_hi = nxt;
-          if (pick < 0 && tgt < nxt) {
-            pick = j;
-            lo_c = run;
-            hi_c = nxt;
-          }
+    for (int e = 0; e < E; e++) {
+      const double nxt = run + w[e];
+      if (w[e] > 0.0) {
+        fall = e;
+        fall_lo = run;
+        fall_hi = nxt;
+        if (hit && pick < 0 && tgt < nxt) {
+          pick = e;
+          lo_c = run;
+          hi_c = nxt;
         }
-        run = nxt;
       }
-      if (pick < 0) {  // past the end by rounding: the last entry with probability
-        pick = last;
-        lo_c = last_lo;
-        hi_c = last_hi;
-      }
-      idx = base + pick;
+      run = nxt;
     }
-    out[shot] = idx;
-    flag[shot] = (src < 0 || tgt - lo_c < kBoundaryTol * T || hi_c - tgt < kBoundaryTol * T) ? 1 : 0;
+    if (pick < 0) {  // past the end by rounding: the last entry with probability
+      pick = fall;
+      lo_c = fall_lo;
+      hi_c = fall_hi;
+    }
+    out[shot] = base + (uint64_t)row * kRowEntries<R> + (uint64_t)(E * lane + pick);
+    flag[shot] = (tgt - lo_c < kBoundaryTol * T || hi_c - tgt < kBoundaryTol * T) ? 1 : 0;
   }
 }
 
+static uint64_t chunks_of(int nbits) { return ((1ull << nbits) + kChunk - 1) / kChunk; }
+static uint64_t runs_of(uint64_t nchunks) { return (nchunks + kScanRun - 1) / kScanRun; }
+
+// chunk sums / prefix, the runs' offsets and the total, the scan's counter
 size_t sample_scratch_bytes(int nbits) {
-  const uint64_t n = 1ull << nbits;
-  const uint64_t nchunks = (n + kChunk - 1) / kChunk;
-  return sizeof(double) * (2 * nchunks + 1);
+  const uint64_t nchunks = chunks_of(nbits);
+  return sizeof(double) * (nchunks + runs_of(nchunks) + 2);
+}
+
+template <typename R>
+static void launch_sample_t(const void* state, int nbits, hipStream_t st, void* scratch, int64_t shots,
+                            const Uniforms& un, uint64_t* d_out, uint8_t* d_flag) {
+  const uint64_t n = 1ull << nbits, nchunks = chunks_of(nbits), nrun = runs_of(nchunks);
+  double* pre = (double*)scratch;
+  double* off = pre + nchunks;
+  unsigned* count = (unsigned*)(off + nrun + 1);
+  const unsigned g1 = (unsigned)std::min<uint64_t>((nchunks + 3) / 4, 1u << 16);
+  hipLaunchKernelGGL(k_chunk_sums<R>, dim3(g1), dim3(256), 0, st, (const C<R>*)state, n, nchunks, pre, count);
+  hipLaunchKernelGGL(k_chunk_scan, dim3((unsigned)nrun), dim3(256), 0, st, pre, nchunks, off, count);
+  hipLaunchKernelGGL(k_sample_find<R>, dim3((unsigned)((shots + 3) / 4)), dim3(256), 0, st, (const C<R>*)state, n,
+                     (const double*)pre, (const double*)off, nchunks, un, shots, d_out, d_flag);
+}
+
+static int launch_sample_u(const void* state, int prec, int nbits, hipStream_t st, void* scratch, int64_t shots,
+                           const Uniforms& un, uint64_t* d_out, uint8_t* d_flag) {
+  if (prec == BT_C64) launch_sample_t<float>(state, nbits, st, scratch, shots, un, d_out, d_flag);
+  else launch_sample_t<double>(state, nbits, st, scratch, shots, un, d_out, d_flag);
+  BT_HIP(hipGetLastError());
+  return BT_OK;
 }
 
 int launch_sample(const void* state, int prec, int nbits, hipStream_t st, void* scratch, int64_t shots,
                   const double* d_u, double u0, uint64_t* d_out, uint8_t* d_flag) {
-  const uint64_t n = 1ull << nbits;
-  const uint64_t nchunks = (n + kChunk - 1) / kChunk;
-  double* sums = (double*)scratch;
-  double* prefix = sums + nchunks;
-  const unsigned g1 = (unsigned)std::min<uint64_t>((nchunks + 3) / 4, 1u << 16);
-  const unsigned g3 = (unsigned)((shots + 3) / 4);
-  if (prec == BT_C64) {
-    hipLaunchKernelGGL(k_chunk_sums<float>, dim3(g1), dim3(256), 0, st, (const C<float>*)state, n, nchunks, sums);
-    hipLaunchKernelGGL(k_chunk_scan, dim3(1), dim3(1024), 0, st, (const double*)sums, nchunks, prefix);
-    hipLaunchKernelGGL(k_sample_find<float>, dim3(g3), dim3(256), 0, st, (const C<float>*)state, n,
-                       (const double*)prefix, nchunks, d_u, u0, shots, d_out, d_flag);
-  } else {
-    hipLaunchKernelGGL(k_chunk_sums<double>, dim3(g1), dim3(256), 0, st, (const C<double>*)state, n, nchunks, sums);
-    hipLaunchKernelGGL(k_chunk_scan, dim3(1), dim3(1024), 0, st, (const double*)sums, nchunks, prefix);
-    hipLaunchKernelGGL(k_sample_find<double>, dim3(g3), dim3(256), 0, st, (const C<double>*)state, n,
-                       (const double*)prefix, nchunks, d_u, u0, shots, d_out, d_flag);
+  return launch_sample_u(state, prec, nbits, st, scratch, shots, Uniforms{d_u, u0, 0, 0, 0, 0}, d_out, d_flag);
+}
+
+// What bt_sample keeps with a state: device scratch and a pinned buffer (the
+// uniforms in, indices and flags out, read and written by the kernels in
+// place), so that a call is three launches and one wait.  At most
+// kSampleKeep bytes of each; a larger request allocates for itself.
+constexpr size_t kSampleKeep = 32ull << 20;
+
+struct SampleBuffers {
+  void* dev = nullptr;
+  void* host = nullptr;
+  size_t dev_bytes = 0, host_bytes = 0;
+};
+
+static void free_buffers(SampleBuffers* b) {
+  if (b->dev) (void)hipFree(b->dev);
+  if (b->host) (void)hipHostFree(b->host);
+  *b = SampleBuffers();
+}
+
+void free_sample_res(SampleBuffers* b) {
+  if (!b) return;
+  free_buffers(b);
+  delete b;
+}
+
+static bool grow_buffers(SampleBuffers* b, size_t dev, size_t host) {
+  if (dev > b->dev_bytes) {
+    if (b->dev) (void)hipFree(b->dev);
+    b->dev = nullptr;
+    b->dev_bytes = 0;
+    if (hipMalloc(&b->dev, dev) != hipSuccess) return false;
+    b->dev_bytes = dev;
   }
-  BT_HIP(hipGetLastError());
-  return BT_OK;
+  if (host > b->host_bytes) {
+    if (b->host) (void)hipHostFree(b->host);
+    b->host = nullptr;
+    b->host_bytes = 0;
+    if (hipHostMalloc(&b->host, host) != hipSuccess) return false;
+    b->host_bytes = host;
+  }
+  return true;
+}
+
+// Shots of state s with uniforms u (or un's stream): indices and the number
+// flagged as near a boundary.
+static int sample_shots(bt_state_s* s, int64_t shots, const double* u, Uniforms un, uint64_t* out, int64_t* nboundary) {
+  const size_t sc = sample_scratch_bytes(s->nbits);
+  const size_t ub = u ? sizeof(double) * (size_t)shots : 0, ob = sizeof(uint64_t) * (size_t)shots;
+  const size_t host = ub + ob + (size_t)shots;
+  SampleBuffers own;
+  SampleBuffers* b = &own;
+  if (sc <= kSampleKeep && host <= kSampleKeep) {  // powers of two: a few sizes over a state's life
+    if (!s->sample) s->sample = new SampleBuffers();
+    b = s->sample;
+  }
+  auto up = [&](size_t x) {
+    if (b == &own) return x;
+    size_t p = 4096;
+    while (p < x) p *= 2;
+    return p;
+  };
+  if (!grow_buffers(b, up(sc), up(host))) {
+    (void)hipGetLastError();
+    free_buffers(&own);
+    return fail(BT_ERR_NOMEM, "bt_sample: buffers");
+  }
+  if (u) {
+    memcpy(b->host, u, ub);
+    un.u = (const double*)b->host;
+  }
+  uint64_t* h_out = (uint64_t*)((char*)b->host + ub);
+  uint8_t* h_flag = (uint8_t*)b->host + ub + ob;
+  int rc = launch_sample_u(s->d, s->prec, s->nbits, s->stream, b->dev, shots, un, h_out, h_flag);
+  if (hipStreamSynchronize(s->stream) != hipSuccess && rc == BT_OK) rc = fail(BT_ERR_HIP, "bt_sample: sync");
+  if (rc == BT_OK) {
+    memcpy(out, h_out, ob);
+    int64_t nb = 0;
+    for (int64_t i = 0; i < shots; i++) nb += h_flag[i];
+    if (nboundary) *nboundary = nb;
+  }
+  free_buffers(&own);
+  return rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -282,28 +476,17 @@ extern "C" int bt_sample(bt_state s, int64_t shots, const double* u, uint64_t* o
   }
   for (int64_t i = 0; i < shots; i++)
     if (!(u[i] >= 0.0 && u[i] < 1.0)) return fail(BT_ERR_ARG, "bt_sample: uniforms must lie in [0, 1)");
-  const size_t sc = sample_scratch_bytes(s->nbits);
-  const size_t ub = sizeof(double) * shots, ob = sizeof(uint64_t) * shots, fb = (size_t)shots;
-  char* buf = nullptr;
-  if (hipMalloc((void**)&buf, sc + ub + ob + fb + 64) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(BT_ERR_NOMEM, "bt_sample: device buffers");
+  return sample_shots(s, shots, u, Uniforms{nullptr, 0.0, 0, 0, 0, 0}, out, nboundary);
+}
+
+extern "C" int bt_sample_stream(bt_state s, int64_t shots, uint64_t seed, uint64_t traj, uint64_t draw0, uint64_t* out,
+                                int64_t* nboundary) {
+  if (!s) return fail(BT_ERR_ARG, "null state");
+  if (s->kind != BT_SV) return fail(BT_ERR_UNSUPPORTED, "bt_sample_stream: state vectors only (sample, ops.jl:46-60)");
+  if (shots < 0 || (shots > 0 && !out)) return fail(BT_ERR_ARG, "bt_sample_stream: bad arguments");
+  if (shots == 0) {
+    if (nboundary) *nboundary = 0;
+    return BT_OK;
   }
-  double* d_u = (double*)(buf + sc);
-  uint64_t* d_out = (uint64_t*)(buf + sc + ub);
-  uint8_t* d_flag = (uint8_t*)(buf + sc + ub + ob);
-  std::vector<uint8_t> flags(shots);
-  int rc = BT_OK;
-  if (hipMemcpyAsync(d_u, u, ub, hipMemcpyHostToDevice, s->stream) != hipSuccess) rc = fail(BT_ERR_HIP, "bt_sample: upload");
-  if (rc == BT_OK) rc = launch_sample(s->d, s->prec, s->nbits, s->stream, buf, shots, d_u, 0.0, d_out, d_flag);
-  if (rc == BT_OK && (hipMemcpyAsync(out, d_out, ob, hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-                      hipMemcpyAsync(flags.data(), d_flag, fb, hipMemcpyDeviceToHost, s->stream) != hipSuccess))
-    rc = fail(BT_ERR_HIP, "bt_sample: download");
-  if (hipStreamSynchronize(s->stream) != hipSuccess && rc == BT_OK) rc = fail(BT_ERR_HIP, "bt_sample: sync");
-  (void)hipFree(buf);
-  if (rc) return rc;
-  int64_t nb = 0;
-  for (int64_t i = 0; i < shots; i++) nb += flags[i];
-  if (nboundary) *nboundary = nb;
-  return BT_OK;
+  return sample_shots(s, shots, nullptr, Uniforms{nullptr, 0.0, seed, traj, draw0, 1}, out, nboundary);
 }

@@ -24,7 +24,7 @@ from typing import Optional, Sequence, Union
 import numpy as np
 
 from . import _lib as L
-from .core import StateVector, current_stream, zero_state
+from .core import StateVector, UniformStream, current_stream, zero_state
 from .gates import gate
 from .noise import QuantumChannel
 from .ops import Op, OpQC, QuantumOps
@@ -66,10 +66,33 @@ def sample_with(state: StateVector, u) -> (np.ndarray, int):
     return out.astype(np.int64), nb.value
 
 
+def _sample_stream(state: StateVector, shots: int, seed: int, traj: int, draw: int):
+    """sample_with on the uniforms u(seed, traj, draw), u(seed, traj, draw + 1),
+    ..., formed on the device."""
+    if not isinstance(state, StateVector):
+        raise TypeError("sample takes a state vector (ops.jl:46)")
+    out = np.zeros(max(int(shots), 0), dtype=np.uint64)
+    nb = ctypes.c_int64()
+    L.check(L.lib().bt_sample_stream(state.handle, int(shots), seed, traj, draw,
+                                     out.ctypes.data_as(ctypes.POINTER(ctypes.c_uint64)), ctypes.byref(nb)))
+    return out.astype(np.int64), nb.value
+
+
+def _sample_rng(state: StateVector, shots: int, rng=None):
+    """`shots` shots on the next draws of rng (the current stream)."""
+    rng = rng or current_stream()
+    shots = int(shots)
+    if type(rng) is UniformStream and shots > 0:  # a subclass or another callable draws for itself
+        r = _sample_stream(state, shots, rng.seed_value, rng.traj, rng.draw)
+        rng.draw += shots
+        return r
+    return sample_with(state, _draws(shots, rng))
+
+
 def sample(state: StateVector, shots: int, rng=None) -> np.ndarray:
     """sample(state, shots) (ops.jl:46-60): `shots` basis indices drawn from
     |psi|^2."""
-    return sample_with(state, _draws(shots, rng))[0]
+    return _sample_rng(state, shots, rng)[0]
 
 
 def get_probs_from_sample(sample_: Sequence[int], N: int):
@@ -127,7 +150,7 @@ def measure(x, number_of_experiment: int = -1, N: Optional[int] = None, label="s
             p = x.probabilities()
             nz = np.nonzero(p)[0]
             return _record(nz, p[nz], n, "0", -1, label)
-        idx, nb = sample_with(x, _draws(number_of_experiment, rng))
+        idx, nb = _sample_rng(x, number_of_experiment, rng)
         b, p = get_probs_from_sample(idx, n)
         return _record(b, p, n, "0", number_of_experiment, label, nb)
     if N is None:
@@ -205,7 +228,7 @@ def measure_circuit(circuit_or_ops, number_of_experiment: int, N: Optional[int] 
     if noiseless:
         st = zero_state(n, prec)
         _, used, _ = run_shot(cc, st, seed, 0, 0, final)
-        idx, nb = sample_with(st, _uniforms(seed, 0, used, number_of_experiment))
+        idx, nb = _sample_stream(st, number_of_experiment, seed, 0, used)
     elif not opts.twirl:
         c = Circuit(cc.ops_for_shot(id) + final, n, opts.noise)
         idx, nb = c.run_batch_sample(number_of_experiment, seed=seed, prec=prec)

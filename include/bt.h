@@ -142,6 +142,10 @@ int bt_expect_each(bt_state s, int pauli, double* out);
  * decide.  Replaces sample(state, shots) (ops.jl:46-60; StatsBase.sample
  * with Weights, whose RNG the explicit uniforms stand in for). */
 int bt_sample(bt_state s, int64_t shots, const double* u, uint64_t* out, int64_t* nboundary);
+/* bt_sample with shot i's uniform taken from the counter stream,
+ * bt_uniform(seed, traj, draw0 + i), generated where it is used. */
+int bt_sample_stream(bt_state s, int64_t shots, uint64_t seed, uint64_t traj, uint64_t draw0, uint64_t* out,
+                     int64_t* nboundary);
 /* bt_sample without any allocation: the same kernels, results and errors,
  * with every device buffer (chunk sums, prefix, uniforms, indices, flags) in
  * one static 32 MiB device array per GPU (a 2^30-amplitude state with about
