@@ -453,6 +453,7 @@ struct bt_circuit_s {
   struct StaticPlan {
     int T = -1, prec = -1, cb = -1;
     size_t tabsz = 0;
+    bool phases = false;  // every pass has operators
     std::vector<unsigned char> tables;
     std::vector<uint8_t> narrow;
   } dm_plan, sv_plan;

@@ -152,7 +152,18 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_grid_pass
   if (threadIdx.x < kAcc) sums[threadIdx.x] = 0.0;
   tile_pass<R, O>(state, GeomConst(tab, sizeof(C<R>)), staged, tile, blockIdx.x, gridDim.x, ntiles,
                   red, sums);
-  if (threadIdx.x < kAcc) part[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = sums[threadIdx.x];
+  if (part && threadIdx.x < kAcc) part[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = sums[threadIdx.x];
+}
+
+// All passes of a state that is one tile in one launch (static plans: no
+// reductions): the launches between them, their cold tables and the trip of
+// the tile through memory cost more than a third of a 12-qubit circuit.
+template <typename R>
+__global__ void __launch_bounds__(TileCfg<R>::NT, 1) k_one_tile(C<R>* state, const unsigned char* tab,
+                                                                uint32_t stride, int npass) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ __align__(16) C<R> staged[2 * kStageEntries<R>];
+  one_tile_passes<R>(state, tab, stride, npass, staged, (C<R>*)smem);
 }
 
 // out[j] = fixed-order sum of the grid's partials of accumulator j
@@ -234,17 +245,25 @@ static unsigned grid_pass_blocks(uint64_t ntiles) {
 }
 
 constexpr int kRing = 8;  // pass tables in flight
+constexpr size_t kTabKeep = 16ull << 20;
 
 // The circuit executor's staging of a state, made on its first run and kept
 // until the state is destroyed (a state is used by one host thread at a
-// time): pinned and device rings of pass tables, reduction partials for the
-// widest grid, the finished sums and their pinned copy, events.
+// time): what a static plan needs, and with the first circuit that decides
+// on reductions pinned and device rings of pass tables, reduction partials
+// for the widest grid, the finished sums and their pinned copy, events.
 struct GridRes {
   void* h_ring = nullptr;
   void* d_ring = nullptr;
   double* d_part = nullptr;
   double* d_acc = nullptr;
   double* h_acc = nullptr;
+  // a static plan's tables: pinned and device, reused once the copy / the
+  // launches that read them are done; at most kTabKeep bytes are kept
+  void* h_tab = nullptr;
+  void* d_tab = nullptr;
+  size_t tab_bytes = 0;
+  hipEvent_t tab_done = nullptr;
   hipEvent_t ev[kRing] = {};
   hipEvent_t e0 = nullptr, e1 = nullptr;
 };
@@ -255,6 +274,9 @@ void free_grid_res(GridRes* g) {
     if (g->ev[i]) (void)hipEventDestroy(g->ev[i]);
   if (g->e0) (void)hipEventDestroy(g->e0);
   if (g->e1) (void)hipEventDestroy(g->e1);
+  if (g->tab_done) (void)hipEventDestroy(g->tab_done);
+  if (g->h_tab) (void)hipHostFree(g->h_tab);
+  if (g->d_tab) (void)hipFree(g->d_tab);
   if (g->h_ring) (void)hipHostFree(g->h_ring);
   if (g->h_acc) (void)hipHostFree(g->h_acc);
   if (g->d_ring) (void)hipFree(g->d_ring);
@@ -275,33 +297,44 @@ static bool pass_narrow(int prec, const TableHead& h) {
   return prec == BT_C64 ? narrow_io<float>(h) : narrow_io<double>(h);
 }
 
-static int grid_res(bt_state_s* s, GridRes** out) {
+// ring: also the rings and reduction buffers of run_grid
+static int grid_res(bt_state_s* s, bool ring, GridRes** out) {
   if (!s->grid) {
-    const size_t tabsz = table_max(s->prec);
-    const int cus = ctx().cus > 0 ? ctx().cus : 256;
     auto* g = new GridRes();
-    bool ok = hipHostMalloc(&g->h_ring, tabsz * kRing) == hipSuccess &&
-              hipMalloc(&g->d_ring, tabsz * kRing) == hipSuccess &&
-              hipMalloc((void**)&g->d_part, sizeof(double) * kAcc * (size_t)cus * 8) == hipSuccess &&
-              hipMalloc((void**)&g->d_acc, sizeof(double) * kAcc) == hipSuccess &&
-              hipHostMalloc((void**)&g->h_acc, sizeof(double) * kAcc) == hipSuccess;
-    for (int i = 0; i < kRing && ok; i++) ok = hipEventCreateWithFlags(&g->ev[i], hipEventDisableTiming) == hipSuccess;
-    ok = ok && hipEventCreate(&g->e0) == hipSuccess && hipEventCreate(&g->e1) == hipSuccess;
-    if (!ok) {
+    if (hipEventCreate(&g->e0) != hipSuccess || hipEventCreate(&g->e1) != hipSuccess ||
+        hipEventCreateWithFlags(&g->tab_done, hipEventDisableTiming) != hipSuccess) {
       (void)hipGetLastError();
       free_grid_res(g);
       return fail(BT_ERR_NOMEM, "run_grid: allocation failed");
     }
     s->grid = g;
   }
-  *out = s->grid;
+  GridRes* g = s->grid;
+  if (ring && !g->h_acc) {
+    const size_t tabsz = table_max(s->prec);
+    const int cus = ctx().cus > 0 ? ctx().cus : 256;
+    bool ok = hipHostMalloc(&g->h_ring, tabsz * kRing) == hipSuccess &&
+              hipMalloc(&g->d_ring, tabsz * kRing) == hipSuccess &&
+              hipMalloc((void**)&g->d_part, sizeof(double) * kAcc * (size_t)cus * 8) == hipSuccess &&
+              hipMalloc((void**)&g->d_acc, sizeof(double) * kAcc) == hipSuccess;
+    for (int i = 0; i < kRing && ok; i++) ok = hipEventCreateWithFlags(&g->ev[i], hipEventDisableTiming) == hipSuccess;
+    ok = ok && hipHostMalloc((void**)&g->h_acc, sizeof(double) * kAcc) == hipSuccess;
+    if (!ok) {
+      (void)hipGetLastError();
+      free_grid_res(g);
+      s->grid = nullptr;
+      return fail(BT_ERR_NOMEM, "run_grid: allocation failed");
+    }
+  }
+  *out = g;
   return BT_OK;
 }
 
-// Host driver of the interpreter over grid passes on state s (SV or DM).
+// Host driver of the interpreter over grid passes on state s (SV or DM), whose
+// norm^2 is r0.
 static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, uint64_t traj, const double* uni,
                     int64_t nuni, int32_t* outs, int64_t outcap, int64_t* nout, bt_run_stats* stats, int fold,
-                    int prec_tile_T) {
+                    int prec_tile_T, double r0 = 1.0) {
   const int nbits = s->nbits;
   std::vector<QOp> slots(bti::kQMax);
   std::unique_ptr<bti::Interp> ip(new bti::Interp());
@@ -317,12 +350,13 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
   ip->outs = outs;
   ip->outcap = outcap;
   ip->fold = fold;
+  ip->r = r0;
   ip->tol_exact = s->prec == BT_C64 ? 1e-6 : 1e-12;
   const size_t tabsz = table_max(s->prec);
   const uint64_t ntiles = 1ull << (nbits - std::min(T, nbits));
   const unsigned blocks = grid_pass_blocks(ntiles);
   GridRes* gr = nullptr;
-  int rc = grid_res(s, &gr);
+  int rc = grid_res(s, true, &gr);
   if (rc) return rc;
   void* const h_ring = gr->h_ring;
   void* const d_ring = gr->d_ring;
@@ -405,10 +439,11 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
 
 // Pass tables of a circuit whose pass plan does not depend on reductions
 // (a density matrix: no sampling, no renormalisation, fold = 0), planned on
-// the host once: tables gets npass packed tables, *tabsz bytes apart,
+// the host once: tables gets npass packed tables, *tabsz bytes apart, *phases
+// (nullable) whether every pass has operators,
 // narrow[i] whether pass i's per-thread byte offsets fit 32 bits.
 int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::vector<unsigned char>* tables,
-                       std::vector<uint8_t>* narrow, size_t* tabsz) {
+                       std::vector<uint8_t>* narrow, size_t* tabsz, bool* phases) {
   const int nbits = s->nbits;
   std::vector<QOp> slots(bti::kQMax);
   std::unique_ptr<bti::Interp> ip(new bti::Interp());
@@ -420,6 +455,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
   std::vector<unsigned char> packed, one(table_max(s->prec));
   std::vector<size_t> size;
   *tabsz = 16;
+  if (phases) *phases = true;
   Plan plan;
   PassResult res;
   memset(&res, 0, sizeof res);
@@ -436,6 +472,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
     size.push_back(bytes);
     *tabsz = std::max(*tabsz, (bytes + 15) / 16 * 16);
     narrow->push_back(pass_narrow(s->prec, head) ? 1 : 0);
+    if (phases) *phases = *phases && head.nph > 0;
     memset(&res, 0, sizeof res);
   }
   if (ip->err) return fail(ip->err, "plan_static_passes: interpreter error (" + std::to_string(ip->err) + ")");
@@ -446,7 +483,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
 }
 
 // Enqueue one grid pass of state s (tile bits T) with its table at dtab;
-// d_part: kAcc x grid doubles of reduction partials (written, unused here).
+// d_part: kAcc x grid doubles of reduction partials (null: none are wanted).
 int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part) {
   const int nbits = s->nbits;
   const uint64_t ntiles = 1ull << (nbits - std::min(T, nbits));
@@ -475,7 +512,7 @@ int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double
 // on states like s: planned once per tiling and kept in the circuit's slot,
 // copied out for this run.
 static int static_plan(bt_state_s* s, bt_circuit_s* c, bool dm, int T, std::vector<unsigned char>* tables,
-                       std::vector<uint8_t>* narrow, size_t* tabsz) {
+                       std::vector<uint8_t>* narrow, size_t* tabsz, bool* phases) {
   const int cb = coalesce_bits(s->prec);
   std::lock_guard<std::mutex> lk(c->mu);
   bt_circuit_s::StaticPlan* P = dm ? &c->dm_plan : &c->sv_plan;
@@ -487,9 +524,9 @@ static int static_plan(bt_state_s* s, bt_circuit_s* c, bool dm, int T, std::vect
       std::string msg;
       rc = lower_dm(c->h, &lowered, &msg);
       if (rc) return fail(rc, msg);
-      rc = plan_static_passes(s, lowered, T, &P->tables, &P->narrow, &P->tabsz);
+      rc = plan_static_passes(s, lowered, T, &P->tables, &P->narrow, &P->tabsz, &P->phases);
     } else {
-      rc = plan_static_passes(s, c->h, T, &P->tables, &P->narrow, &P->tabsz);
+      rc = plan_static_passes(s, c->h, T, &P->tables, &P->narrow, &P->tabsz, &P->phases);
     }
     if (rc) return rc;
     P->T = T;
@@ -499,41 +536,97 @@ static int static_plan(bt_state_s* s, bt_circuit_s* c, bool dm, int T, std::vect
   *tables = P->tables;
   *narrow = P->narrow;
   *tabsz = P->tabsz;
+  *phases = P->phases;
   return BT_OK;
+}
+
+// Enqueue a static plan on state s: the tables in one copy, the passes back
+// to back with no host round trip between them, or in one launch when the
+// state is one tile.  The tables are staged in buffers kept with the state.
+// timed: record gr->e0 / e1 around the passes.
+static int enqueue_static(bt_state_s* s, const std::vector<unsigned char>& tables, const std::vector<uint8_t>& narrow,
+                          size_t tabsz, int T, bool one_launch, GridRes* gr, bool timed) {
+  if (tables.empty()) {
+    if (timed) {
+      (void)hipEventRecord(gr->e0, s->stream);
+      (void)hipEventRecord(gr->e1, s->stream);
+    }
+    return BT_OK;
+  }
+  BT_HIP(hipEventSynchronize(gr->tab_done));  // earlier launches from these buffers are done
+  if (tables.size() > gr->tab_bytes) {
+    if (gr->h_tab) (void)hipHostFree(gr->h_tab);
+    if (gr->d_tab) (void)hipFree(gr->d_tab);
+    gr->h_tab = gr->d_tab = nullptr;
+    gr->tab_bytes = 0;
+    size_t want = 1 << 16;
+    while (want < tables.size()) want *= 2;
+    if (hipHostMalloc(&gr->h_tab, want) != hipSuccess || hipMalloc(&gr->d_tab, want) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(BT_ERR_NOMEM, "run: pass tables");
+    }
+    gr->tab_bytes = want;
+  }
+  memcpy(gr->h_tab, tables.data(), tables.size());
+  BT_HIP(hipMemcpyAsync(gr->d_tab, gr->h_tab, tables.size(), hipMemcpyHostToDevice, s->stream));
+  int rc = BT_OK;
+  const int Tn = std::min(T, s->nbits);
+  if (one_launch) {
+    const int lds = (int)(((size_t)1 << Tn) * s->elem());
+    if (timed) (void)hipEventRecord(gr->e0, s->stream);
+    if (s->prec == BT_C64) {
+      (void)hipFuncSetAttribute((const void*)k_one_tile<float>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      hipLaunchKernelGGL((k_one_tile<float>), dim3(1), dim3(TileCfg<float>::NT), lds, s->stream, (C<float>*)s->d,
+                         (const unsigned char*)gr->d_tab, (uint32_t)tabsz, (int)narrow.size());
+    } else {
+      (void)hipFuncSetAttribute((const void*)k_one_tile<double>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      hipLaunchKernelGGL((k_one_tile<double>), dim3(1), dim3(TileCfg<double>::NT), lds, s->stream, (C<double>*)s->d,
+                         (const unsigned char*)gr->d_tab, (uint32_t)tabsz, (int)narrow.size());
+    }
+    if (hipGetLastError() != hipSuccess) rc = fail(BT_ERR_HIP, "run: one-tile launch");
+  } else {
+    grid_pass_lds_attr(s->prec, Tn);
+    if (timed) (void)hipEventRecord(gr->e0, s->stream);
+    for (size_t i = 0; rc == BT_OK && i < narrow.size(); i++)
+      rc = launch_grid_pass(s, (const unsigned char*)gr->d_tab + i * tabsz, narrow[i] != 0, T, nullptr);
+  }
+  if (timed) (void)hipEventRecord(gr->e1, s->stream);
+  (void)hipEventRecord(gr->tab_done, s->stream);
+  return rc;
+}
+
+// Give back table buffers past what is kept (the stream is idle).
+static void trim_tables(GridRes* gr) {
+  if (gr->tab_bytes <= kTabKeep) return;
+  (void)hipHostFree(gr->h_tab);
+  (void)hipFree(gr->d_tab);
+  gr->h_tab = gr->d_tab = nullptr;
+  gr->tab_bytes = 0;
+}
+
+// Whether a static plan of state s runs as one launch: the state is one tile
+// and every pass has phases (a pass without operators has nothing to relay).
+static bool one_launch_plan(bt_state_s* s, const std::vector<uint8_t>& narrow, int T, bool phases) {
+  return phases && !narrow.empty() && s->nbits <= T;
 }
 
 // Passes whose plan depends on nothing they compute (a density matrix, a
 // gate-only state-vector circuit) run eagerly from tables planned on the
-// host beforehand: uploaded in one copy and launched back to back with no
-// host round trip between them.
+// host beforehand.
 static int run_static(bt_state_s* s, const std::vector<unsigned char>& tables, const std::vector<uint8_t>& narrow,
-                      size_t tabsz, int T, bt_run_stats* stats) {
+                      size_t tabsz, bool phases, int T, bt_run_stats* stats) {
   GridRes* gr = nullptr;
-  int rc = grid_res(s, &gr);
+  int rc = grid_res(s, false, &gr);
   if (rc) return rc;
-  void* d_tab = nullptr;
-  if (!tables.empty() && hipMalloc(&d_tab, tables.size()) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(BT_ERR_NOMEM, "run: pass tables");
-  }
-  if (d_tab && hipMemcpyAsync(d_tab, tables.data(), tables.size(), hipMemcpyHostToDevice, s->stream) != hipSuccess)
-    rc = fail(BT_ERR_HIP, "run: table upload");
-  grid_pass_lds_attr(s->prec, std::min(T, s->nbits));
-  if (rc == BT_OK) (void)hipEventRecord(gr->e0, s->stream);
-  for (size_t i = 0; rc == BT_OK && i < narrow.size(); i++)
-    rc = launch_grid_pass(s, (const unsigned char*)d_tab + i * tabsz, narrow[i] != 0, T, gr->d_part);
-  if (rc == BT_OK) {
-    (void)hipEventRecord(gr->e1, s->stream);
-    if (hipStreamSynchronize(s->stream) != hipSuccess) rc = fail(BT_ERR_HIP, "run: sync");
-  } else {
-    (void)hipStreamSynchronize(s->stream);  // the upload is done before the tables are freed
-  }
-  if (d_tab) (void)hipFree(d_tab);
+  const bool one = one_launch_plan(s, narrow, T, phases);
+  rc = enqueue_static(s, tables, narrow, tabsz, T, one, gr, true);
+  if (hipStreamSynchronize(s->stream) != hipSuccess && rc == BT_OK) rc = fail(BT_ERR_HIP, "run: sync");
+  trim_tables(gr);
   if (stats) {
     memset(stats, 0, sizeof *stats);
     stats->passes = (int64_t)narrow.size();
-    stats->bytes = 2.0 * (double)narrow.size() * (double)(1ull << s->nbits) * (double)s->elem();
-    stats->launches = (int64_t)narrow.size();
+    stats->bytes = 2.0 * (one ? 1.0 : (double)narrow.size()) * (double)(1ull << s->nbits) * (double)s->elem();
+    stats->launches = one ? 1 : (int64_t)narrow.size();
     float ms = 0;
     if (rc == BT_OK && hipEventElapsedTime(&ms, gr->e0, gr->e1) == hipSuccess) stats->kernel_ms = ms;
   }
@@ -622,10 +715,53 @@ int bt_run_circuit(bt_state s, bt_circuit c, uint64_t seed, uint64_t traj, const
   std::vector<unsigned char> tables;
   std::vector<uint8_t> narrow;
   size_t tabsz = 0;
-  rc = static_plan(s, c, false, T, &tables, &narrow, &tabsz);
+  bool phases = false;
+  rc = static_plan(s, c, false, T, &tables, &narrow, &tabsz, &phases);
   if (rc) return rc;
   if (nout) *nout = 0;
-  return run_static(s, tables, narrow, tabsz, T, stats);
+  return run_static(s, tables, narrow, tabsz, phases, T, stats);
+}
+
+int bt_apply_ops(bt_state s, const bt_ir_op* ops, int nops, const double* pool, int64_t npool, const double* uniforms,
+                 int64_t nuni, int* outcomes, int64_t outcap, int64_t* nout) {
+  if (!s) return fail(BT_ERR_ARG, "null state");
+  int rc = ensure_device();
+  if (rc) return rc;
+  if (s->kind != BT_SV) return fail(BT_ERR_UNSUPPORTED, "bt_apply_ops: state vectors only");
+  btc::CircuitHost ch;
+  std::string msg;
+  rc = btc::analyze(s->n, ops, nops, nops, pool, npool, &ch, &msg);
+  if (rc) return fail(rc, msg);
+  bool gates_only = true;
+  for (const bt_ir_op& op : ch.ops) gates_only = gates_only && op.kind == BT_OP_GATE;
+  if (nuni < ch.max_draws || (ch.max_draws > 0 && !uniforms))
+    return fail(BT_ERR_DRAWS, "too few uniforms for the operations");
+  if (nout) *nout = 0;
+  const int T = tile_bits_for(s->prec, s->nbits);
+  if (!gates_only) {
+    // probabilities are those of the state as it is: the interpreter starts
+    // from its norm
+    double n2 = 0;
+    rc = launch_norm2(s, &n2);
+    if (rc) return rc;
+    if (!(n2 > 0) || !std::isfinite(n2)) return fail(BT_ERR_STATE, "bt_apply_ops: the state has no norm");
+    return run_grid(s, ch, 0, 0, uniforms, nuni, outcomes, outcap, nout, nullptr, 1, T, n2);
+  }
+  std::vector<unsigned char> tables;
+  std::vector<uint8_t> narrow;
+  size_t tabsz = 0;
+  bool phases = false;
+  rc = plan_static_passes(s, ch, T, &tables, &narrow, &tabsz, &phases);
+  if (rc) return rc;
+  GridRes* gr = nullptr;
+  rc = grid_res(s, false, &gr);
+  if (rc) return rc;
+  rc = enqueue_static(s, tables, narrow, tabsz, T, one_launch_plan(s, narrow, T, phases), gr, false);
+  if (gr->tab_bytes > kTabKeep) {
+    (void)hipStreamSynchronize(s->stream);
+    trim_tables(gr);
+  }
+  return rc;
 }
 
 int bt_run_circuit_dm(bt_state rho, bt_circuit c, bt_run_stats* stats) {
@@ -638,9 +774,10 @@ int bt_run_circuit_dm(bt_state rho, bt_circuit c, bt_run_stats* stats) {
   std::vector<unsigned char> tables;
   std::vector<uint8_t> narrow;
   size_t tabsz = 0;
-  rc = static_plan(rho, c, true, T, &tables, &narrow, &tabsz);
+  bool phases = false;
+  rc = static_plan(rho, c, true, T, &tables, &narrow, &tabsz, &phases);
   if (rc) return rc;
-  return run_static(rho, tables, narrow, tabsz, T, stats);
+  return run_static(rho, tables, narrow, tabsz, phases, T, stats);
 }
 
 int bt_run_batch_persistent(bt_circuit c, int prec, uint64_t seed, int64_t traj0, int64_t ntraj, int* outcomes, int64_t outcap,

@@ -420,7 +420,7 @@ extern "C" int bt_graph_create_dm(bt_state rho, bt_circuit c, bt_graph* out) {
   std::vector<unsigned char> tables;
   std::vector<uint8_t> narrow;
   size_t tabsz = 0;
-  rc = plan_static_passes(rho, dm, T, &tables, &narrow, &tabsz);
+  rc = plan_static_passes(rho, dm, T, &tables, &narrow, &tabsz, nullptr);
   if (rc) return rc;
   auto* g = new bt_graph_s();
   g->s = rho;

@@ -121,7 +121,7 @@ namespace bt {
 // pass writes kGridAccRows rows of reduction partials per workgroup
 constexpr int kGridAccRows = 65;
 int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::vector<unsigned char>* tables,
-                       std::vector<uint8_t>* narrow, size_t* tabsz);
+                       std::vector<uint8_t>* narrow, size_t* tabsz, bool* phases);
 int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part);
 void grid_pass_lds_attr(int prec, int T);
 int dm_tile_bits(bt_state_s* rho);              // tile bits of a density matrix's passes

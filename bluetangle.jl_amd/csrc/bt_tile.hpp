@@ -639,7 +639,7 @@ constexpr size_t kTableMax =
 // Build a pass's table in `out` (kTableMax<R> bytes, 16-byte aligned);
 // *bytes: its size.  *head (nullable): a copy of what the host needs of it.
 struct TableHead {
-  int32_t red_swap, top_thr;
+  int32_t red_swap, top_thr, nph;
 };
 template <typename R>
 inline int build_table(const Plan& plan, const QOp* slots, int nbits, unsigned char* out, size_t* bytes,
@@ -658,7 +658,7 @@ inline int build_table(const Plan& plan, const QOp* slots, int nbits, unsigned c
     n += sizeof(C<R>) * (size_t)g->nmats;
   }
   *bytes = n;
-  if (head) *head = TableHead{g->red_swap, g->top_thr};
+  if (head) *head = TableHead{g->red_swap, g->top_thr, g->nph};
   return BT_OK;
 }
 
@@ -1416,6 +1416,27 @@ __device__ __forceinline__ void pass_fetch(C<R>* raw, const C<R>* __restrict__ s
   }
 }
 
+// Registers of a tile from its fetched values: scaled, and zero where the
+// register is phantom or the thread inactive.  fresh: the state is |0...0>
+// and nothing was fetched (first: this thread's register 0 is its amplitude 0).
+template <typename R>
+__device__ __forceinline__ void pass_take(C<R>* v, const C<R>* raw, R scale, bool active, int nvalid_mask, int fresh,
+                                          bool first) {
+  constexpr int NR = 1 << TileCfg<R>::RB;
+  if (!fresh && active && nvalid_mask == 0) {
+#pragma unroll
+    for (int r = 0; r < NR; r++) v[r] = cmake<C<R>>(raw[r].x * scale, raw[r].y * scale);
+    return;
+  }
+  const int nm = hide(nvalid_mask);
+#pragma unroll
+  for (int r = 0; r < NR; r++) {
+    const bool ok = active && !(r & nm);
+    if (fresh) v[r] = cmake<C<R>>(ok && r == 0 && first ? scale : (R)0, (R)0);
+    else v[r] = cmake<C<R>>(ok ? raw[r].x * scale : (R)0, ok ? raw[r].y * scale : (R)0);
+  }
+}
+
 template <typename R, typename O>
 __device__ __forceinline__ void pass_store(const C<R>* v, C<R>* __restrict__ state, const IoRegs<R, O>& io,
                                            uint64_t base, bool active, int nvalid_mask) {
@@ -1701,6 +1722,50 @@ __device__ __forceinline__ uint64_t deposit(uint64_t t, uint64_t m) {
   return r;
 }
 
+// The operators of phase p on its registers v (layout p), for a tile at base.
+template <typename R, typename G>
+__device__ __forceinline__ void phase_ops(C<R>* v, const G& geo, int p, uint64_t base, int T, const C<R>* staged,
+                                          C<R>* lds, uint32_t tid, uint32_t ltid, bool active, int nvalid_mask) {
+  const size_t pa = offsetof(PassGeom, ph) + (size_t)p * sizeof(RPhase);
+  const int op0 = (int)geo.w(pa + offsetof(RPhase, op0)), op1 = op0 + (int)geo.w(pa + offsetof(RPhase, nops));
+  const int tm = (int)((geo.w(pa + 4) >> 8) & 0xffu);
+  int o = op0;
+  switch (tm) {  // the openings of kPhaseTemplates, straight-line
+    case 1:
+      op_reg<R, 0x0c>(v, geo, o, staged);
+      op_reg<R, 0x03>(v, geo, o + 1, staged);
+      op_reg<R, 0x06>(v, geo, o + 2, staged);
+      o += 3;
+      break;
+    case 2:
+      op_reg<R, 0x0c>(v, geo, o, staged);
+      op_reg<R, 0x03>(v, geo, o + 1, staged);
+      o += 2;
+      break;
+    case 3:
+      op_reg<R, 0x03>(v, geo, o, staged);
+      o += 1;
+      break;
+    default: break;
+  }
+  for (; o < op1; o++) {
+    const uint64_t gctrl = ((uint64_t)geo.w(offsetof(PassGeom, ops) + (size_t)o * sizeof(ROp) + offsetof(ROp, gctrl) + 4) << 32) |
+                           (uint32_t)BT_GOP(o, gctrl);
+    if ((base & gctrl) != gctrl) continue;
+    const int k = BT_GOP(o, k);
+    if (k <= 2) {
+      op_any<R>(BT_GOP(o, mask), v, geo, o, staged);
+    } else {
+      image_write<R>(v, lds, geo, p, tid, active, nvalid_mask);
+      __syncthreads();
+      if (k == 3) op_image<R, 3>(lds, T, geo, o, staged, tid);
+      else op_image<R, 4>(lds, T, geo, o, staged, tid);
+      __syncthreads();
+      image_read<R>(v, lds, geo, p, ltid);
+    }
+  }
+}
+
 // One pass over tiles t = t0, t0 + tstep, ... < tend.  Reductions are added
 // to sums[0..kAcc) (LDS, zeroed by the caller): [0] norm^2, [1..16]
 // histogram, [17..32] packed rho; each wavefront accumulates its tiles in
@@ -1768,21 +1833,7 @@ __device__ __forceinline__ void tile_pass(C<R>* __restrict__ state, const G& geo
       C<R> v[NR];
       const int lay = nph > 0 ? p : kLayIn;
       if (p == 0) {
-        if (!fresh && active && nvalid_mask == 0) {
-#pragma unroll
-          for (int r = 0; r < NR; r++) v[r] = cmake<C<R>>(nx[r].x * scale, nx[r].y * scale);
-        } else {
-          const int nm = hide(nvalid_mask);
-#pragma unroll
-          for (int r = 0; r < NR; r++) {
-            const bool ok = active && !(r & nm);
-            if (fresh) {
-              v[r] = cmake<C<R>>(ok && r == 0 && base == 0 && in.thr == 0 ? scale : (R)0, (R)0);
-            } else {
-              v[r] = cmake<C<R>>(ok ? nx[r].x * scale : (R)0, ok ? nx[r].y * scale : (R)0);
-            }
-          }
-        }
+        pass_take<R>(v, nx, scale, active, nvalid_mask, fresh, base == 0 && in.thr == 0);
         if (!fresh && more) {
           in.again();
           pass_fetch<R, O>(nx, state, in, nbase);
@@ -1793,46 +1844,7 @@ __device__ __forceinline__ void tile_pass(C<R>* __restrict__ state, const G& geo
         }
       }
       if (p > 0 || !in_direct) image_read<R>(v, lds, geo, lay, ltid);
-      if (nph > 0) {
-        const size_t pa = offsetof(PassGeom, ph) + (size_t)p * sizeof(RPhase);
-        const int op0 = (int)geo.w(pa + offsetof(RPhase, op0)), op1 = op0 + (int)geo.w(pa + offsetof(RPhase, nops));
-        const int tm = (int)((geo.w(pa + 4) >> 8) & 0xffu);
-        int o = op0;
-        switch (tm) {  // the openings of kPhaseTemplates, straight-line
-          case 1:
-            op_reg<R, 0x0c>(v, geo, o, staged);
-            op_reg<R, 0x03>(v, geo, o + 1, staged);
-            op_reg<R, 0x06>(v, geo, o + 2, staged);
-            o += 3;
-            break;
-          case 2:
-            op_reg<R, 0x0c>(v, geo, o, staged);
-            op_reg<R, 0x03>(v, geo, o + 1, staged);
-            o += 2;
-            break;
-          case 3:
-            op_reg<R, 0x03>(v, geo, o, staged);
-            o += 1;
-            break;
-          default: break;
-        }
-        for (; o < op1; o++) {
-          const uint64_t gctrl = ((uint64_t)geo.w(offsetof(PassGeom, ops) + (size_t)o * sizeof(ROp) + offsetof(ROp, gctrl) + 4) << 32) |
-                                 (uint32_t)BT_GOP(o, gctrl);
-          if ((base & gctrl) != gctrl) continue;
-          const int k = BT_GOP(o, k);
-          if (k <= 2) {
-            op_any<R>(BT_GOP(o, mask), v, geo, o, staged);
-          } else {
-            image_write<R>(v, lds, geo, lay, tid, active, nvalid_mask);
-            __syncthreads();
-            if (k == 3) op_image<R, 3>(lds, T, geo, o, staged, tid);
-            else op_image<R, 4>(lds, T, geo, o, staged, tid);
-            __syncthreads();
-            image_read<R>(v, lds, geo, lay, ltid);
-          }
-        }
-      }
+      if (nph > 0) phase_ops<R>(v, geo, p, base, T, staged, lds, tid, ltid, active, nvalid_mask);
       if (p + 1 < np || !out_direct || redt == bti::RED_RHO) {
         image_write<R>(v, lds, geo, lay, tid, active, nvalid_mask);
         __syncthreads();
@@ -1907,6 +1919,84 @@ __device__ __forceinline__ void tile_pass(C<R>* __restrict__ state, const G& geo
     sums[threadIdx.x] += t;
   }
   __syncthreads();
+}
+
+// Every pass of a state that is one tile, by one workgroup: the tile is read
+// once, stays in its LDS image from pass to pass (every pass has the same
+// tile bits, so local indices agree) and is stored once.  Passes without
+// reductions or input scale only.  Table q is at tab + q * stride; staged
+// holds two passes' operators: the next pass's are requested before this
+// pass's phases run and written after them.
+template <typename R>
+__device__ __forceinline__ void one_tile_passes(C<R>* __restrict__ state, const unsigned char* tab, uint32_t stride,
+                                                int npass, C<R>* staged, C<R>* lds) {
+  constexpr int NT = TileCfg<R>::NT;
+  constexpr int NR = 1 << TileCfg<R>::RB;
+  constexpr int W = (int)((sizeof(C<R>) * kStageEntries<R> + 16 * NT - 1) / (16 * NT));  // 16-byte words per thread
+  const uint32_t tid = threadIdx.x;
+  auto request = [&](const GeomConst& g, float4* w) {
+    const int n = (int)g.w(offsetof(PassGeom, nstage)) * (int)sizeof(C<R>) / 16;
+#pragma unroll
+    for (int i = 0; i < W; i++)
+      if ((int)tid + i * NT < n) w[i] = ((const float4*)g.staged)[tid + i * NT];
+  };
+  auto put = [&](const GeomConst& g, const float4* w, C<R>* to) {
+    const int n = (int)g.w(offsetof(PassGeom, nstage)) * (int)sizeof(C<R>) / 16;
+#pragma unroll
+    for (int i = 0; i < W; i++)
+      if ((int)tid + i * NT < n) ((float4*)to)[tid + i * NT] = w[i];
+  };
+  float4 w[W];
+  for (int q = 0; q < npass; q++) {
+    const GeomConst geo0(tab + (size_t)q * stride, sizeof(C<R>));
+    const GeomConst geo = geo0.again();
+    const int T = BT_G(T), tb = BT_G(tb), nrb = BT_G(nrb), nph = BT_G(nph);
+    const uint32_t ltid = tid & ((1u << tb) - 1u);
+    const bool active = tid < (1u << tb);
+    const int nvalid_mask = (NR - 1) & ~((1 << nrb) - 1);
+    C<R>* ops = staged + (q & 1) * kStageEntries<R>;
+    const bool last = q + 1 == npass;
+    bool fetched = false;
+    C<R> nx[NR];
+    if (q == 0) {
+      const IoRegs<R, uint32_t> in(geo, offsetof(PassGeom, thr_in), offsetof(PassGeom, reg_in), ltid);
+      pass_fetch<R, uint32_t>(nx, state, in, 0);
+      fetched = true;
+      request(geo, w);
+      put(geo, w, ops);
+      geo.template warm<R>();
+      __syncthreads();
+    }
+    const GeomConst gnext(tab + (size_t)(last ? q : q + 1) * stride, sizeof(C<R>));
+    if (!last) request(gnext, w);
+    for (int p = 0; p < nph; p++) {
+      const GeomConst gp = geo0.again();
+      C<R> v[NR];
+      if (p == 0 && fetched) {
+        pass_take<R>(v, nx, (R)1, active, nvalid_mask, 0, false);
+        if (BT_G(in_direct) == 0) {
+          image_write<R>(v, lds, gp, kLayIn, tid, active, nvalid_mask);
+          __syncthreads();
+          image_read<R>(v, lds, gp, p, ltid);
+        }
+      } else {
+        image_read<R>(v, lds, gp, p, ltid);
+      }
+      phase_ops<R>(v, gp, p, 0, T, ops, lds, tid, ltid, active, nvalid_mask);
+      image_write<R>(v, lds, gp, p, tid, active, nvalid_mask);
+      if (p + 1 < nph || last) __syncthreads();
+    }
+    if (last) {
+      C<R> v[NR];
+      image_read<R>(v, lds, geo, kLayOut, ltid);
+      const IoRegs<R, uint32_t> out(geo, offsetof(PassGeom, thr_out), offsetof(PassGeom, reg_out), ltid);
+      pass_store<R, uint32_t>(v, state, out, 0, active, nvalid_mask);
+    } else {
+      put(gnext, w, staged + ((q + 1) & 1) * kStageEntries<R>);
+      gnext.template warm<R>();
+      __syncthreads();
+    }
+  }
 }
 #endif
 
