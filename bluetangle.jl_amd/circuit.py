@@ -28,6 +28,7 @@ class IR:
         self.ops: List[L.IrOp] = []
         self.pool: List[np.ndarray] = []
         self.pool_len = 0
+        self._kraus = {}  # id of a Kraus list -> (the list, its offset): a noise model repeats a few of them
 
     def add_matrix(self, m) -> int:
         m = np.asarray(m, dtype=np.complex128)
@@ -35,6 +36,15 @@ class IR:
         self.pool.append(_colmajor(m))
         self.pool_len += m.shape[0] * m.shape[1]
         return off
+
+    def add_kraus(self, kraus) -> int:
+        seen = self._kraus.get(id(kraus))
+        if seen is None:
+            off = self.add_matrix(kraus[0])
+            for K in kraus[1:]:
+                self.add_matrix(K)
+            seen = self._kraus[id(kraus)] = (kraus, off)  # kept, so that the id stays its own
+        return seen[1]
 
     def op(self, kind, bits, k=None, prob_bits=None, ctrl=0, mat=0, nkraus=0, basis=0, record=0):
         o = L.IrOp()
@@ -80,10 +90,7 @@ def _gate_record(ir, N, q, mat, qubit, target, control):
 def _channel_record(ir, N, kraus, qubit, target):
     q = int(round(math.log2(kraus[0].shape[0])))
     a, p = channel_bits(N, q, qubit, target)
-    off = ir.add_matrix(kraus[0])
-    for K in kraus[1:]:
-        ir.add_matrix(K)
-    return ir.op(L.BT_OP_CHANNEL, a, prob_bits=p, mat=off, nkraus=len(kraus))
+    return ir.op(L.BT_OP_CHANNEL, a, prob_bits=p, mat=ir.add_kraus(kraus), nkraus=len(kraus))
 
 
 def _noise_records(ir, N, op, noise):

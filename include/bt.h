@@ -87,6 +87,18 @@ uint64_t bt_state_bytes(int nqubits, int kind, int prec);
  * SV: psi <- M psi on bits (k <= 5) where all bits of ctrl_mask are 1.
  * DM: rho <- E rho E' (hilbert.jl:655-656), k <= 3. */
 int bt_apply_matrix(bt_state s, int k, const double* mat, const int* bits, uint64_t ctrl_mask);
+/* A list of operations (the circuit IR without BT_OP_IF, matrices in pool) on
+ * a state vector as it is, in order, as fused passes: apply(ops::Vector, psi)
+ * (hilbert.jl:517-557), where every gate by itself is a read and a write of
+ * the state and every channel or measurement a reduction and a wait besides.
+ * Uniforms are consumed as the per-op entries consume theirs (one per channel
+ * and measurement, two for BT_BASIS_R); probabilities are those of the state,
+ * normalised or not.  Gates alone are enqueued on the state's stream like
+ * bt_apply_matrix.  BT_ERR_STATE, with the state untouched, if sampling is
+ * asked of a state without a finite positive norm. */
+struct bt_ir_op_s;
+int bt_apply_ops(bt_state s, const struct bt_ir_op_s* ops, int nops, const double* pool, int64_t npool,
+                 const double* uniforms, int64_t nuni, int* outcomes, int64_t outcap, int64_t* nout);
 /* OpF(name, mat) (struct.jl:716-720): psi <- M psi with a full 2^N x 2^N
  * matrix, column-major complex128; FP64 accumulation.  SV states only (the
  * reference's matrix OpF has no density-matrix method). */
@@ -166,7 +178,7 @@ int bt_gather(bt_state s, const uint64_t* idx, uint64_t n, double* out);
 #define BT_OP_RESET 3
 #define BT_OP_IF 4
 
-typedef struct {
+typedef struct bt_ir_op_s {
   int32_t kind;         /* BT_OP_* */
   int32_t k;            /* target bits: gates 1..5, channels 1..3, measure/reset/if 1 */
   int32_t bits[5];      /* target bit positions, bits[0] = MSB of the local index */
