@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_batch(Bat
 // O: type of the per-thread byte offset (narrow_io)
 template <typename R, typename O>
 __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_grid_pass(C<R>* state, const unsigned char* tab, uint64_t ntiles,
-                                                              double* part) {
+                                                              double* part, unsigned* count, double* out, int nacc) {
   constexpr int NT = TileCfg<R>::NT;
   extern __shared__ __align__(16) unsigned char smem[];
   C<R>* tile = (C<R>*)smem;
@@ -152,7 +152,7 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_grid_pass
   if (threadIdx.x < kAcc) sums[threadIdx.x] = 0.0;
   tile_pass<R, O>(state, GeomConst(tab, sizeof(C<R>)), staged, tile, blockIdx.x, gridDim.x, ntiles,
                   red, sums);
-  if (part && threadIdx.x < kAcc) part[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = sums[threadIdx.x];
+  if (out) item_finish<NT>(sums, red, part, blockIdx.x, gridDim.x, count, out, nacc);
 }
 
 // All passes of a state that is one tile in one launch (static plans: no
@@ -164,12 +164,6 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, 1) k_one_tile(C<R>* state, con
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ __align__(16) C<R> staged[2 * kStageEntries<R>];
   one_tile_passes<R>(state, tab, stride, npass, staged, (C<R>*)smem);
-}
-
-// out[j] = fixed-order sum of the grid's partials of accumulator j
-__global__ void __launch_bounds__(256) k_finalize_acc(const double* part, int nblocks, double* out) {
-  const double t = sum_blocks(part + (uint64_t)blockIdx.x * nblocks, (uint32_t)nblocks);
-  if (threadIdx.x == 0) out[blockIdx.x] = t;
 }
 
 }  // namespace bt
@@ -235,9 +229,6 @@ int tile_bits_for(int prec, int nbits) {
   return std::min(T, nbits);
 }
 
-
-static_assert(kGridAccRows == kAcc, "grid pass partial rows");
-
 // Workgroups of a grid pass over ntiles tiles: eight per CU at most.
 static unsigned grid_pass_blocks(uint64_t ntiles) {
   const int cus = ctx().cus > 0 ? ctx().cus : 256;
@@ -251,13 +242,13 @@ constexpr size_t kTabKeep = 16ull << 20;
 // until the state is destroyed (a state is used by one host thread at a
 // time): what a static plan needs, and with the first circuit that decides
 // on reductions pinned and device rings of pass tables, reduction partials
-// for the widest grid, the finished sums and their pinned copy, events.
+// for the widest grid, the pinned finished sums, events.
 struct GridRes {
   void* h_ring = nullptr;
   void* d_ring = nullptr;
   double* d_part = nullptr;
-  double* d_acc = nullptr;
-  double* h_acc = nullptr;
+  unsigned* d_count = nullptr;  // behind the partials
+  double* h_acc = nullptr;      // the finished sums (pinned, written by the pass)
   // a static plan's tables: pinned and device, reused once the copy / the
   // launches that read them are done; at most kTabKeep bytes are kept
   void* h_tab = nullptr;
@@ -281,7 +272,6 @@ void free_grid_res(GridRes* g) {
   if (g->h_acc) (void)hipHostFree(g->h_acc);
   if (g->d_ring) (void)hipFree(g->d_ring);
   if (g->d_part) (void)hipFree(g->d_part);
-  if (g->d_acc) (void)hipFree(g->d_acc);
   delete g;
 }
 
@@ -315,8 +305,9 @@ static int grid_res(bt_state_s* s, bool ring, GridRes** out) {
     const int cus = ctx().cus > 0 ? ctx().cus : 256;
     bool ok = hipHostMalloc(&g->h_ring, tabsz * kRing) == hipSuccess &&
               hipMalloc(&g->d_ring, tabsz * kRing) == hipSuccess &&
-              hipMalloc((void**)&g->d_part, sizeof(double) * kAcc * (size_t)cus * 8) == hipSuccess &&
-              hipMalloc((void**)&g->d_acc, sizeof(double) * kAcc) == hipSuccess;
+              hipMalloc((void**)&g->d_part, sizeof(double) * kAcc * (size_t)cus * 8 + 16) == hipSuccess;
+    g->d_count = (unsigned*)(g->d_part + (size_t)kAcc * cus * 8);
+    ok = ok && hipMemset(g->d_count, 0, 16) == hipSuccess;
     for (int i = 0; i < kRing && ok; i++) ok = hipEventCreateWithFlags(&g->ev[i], hipEventDisableTiming) == hipSuccess;
     ok = ok && hipHostMalloc((void**)&g->h_acc, sizeof(double) * kAcc) == hipSuccess;
     if (!ok) {
@@ -353,15 +344,11 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
   ip->r = r0;
   ip->tol_exact = s->prec == BT_C64 ? 1e-6 : 1e-12;
   const size_t tabsz = table_max(s->prec);
-  const uint64_t ntiles = 1ull << (nbits - std::min(T, nbits));
-  const unsigned blocks = grid_pass_blocks(ntiles);
   GridRes* gr = nullptr;
   int rc = grid_res(s, true, &gr);
   if (rc) return rc;
   void* const h_ring = gr->h_ring;
   void* const d_ring = gr->d_ring;
-  double* const d_part = gr->d_part;
-  double* const d_acc = gr->d_acc;
   double* const h_acc = gr->h_acc;
   hipEvent_t* const ev = gr->ev;
   hipEvent_t const e0 = gr->e0, e1 = gr->e1;
@@ -399,17 +386,16 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
       break;
     }
     (void)hipEventRecord(ev[slot], s->stream);
-    rc = launch_grid_pass(s, dslot, pass_narrow(s->prec, head), T, d_part);
-    if (rc) break;
     // the host waits for a pass's sums only when a decision needs them or
     // the norm is folded into the next pass (fold = 0, a density matrix:
     // passes follow one another without a round trip)
-    if (plan.red != bti::RED_NONE || (plan.aligned && fold)) {
-      hipLaunchKernelGGL(k_finalize_acc, dim3(kAcc), dim3(256), 0, s->stream, (const double*)d_part, (int)blocks,
-                         d_acc);
-      if (hipMemcpyAsync(h_acc, d_acc, sizeof(double) * kAcc, hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-          hipStreamSynchronize(s->stream) != hipSuccess) {
-        rc = fail(BT_ERR_HIP, "run_grid: reduction copy");
+    const bool want = plan.red != bti::RED_NONE || (plan.aligned && fold);
+    rc = launch_grid_pass(s, dslot, pass_narrow(s->prec, head), T, gr->d_part, gr->d_count, want ? h_acc : nullptr,
+                          acc_count(plan));
+    if (rc) break;
+    if (want) {
+      if (hipStreamSynchronize(s->stream) != hipSuccess) {
+        rc = fail(BT_ERR_HIP, "run_grid: pass");
         break;
       }
       to_result(plan, red_swap, h_acc, &res);
@@ -483,8 +469,10 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
 }
 
 // Enqueue one grid pass of state s (tile bits T) with its table at dtab;
-// d_part: kAcc x grid doubles of reduction partials (null: none are wanted).
-int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part) {
+// out (pinned host memory, null: no sums are wanted) gets the pass's first
+// nacc sums; d_part: kAcc x grid doubles of partials, d_count: a zero.
+int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part, unsigned* d_count,
+                     double* out, int nacc) {
   const int nbits = s->nbits;
   const uint64_t ntiles = 1ull << (nbits - std::min(T, nbits));
   const unsigned blocks = grid_pass_blocks(ntiles);
@@ -492,17 +480,17 @@ int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double
   if (s->prec == BT_C64) {
     if (narrow)
       hipLaunchKernelGGL((k_grid_pass<float, uint32_t>), dim3(blocks), dim3(TileCfg<float>::NT), lds, s->stream,
-                         (C<float>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
+                         (C<float>*)s->d, (const unsigned char*)dtab, ntiles, d_part, d_count, out, nacc);
     else
       hipLaunchKernelGGL((k_grid_pass<float, uint64_t>), dim3(blocks), dim3(TileCfg<float>::NT), lds, s->stream,
-                         (C<float>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
+                         (C<float>*)s->d, (const unsigned char*)dtab, ntiles, d_part, d_count, out, nacc);
   } else {
     if (narrow)
       hipLaunchKernelGGL((k_grid_pass<double, uint32_t>), dim3(blocks), dim3(TileCfg<double>::NT), lds, s->stream,
-                         (C<double>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
+                         (C<double>*)s->d, (const unsigned char*)dtab, ntiles, d_part, d_count, out, nacc);
     else
       hipLaunchKernelGGL((k_grid_pass<double, uint64_t>), dim3(blocks), dim3(TileCfg<double>::NT), lds, s->stream,
-                         (C<double>*)s->d, (const unsigned char*)dtab, ntiles, d_part);
+                         (C<double>*)s->d, (const unsigned char*)dtab, ntiles, d_part, d_count, out, nacc);
   }
   BT_HIP(hipGetLastError());
   return BT_OK;
@@ -588,7 +576,7 @@ static int enqueue_static(bt_state_s* s, const std::vector<unsigned char>& table
     grid_pass_lds_attr(s->prec, Tn);
     if (timed) (void)hipEventRecord(gr->e0, s->stream);
     for (size_t i = 0; rc == BT_OK && i < narrow.size(); i++)
-      rc = launch_grid_pass(s, (const unsigned char*)gr->d_tab + i * tabsz, narrow[i] != 0, T, nullptr);
+      rc = launch_grid_pass(s, (const unsigned char*)gr->d_tab + i * tabsz, narrow[i] != 0, T);
   }
   if (timed) (void)hipEventRecord(gr->e1, s->stream);
   (void)hipEventRecord(gr->tab_done, s->stream);

@@ -317,7 +317,6 @@ struct bt_graph_s {
   hipGraphExec_t exec = nullptr;
   float* d_al = nullptr;
   void* d_tab = nullptr;    // density-matrix graphs: the passes' tables
-  double* d_part = nullptr; // and their (unused) reduction partials
   std::vector<btf::Block> blocks;
   int64_t nblocks = 0;
 };
@@ -396,7 +395,6 @@ extern "C" int bt_graph_destroy(bt_graph g) {
   if (g->graph) (void)hipGraphDestroy(g->graph);
   if (g->d_al) (void)hipFree(g->d_al);
   if (g->d_tab) (void)hipFree(g->d_tab);
-  if (g->d_part) (void)hipFree(g->d_part);
   delete g;
   return BT_OK;
 }
@@ -429,13 +427,10 @@ extern "C" int bt_graph_create_dm(bt_state rho, bt_circuit c, bt_graph* out) {
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
     if (g->d_tab) (void)hipFree(g->d_tab);
-    if (g->d_part) (void)hipFree(g->d_part);
     delete g;
     return r;
   };
-  const int cus = ctx().cus > 0 ? ctx().cus : 256;
-  if (hipMalloc(&g->d_tab, std::max<size_t>(tables.size(), 16)) != hipSuccess ||
-      hipMalloc((void**)&g->d_part, sizeof(double) * kGridAccRows * (size_t)cus * 8) != hipSuccess)
+  if (hipMalloc(&g->d_tab, std::max<size_t>(tables.size(), 16)) != hipSuccess)
     return cleanup(fail(BT_ERR_NOMEM, "bt_graph_create_dm: tables"));
   if (!tables.empty() && hipMemcpy(g->d_tab, tables.data(), tables.size(), hipMemcpyHostToDevice) != hipSuccess)
     return cleanup(fail(BT_ERR_HIP, "bt_graph_create_dm: table upload"));
@@ -445,7 +440,7 @@ extern "C" int bt_graph_create_dm(bt_state rho, bt_circuit c, bt_graph* out) {
     return cleanup(fail(BT_ERR_HIP, "bt_graph_create_dm: begin capture"));
   int crc = BT_OK;
   for (size_t i = 0; crc == BT_OK && i < narrow.size(); i++)
-    crc = launch_grid_pass(rho, (const unsigned char*)g->d_tab + i * tabsz, narrow[i] != 0, T, g->d_part);
+    crc = launch_grid_pass(rho, (const unsigned char*)g->d_tab + i * tabsz, narrow[i] != 0, T);
   const hipError_t ec = hipStreamEndCapture(rho->stream, &g->graph);
   if (crc) return cleanup(crc);
   if (ec != hipSuccess || !g->graph) return cleanup(fail(BT_ERR_HIP, "bt_graph_create_dm: end capture"));

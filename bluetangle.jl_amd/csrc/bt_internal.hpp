@@ -117,12 +117,11 @@ struct CircuitHost;
 }
 
 namespace bt {
-// density-matrix executor pieces shared with the graph capture; a grid
-// pass writes kGridAccRows rows of reduction partials per workgroup
-constexpr int kGridAccRows = 65;
+// density-matrix executor pieces shared with the graph capture
 int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::vector<unsigned char>* tables,
                        std::vector<uint8_t>* narrow, size_t* tabsz, bool* phases);
-int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part);
+int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part = nullptr,
+                     unsigned* d_count = nullptr, double* out = nullptr, int nacc = 0);
 void grid_pass_lds_attr(int prec, int T);
 int dm_tile_bits(bt_state_s* rho);              // tile bits of a density matrix's passes
 int dm_tile_bits_for(int prec, int nbits);      // the same for vec(rho) of nbits index bits

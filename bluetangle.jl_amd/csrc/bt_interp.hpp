@@ -373,8 +373,7 @@ struct Interp {
   }
 
   BT_HD uint64_t fill_low(uint64_t tile) {
-    int cnt = 0;
-    for (int b = 0; b < P.nbits; b++) cnt += (tile >> b) & 1;
+    int cnt = popc(tile);
     for (int b = 0; b < P.nbits && cnt < T; b++)
       if (!((tile >> b) & 1)) {
         tile |= 1ull << b;
@@ -383,14 +382,7 @@ struct Interp {
     return tile;
   }
 
-  BT_HD static int popc(uint64_t x) {
-    int c = 0;
-    while (x) {
-      x &= x - 1;
-      c++;
-    }
-    return c;
-  }
+  BT_HD static int popc(uint64_t x) { return __builtin_popcountll(x); }
 
   // Greedy over the queue, seeded with the first operator: the target bits
   // of the operators that fit in `cap` bits, in queue order, skipping those

@@ -35,7 +35,6 @@ constexpr int kMatEntries = bti::Interp::kPassMatEntries;
 // the packed reduced rho (diagonal, then Re/Im of rho[a, b] for a < b: 16
 // doubles over 2 bits, 64 over 3)
 constexpr int kAcc = 65;
-constexpr int kAccSmall = 17;  // enough unless a pass reduces rho over 3 bits
 constexpr int kRB = 5;     // register bits (most)
 constexpr int kTB = 8;     // thread bits (most)
 constexpr int kMaxPh = 28;
@@ -144,14 +143,7 @@ struct PassGeom {
 // ---------------------------------------------------------------------------
 // host/device: plan + queue slots -> register-tile geometry and matrices
 // ---------------------------------------------------------------------------
-__host__ __device__ inline int popc32(uint32_t x) {
-  int c = 0;
-  while (x) {
-    x &= x - 1;
-    c++;
-  }
-  return c;
-}
+__host__ __device__ inline int popc32(uint32_t x) { return __builtin_popcount(x); }
 
 // Layout with register positions 0..nrb-1 holding the given local bits
 // (ascending) and the rest phantom.
@@ -1181,19 +1173,63 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// Fixed-order sum of per-workgroup partials laid out accumulator-major
-// (part[j * stride + block]): one workgroup of 256 threads per (item j).
-__device__ __forceinline__ double sum_blocks(const double* __restrict__ p, uint32_t n) {
-  __shared__ double sh[256];
-  double t = 0.0;
-  for (uint32_t b = threadIdx.x; b < n; b += 256) t += p[b];
-  sh[threadIdx.x] = t;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
+// Finish the reductions of one pass over one state in the pass's own launch:
+// every workgroup stores its nacc sums (LDS) as partials, accumulator-major
+// (part[j * nb + block]); the last of the state's nb workgroups adds them in
+// a fixed order that depends on nb and nacc alone (P threads per
+// accumulator, each over every P-th workgroup, then a fixed tree) and writes
+// the totals to out (pinned host memory): no second launch and no copy.
+// The partials cross the XCDs' L2 caches: agent-scope stores, complete before
+// the state's count is raised, and agent-scope loads after it.  count is 0
+// between launches.  red: NT/64 doubles of LDS.  One noisy trajectory of 22
+// qubits in 30 passes: 1.29 -> 1.25 ms against a totals launch and a copy.
+template <int NT>
+__device__ __forceinline__ void item_finish(const double* sums, double* red, double* part, uint32_t block,
+                                            uint32_t nb, unsigned* count, double* out, int nacc) {
+  __shared__ int last;
+  const int tid = threadIdx.x;
+  if (nb == 1) {
+    if (tid < nacc) out[tid] = sums[tid];
+    return;
   }
-  return sh[0];
+  if (tid < nacc)
+    __hip_atomic_store(part + (uint64_t)tid * nb + block, sums[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials have reached the point of coherence
+  __syncthreads();
+  if (tid == 0) last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+  __syncthreads();
+  if (!last) return;
+  if (tid == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // a power of two of threads per accumulator, 16 at least: a norm alone gets all
+  const int P = nacc <= 1 ? NT : nacc <= 2 ? NT / 2 : nacc <= 5 ? NT / 8 : NT / 16;
+  static_assert(NT == 256, "thread split of the totals");
+  const int W = P < 64 ? P : 64;
+  const int q = tid & (P - 1);
+  for (int j0 = 0; j0 < nacc; j0 += NT / P) {
+    const int j = j0 + tid / P;
+    double t = 0.0;
+    if (j < nacc) {
+      const double* p = part + (uint64_t)j * nb;
+      uint32_t b = (uint32_t)q;
+      for (; b + 7u * P < nb; b += 8u * P) {  // eight loads in flight
+        double x[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = __hip_atomic_load(p + b + i * P, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < 8; i++) t += x[i];
+      }
+      for (; b < nb; b += P) t += __hip_atomic_load(p + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (int o = W / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+    if (P > 64) {
+      __syncthreads();
+      if ((tid & 63) == 0) red[tid >> 6] = t;
+      __syncthreads();
+      t = 0.0;
+      for (int w = 0; w < P / 64; w++) t += red[((tid - q) >> 6) + w];
+    }
+    if (q == 0 && j < nacc) out[j] = t;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2017,6 +2053,11 @@ __host__ __device__ inline void unpack_rho(int k, const double* packed, double* 
       rho[2 * (B + A * D) + 1] = -packed[p + 1];
       p += 2;
     }
+}
+
+// How many of a pass's sums its result takes (to_result).
+__host__ __device__ inline int acc_count(const Plan& plan) {
+  return plan.red == bti::RED_HIST ? 1 + (1 << plan.red_k) : plan.red == bti::RED_RHO ? 1 + (1 << 2 * plan.red_k) : 1;
 }
 
 __host__ __device__ inline void to_result(const Plan& plan, int red_swap, const double* sum, PassResult* res) {
