@@ -434,6 +434,13 @@ inline int lower_dm(const CircuitHost& c, CircuitHost* out, std::string* msg) {
   return BT_OK;
 }
 
+// Whether a trajectory reads its state to decide a branch.
+inline bool decides(const CircuitHost& c) {
+  for (size_t i = 0; i < c.ops.size(); i++)
+    if (c.ops[i].kind != BT_OP_GATE && !(c.ops[i].kind == BT_OP_CHANNEL && c.chan[i].mode == bti::CH_PAULI)) return true;
+  return false;
+}
+
 }  // namespace btc
 
 // A validated circuit and its device copies (uploaded on first use).
