@@ -339,6 +339,7 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
   bti::Program prog{ch.ops.data(), ch.ntop, ch.pool.data(), ch.chan.data(), ch.chanw.data(), nbits};
   const int T = prec_tile_T;
   ip->init(prog, slots.data(), T, coalesce_bits(s->prec, btc::decides(ch)));
+  ip->stream = 1;
   ip->seed = seed;
   ip->traj = traj;
   if (uni) {
@@ -442,6 +443,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
   std::unique_ptr<bti::Interp> ip(new bti::Interp());
   bti::Program prog{ch.ops.data(), ch.ntop, ch.pool.data(), ch.chan.data(), ch.chanw.data(), nbits};
   ip->init(prog, slots.data(), T, coalesce_bits(s->prec, false));
+  ip->stream = 1;
   ip->fold = 0;
   tables->clear();
   narrow->clear();

@@ -146,13 +146,14 @@ struct Interp {
   int32_t nq;
   uint64_t used_slots;
   int32_t fold;        // 0: no renormalisation bookkeeping (density matrices)
+  int32_t stream;      // 1: a full queue makes room with one pass (see step)
   // control
   int32_t pc, end, sp, ret_pc, ret_end;
   int64_t draw;
   double norm2;        // measured norm^2 of the last aligned state
   double c2, r, pend_scale;
   int32_t c2_known, r_known;
-  int32_t flushing, after, awaiting, done_program, final_stage;
+  int32_t flushing, room, after, awaiting, done_program, final_stage;
   int32_t red_req, red_k, red_bits[kGroupMax], red_done;
   PassResult last;
   // pending decision
@@ -174,6 +175,7 @@ struct Interp {
     nq = 0;
     used_slots = 0;
     fold = 1;
+    stream = 0;
     T = tile_bits < prog.nbits ? tile_bits : prog.nbits;
     cmin = coalesce_bits;
     if (cmin > T) cmin = T;
@@ -186,7 +188,7 @@ struct Interp {
     r = 1.0;
     pend_scale = 1.0;
     c2_known = r_known = 1;
-    flushing = after = awaiting = done_program = final_stage = 0;
+    flushing = room = after = awaiting = done_program = final_stage = 0;
     red_req = RED_NONE;
     red_done = 1;
     nout = 0;
@@ -748,13 +750,13 @@ struct Interp {
     for (int guard = 0; guard < (1 << 30); guard++) {
       if (err) return 0;
       if (flushing) {
-        if (nq > 0 || !red_done) {
+        if ((nq > 0 || !red_done) && !(room && --room == 0)) {
           make_plan(plan);
           if (err) return 0;
           awaiting = 1;
           return 1;
         }
-        flushing = 0;
+        flushing = room = 0;
         int a = after;
         after = 0;
         if (a == 1) decide_group();
@@ -802,6 +804,13 @@ struct Interp {
       }
       if (nq >= kQMax - 2) {
         start_flush(RED_NONE, 0, nullptr);
+        // While the factors c and r are known nothing has to be measured, and
+        // the queue need not be emptied: one pass makes room, and what it
+        // leaves is packed with the operators that follow.  Emptying it ends
+        // every 40 operators with passes of a few.  Passes, emptying / this
+        // way: 27 qubits, 8 brickwork layers 11 / 9; 24 qubits, 16 layers
+        // 16 / 10; 20 qubits, 24 layers of distant pairs 32 / 21.
+        if (stream && c2_known && r_known) room = 2;
         continue;
       }
       const bt_ir_op& op = P.ops[pc];

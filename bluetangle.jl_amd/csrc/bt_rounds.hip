@@ -279,6 +279,7 @@ class RoundEngine {
     // kMaxQK bits of vec(rho), so a smaller tile setting is raised to hold it
     const int T = j->fold ? tile_T(j->nbits) : dm_tile_bits_for(prec_, j->nbits);
     j->ip->init(prog, j->slots.get(), T, coalesce_bits(prec_, btc::decides(*j->circ)));
+    j->ip->stream = 1;
     j->ip->seed = j->seed;
     j->ip->traj = j->traj;
     j->ip->fold = j->fold;
