@@ -112,7 +112,9 @@ constexpr PhaseTemplate kPhaseTemplates[] = {
 };
 constexpr int kNumPhaseTemplates = (int)(sizeof(kPhaseTemplates) / sizeof(kPhaseTemplates[0]));
 
-constexpr int kLayIn = kMaxPh, kLayOut = kMaxPh + 1;  // slot tables of the load / store layouts
+// slot tables of the load / store layouts, and of the store layout in an
+// image without relabelling
+constexpr int kLayIn = kMaxPh, kLayOut = kMaxPh + 1, kLayEnd = kMaxPh + 2;
 
 struct PassGeom {
   int32_t T, nrb, tb, ncomp, write, need_norm, red, red_k, red_swap, nph, nops, nmats, nstage;
@@ -130,11 +132,11 @@ struct PassGeom {
   uint8_t thr_in[12], thr_out[12], reg_in[8], reg_out[8];
   int32_t in_direct, out_direct;  // first phase reads / last phase stores in its own layout
   int32_t top_thr;                // highest global bit on a thread in either layout
-  int32_t pad2;
+  int32_t relabel;                // the image ends the pass relabelled (kLayOut reads it)
   uint64_t outside;               // global bits outside the tile
   uint32_t red_loff[8];      // RED_RHO: local offset of each packed index
   int32_t red_ls[4];         // RED_RHO: the local bits, ascending; RED_HIST: local bit of bin bit j (-1: outside)
-  LSlots lay[kMaxPh + 2];    // slot tables: phases, then kLayIn, kLayOut
+  LSlots lay[kMaxPh + 3];    // slot tables: phases, then kLayIn, kLayOut, kLayEnd
   double scale;
   RPhase ph[kMaxPh];
   ROp ops[bti::kPMax];  // last: a packed table holds only the used ones
@@ -160,16 +162,17 @@ __host__ __device__ __forceinline__ uint32_t swz(uint32_t l) {
   return l ^ (((l >> W) ^ (l >> (2 * W))) & ((1u << W) - 1u));
 }
 
+// at: where the image holds the unit index of each local bit (see LinMap).
 template <typename R>
-__host__ __device__ inline void make_slots(const int8_t* rb, int T, LSlots* s) {
+__host__ __device__ inline void make_slots(const int8_t* rb, int T, const uint32_t* at, LSlots* s) {
   uint32_t regm = 0;
   for (int j = 0; j < kRB; j++) {
     if (rb[j] >= 0) regm |= 1u << rb[j];
-    s->rs[j] = rb[j] >= 0 ? (uint16_t)swz<R>(1u << rb[j]) : (uint16_t)0;
+    s->rs[j] = rb[j] >= 0 ? (uint16_t)swz<R>(at[rb[j]]) : (uint16_t)0;
   }
   int i = 0;
   for (int b = 0; b < T && i < kTB; b++)
-    if (!((regm >> b) & 1)) s->ts[i++] = (uint16_t)swz<R>(1u << b);
+    if (!((regm >> b) & 1)) s->ts[i++] = (uint16_t)swz<R>(at[b]);
   for (; i < kTB; i++) s->ts[i] = 0;
   s->pad[0] = s->pad[1] = s->pad[2] = 0;
 }
@@ -209,6 +212,42 @@ __host__ __device__ inline void stage_ops(const PassGeom& g, const C<R>* mats, C
       out[op.stage + e] = x;
     }
   }
+}
+
+// CNOT, SWAP and their products on two bits map basis states by a linear map
+// of their index bits, |j> -> |A j> over GF(2).  The tile image is addressed
+// by XORs of one slot per index bit, so such an operator between two phases
+// is a change of the slots the later phase uses and costs nothing: the image
+// holds the amplitude of local index i at M i, and the operator turns M into
+// M A^-1.  The two halves of every CNOT on a density matrix were 4 of the 7
+// operators of its phases, and the CNOTs that no rotation absorbs end every
+// circuit: exact evolution of 8 qubits, 16 layers 478 -> 355 us, of 12
+// qubits, 4 layers 1110 -> 889 us; a 30-qubit circuit of 2 layers 19.3 ->
+// 16.7 ms.
+// inv2: A^-1 of a two-bit operator given by its expanded column -> row map
+// (operand order, operand 0 = bit 1); false if it is no such map.
+__host__ __device__ inline bool linear_inverse(const QOp& q, int nc, int* inv2) {
+  if (q.k + nc != 2) return false;
+  const int D = 1 << q.k;
+  int seen = 0;
+  for (int c = 0; c < 4; c++) {
+    const int cc = c >> q.k, tc = c & (D - 1);
+    int row = -1;
+    if (cc != (1 << nc) - 1) {
+      row = c;
+    } else {
+      for (int r = 0; r < D; r++) {
+        const double re = q.m[2 * (r + tc * D)], im = q.m[2 * (r + tc * D) + 1];
+        if (re == 0.0 && im == 0.0) continue;
+        if (re != 1.0 || im != 0.0 || row >= 0) return false;
+        row = (cc << q.k) | r;
+      }
+    }
+    if (row < 0) return false;
+    seen |= 1 << row;
+    inv2[row] = c;
+  }
+  return seen == 15 && inv2[0] == 0;  // a permutation that keeps 0 is linear on two bits
 }
 
 template <typename R>
@@ -286,49 +325,105 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
       if (ta & to) pred[o] |= 1u << a;
     }
   }
+  // Operators that only relabel the tile image (host planning; a pass whose
+  // reduction or wide operator reads the image by index keeps them all).
+  uint32_t lin = 0;
+  int inv2[bti::kPMax][4];
+#if !defined(__HIP_DEVICE_COMPILE__)
+  if (plan.red == bti::RED_NONE) {
+    bool wide = false;
+    for (int o = 0; o < nops; o++) {
+      const QOp& q = slots[plan.qidx[o]];
+      wide = wide || lk[o] >= 3;
+      const bool outside = (q.ctrl & ~tmask) != 0;
+      if (lk[o] == 2 && !outside && linear_inverse(q, lk[o] - q.k, inv2[o])) lin |= 1u << o;
+    }
+    if (wide) lin = 0;
+  }
+#endif
   int nph = 0;
   uint32_t cur = 0;  // register-bit mask of the last phase
   int ph_of[bti::kPMax];
   int exec[bti::kPMax];  // execution order
   int ne = 0;
   uint32_t ph_mask[kMaxPh];
-  uint32_t done = 0;
+  uint32_t lin_at[kMaxPh + 1];  // linear operators in front of each phase / behind the last
   const uint32_t all = nops >= 32 ? 0xffffffffu : (1u << nops) - 1u;
-  while (done != all) {
-    uint32_t best = 0, best_m = 0;
-    int best_n = -1;
-    for (int sd = 0; sd < nops; sd++) {
-      if (((done >> sd) & 1) || (pred[sd] & ~done)) continue;
-      uint32_t sel = 1u << sd, m = opm[sd];
-      int n = 1;
-      for (bool grew = true; grew;) {
-        grew = false;
-        for (int o = 0; o < nops; o++) {
-          if (((done | sel) >> o) & 1) continue;
-          if (pred[o] & ~(done | sel)) continue;
-          if (popc32(m | opm[o]) > nrb) continue;
-          sel |= 1u << o;
-          m |= opm[o];
-          n++;
-          grew = true;
+  auto split = [&](uint32_t lin) -> bool {
+    uint32_t done = 0;
+    nph = ne = 0;
+    cur = 0;
+    for (int p = 0; p <= kMaxPh; p++) lin_at[p] = 0;
+    for (;;) {
+      for (int o = 0; o < nops; o++)
+        if (((lin & ~done) >> o) & 1 && !(pred[o] & ~done)) {
+          done |= 1u << o;
+          lin_at[nph] |= 1u << o;
+        }
+      if (done == all) return true;
+      uint32_t best = 0, best_m = 0;
+      int best_n = -1;
+      for (int sd = 0; sd < nops; sd++) {
+        if (((done | lin) >> sd) & 1 || (pred[sd] & ~done)) continue;
+        uint32_t sel = 1u << sd, m = opm[sd];
+        int n = 1;
+        for (bool grew = true; grew;) {
+          grew = false;
+          for (int o = 0; o < nops; o++) {
+            if (((done | lin | sel) >> o) & 1) continue;
+            if (pred[o] & ~(done | sel)) continue;
+            if (popc32(m | opm[o]) > nrb) continue;
+            sel |= 1u << o;
+            m |= opm[o];
+            n++;
+            grew = true;
+          }
+        }
+        if (n > best_n) {
+          best_n = n;
+          best = sel;
+          best_m = m;
         }
       }
-      if (n > best_n) {
-        best_n = n;
-        best = sel;
-        best_m = m;
-      }
+      if (best_n <= 0 || nph >= kMaxPh) return false;
+      for (int o = 0; o < nops; o++)
+        if ((best >> o) & 1) {
+          ph_of[o] = nph;
+          exec[ne++] = o;
+        }
+      ph_mask[nph++] = best_m;
+      cur = best_m;
+      done |= best;
     }
-    if (best_n <= 0 || nph >= kMaxPh) return BT_ERR_UNSUPPORTED;
-    for (int o = 0; o < nops; o++)
-      if ((best >> o) & 1) {
-        ph_of[o] = nph;
-        exec[ne++] = o;
+  };
+  bool ok = split(lin);
+  if (lin) {
+    // Relabelling ends a phase, so it can cost more than it saves.  A phase
+    // (an image round trip and a barrier) is 1.5 straight-line operators, an
+    // operator behind the phase's opening two (the dispatch moves the
+    // registers).
+    auto cost = [&]() {
+      int c = 0;
+      for (int p = 0; p < nph; p++) {
+        int n = 0;
+        uint32_t first = 0;
+        for (int e = 0; e < ne; e++)
+          if (ph_of[exec[e]] == p) {
+            const bool open = n == 0 || (n == 1 && !(first & opm[exec[e]]));
+            c += open ? 2 : 4;
+            first |= opm[exec[e]];
+            n++;
+          }
+        c += 3;
       }
-    ph_mask[nph++] = best_m;
-    cur = best_m;
-    done |= best;
+      return c + (lin_at[nph] ? 2 : 0);
+    };
+    const int with = ok ? cost() : 1 << 30;
+    if (split(0) && cost() <= with) lin = 0;
+    else ok = split(lin);
+    if (!lin) ok = true;
   }
+  if (!ok) return BT_ERR_UNSUPPORTED;
   uint32_t redm = 0;
   if (plan.red == bti::RED_RHO && plan.red_k == 3) {
     // read from the tile image in LDS after the last phase: no register
@@ -362,7 +457,7 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     // anyway, so the order is free: an opening pair of disjoint two-bit
     // operators goes to positions (2,3) then (0,1) and a lone opening pair to
     // (0,1): the straight-line templates.
-    if (p > 0 && ph_mask[p] == ph_mask[p - 1]) {
+    if (p > 0 && ph_mask[p] == ph_mask[p - 1] && !lin_at[p]) {
       for (int j = 0; j < kRB; j++) g->ph[p].rb[j] = g->ph[p - 1].rb[j];
       continue;
     }
@@ -389,6 +484,19 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     put(ph_mask[p]);  // the rest, ascending
     if (cnt == n) set_layout(g->ph[p].rb, order, n);
   }
+  // A relabelling in front of a phase (or the store) needs the image even
+  // between equal layouts: the register order says so.
+  auto differ = [&](int8_t* rb, const int8_t* from) {
+    bool same = true;
+    for (int j = 0; j < kRB; j++) same = same && rb[j] == from[j];
+    if (same) {
+      const int8_t t = rb[0];
+      rb[0] = rb[1];
+      rb[1] = t;
+    }
+  };
+  for (int p = 1; p < nph; p++)
+    if (lin_at[p]) differ(g->ph[p].rb, g->ph[p - 1].rb);
   g->nph = nph;
   // load/store layouts: the top local bits in registers, unless the first /
   // last phase's layout holds at most two of the lowest four local bits in
@@ -400,10 +508,12 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     set_layout(g->io_in, bits, n);
     set_layout(g->io_out, bits, n);
     const uint32_t low = (1u << (g->tb < 4 ? g->tb : 4)) - 1u;
-    if (nph > 0 && popc32(ph_mask[0] & low) <= 2)
+    if (nph > 0 && popc32(ph_mask[0] & low) <= 2 && !lin_at[0])
       for (int j = 0; j < kRB; j++) g->io_in[j] = g->ph[0].rb[j];
-    if (nph > 0 && popc32(ph_mask[nph - 1] & low) <= 2)
+    if (nph > 0 && popc32(ph_mask[nph - 1] & low) <= 2 && !lin_at[nph])
       for (int j = 0; j < kRB; j++) g->io_out[j] = g->ph[nph - 1].rb[j];
+    if (nph > 0 && lin_at[0]) differ(g->io_in, g->ph[0].rb);
+    if (lin_at[nph]) differ(g->io_out, nph > 0 ? g->ph[nph - 1].rb : g->io_in);
     // a histogram is cheapest when its bits stay off the store layout's
     // registers: each thread's 2^RB amplitudes then share one bin per tile
     g->hist_fast = 0;
@@ -437,8 +547,8 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
   //    permuted to the ascending position convention (index bit j <-> j-th
   //    lowest position)
   int moff = 0, nstage = 0;
-  g->nops = plan.nops;
-  for (int e = 0; e < plan.nops; e++) {
+  g->nops = ne;
+  for (int e = 0; e < ne; e++) {
     const int o = exec[e];
     const QOp& q = slots[plan.qidx[o]];
     const RPhase& ph = g->ph[ph_of[o]];
@@ -537,7 +647,7 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
   // the input scale rides on the first operator that every amplitude of
   // every tile goes through (no out-of-tile control), sparing the per-tile
   // multiply of each register
-  for (int e = 0; e < plan.nops && g->scale != 1.0; e++) {
+  for (int e = 0; e < ne && g->scale != 1.0; e++) {
     const ROp& r = g->ops[e];
     if (r.gctrl) continue;
     const int D2 = 1 << r.k;
@@ -574,9 +684,24 @@ __host__ __device__ __attribute__((noinline)) int build_geom(const Plan& plan, c
     if (g->io_out[j] != last_rb[j]) g->out_direct = 0;
   }
   g->outside = (nbits < 64 ? (1ull << nbits) - 1ull : ~0ull) & ~tmask;
-  for (int p = 0; p < nph; p++) make_slots<R>(g->ph[p].rb, T, &g->lay[p]);
-  make_slots<R>(g->io_in, T, &g->lay[kLayIn]);
-  make_slots<R>(g->io_out, T, &g->lay[kLayOut]);
+  uint32_t at[bti::kMaxT];
+  for (int b = 0; b < T; b++) at[b] = 1u << b;
+  make_slots<R>(g->io_in, T, at, &g->lay[kLayIn]);
+  make_slots<R>(g->io_out, T, at, &g->lay[kLayEnd]);
+  for (int p = 0; p <= nph; p++) {
+    for (int o = 0; o < nops; o++)
+      if ((lin_at[p] >> o) & 1) {
+        const int x = lbits[o][0], y = lbits[o][1];  // operand 0 = bit 1 of the operand index
+        const uint32_t ax = at[x], ay = at[y];
+        at[x] = (inv2[o][2] & 2 ? ax : 0) ^ (inv2[o][2] & 1 ? ay : 0);
+        at[y] = (inv2[o][1] & 2 ? ax : 0) ^ (inv2[o][1] & 1 ? ay : 0);
+      }
+    if (p < nph) make_slots<R>(g->ph[p].rb, T, at, &g->lay[p]);
+    else make_slots<R>(g->io_out, T, at, &g->lay[kLayOut]);
+  }
+  g->relabel = 0;
+  for (int b = 0; b < T; b++)
+    if (at[b] != 1u << b) g->relabel = 1;
   // 5. reductions
   if (plan.red == bti::RED_HIST) {
     for (int i = 0; i < plan.red_k; i++) g->red_bits[i] = plan.red_bits[i];
@@ -2021,6 +2146,13 @@ __device__ __forceinline__ void one_tile_passes(C<R>* __restrict__ state, const 
       phase_ops<R>(v, gp, p, 0, T, ops, lds, tid, ltid, active, nvalid_mask);
       image_write<R>(v, lds, gp, p, tid, active, nvalid_mask);
       if (p + 1 < nph || last) __syncthreads();
+    }
+    if (!last && BT_G(relabel)) {  // the next pass finds a plain image
+      __syncthreads();
+      C<R> v[NR];
+      image_read<R>(v, lds, geo, kLayOut, ltid);
+      __syncthreads();
+      image_write<R>(v, lds, geo, kLayEnd, tid, active, nvalid_mask);
     }
     if (last) {
       C<R> v[NR];
