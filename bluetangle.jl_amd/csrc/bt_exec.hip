@@ -225,10 +225,15 @@ int default_tile_bits(int prec) {
 // a tenth measured after each of 32 layers, 339 / 325 / 335 ms in 72 / 58
 // passes each; one trajectory of 12 layers 1.24 / 1.18 / 1.24 ms; complex128
 // at 3 / 2: 1.84 / 1.67 ms).  Full passes prefer the longer runs (30 qubits,
-// 2 layers: 19.3 / 20.8 ms).
-int coalesce_bits(int prec, bool deciding) {
+// 2 layers: 19.3 / 20.8 ms), except where the state stays in the caches: up
+// to 2^17 amplitudes at 2 bits (density matrices of 8 qubits, 16 layers,
+// complex64 at 4 / 2 bits 350 / 324 us, complex128 at 3 / 2 235 / 224 us, of
+// 7 qubits 285 / 275 us; state vectors level; from 2^18 up level, then slower).
+int coalesce_bits(int prec, bool deciding, int nbits) {
   const int p = prec == BT_C64 ? 0 : 1;
-  return g_coalesce_override[p] ? g_coalesce_override[p] : (prec == BT_C64 ? 4 : 3) - (deciding ? 1 : 0);
+  if (g_coalesce_override[p]) return g_coalesce_override[p];
+  const int c = (prec == BT_C64 ? 4 : 3) - (deciding ? 1 : 0);
+  return !deciding && nbits <= 17 ? std::min(c, 2) : c;
 }
 
 int tile_bits_for(int prec, int nbits) {
@@ -338,7 +343,7 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
   std::unique_ptr<bti::Interp> ip(new bti::Interp());
   bti::Program prog{ch.ops.data(), ch.ntop, ch.pool.data(), ch.chan.data(), ch.chanw.data(), nbits};
   const int T = prec_tile_T;
-  ip->init(prog, slots.data(), T, coalesce_bits(s->prec, btc::decides(ch)));
+  ip->init(prog, slots.data(), T, coalesce_bits(s->prec, btc::decides(ch), nbits));
   ip->stream = 1;
   ip->seed = seed;
   ip->traj = traj;
@@ -442,7 +447,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
   std::vector<QOp> slots(bti::kQMax);
   std::unique_ptr<bti::Interp> ip(new bti::Interp());
   bti::Program prog{ch.ops.data(), ch.ntop, ch.pool.data(), ch.chan.data(), ch.chanw.data(), nbits};
-  ip->init(prog, slots.data(), T, coalesce_bits(s->prec, false));
+  ip->init(prog, slots.data(), T, coalesce_bits(s->prec, false, nbits));
   ip->stream = 1;
   ip->fold = 0;
   tables->clear();
@@ -510,7 +515,7 @@ int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double
 // copied out for this run.
 static int static_plan(bt_state_s* s, bt_circuit_s* c, bool dm, int T, std::vector<unsigned char>* tables,
                        std::vector<uint8_t>* narrow, size_t* tabsz, bool* phases) {
-  const int cb = coalesce_bits(s->prec, false);
+  const int cb = coalesce_bits(s->prec, false, s->nbits);
   std::lock_guard<std::mutex> lk(c->mu);
   bt_circuit_s::StaticPlan* P = dm ? &c->dm_plan : &c->sv_plan;
   if (P->T != T || P->prec != s->prec || P->cb != cb) {
@@ -646,10 +651,9 @@ void grid_pass_lds_attr(int prec, int T) {
 // kMaxQK bits of vec(rho), so a smaller tile setting is raised to hold it.
 // Small complex64 density matrices (vec(rho) of at most 2^20 entries,
 // N <= 10) run on tiles of at most 2^12 entries: half the LDS per
-// workgroup, so twice the workgroups per CU and per state, for the 16 x 16
-// superoperators applied in LDS (measured on noisy brickworks, 16 layers:
-// N = 8 2.99 vs 3.37 ms, N = 10 3.94 vs 4.57 ms per circuit; from N = 11 up
-// 2^13-entry tiles are faster).  A smaller tile setting is kept.
+// workgroup, so twice the workgroups per CU and per state (noisy brickworks:
+// N = 8, 16 layers 324 vs 332 us; N = 7, 9 and 10 level; N = 11, 4 layers 466
+// vs 331 us the other way).  A smaller tile setting is kept.
 int dm_tile_bits_for(int prec, int nbits) {
   int T = tile_bits_for(prec, nbits);
   if (prec == BT_C64 && nbits <= 20) T = std::min(T, 12);
@@ -860,7 +864,7 @@ int bt_run_batch_persistent(bt_circuit c, int prec, uint64_t seed, int64_t traj0
   a.prog = bti::Program{c->d_ops, c->h.ntop, c->d_pool, c->d_chan, c->d_chanw, nbits};
   a.nbits = nbits;
   a.T = T;
-  a.cmin = coalesce_bits(prec, false);
+  a.cmin = coalesce_bits(prec, false, 64);
   a.want_final = final_states ? 1 : 0;
   a.seed = seed;
   a.traj0 = traj0;
@@ -944,7 +948,7 @@ int bt_set_tuning(int prec, int tile_bits, int coalesce, int tiles_per_blk) {
 int bt_get_tuning(int prec, int* tile_bits, int* coalesce, int* tiles_per_blk) {
   if (prec != BT_C64 && prec != BT_C128) return fail(BT_ERR_ARG, "bad precision");
   if (tile_bits) *tile_bits = g_tile_override[prec] ? g_tile_override[prec] : default_tile_bits(prec);
-  if (coalesce) *coalesce = coalesce_bits(prec, false);
+  if (coalesce) *coalesce = coalesce_bits(prec, false, 64);
   if (tiles_per_blk) *tiles_per_blk = tiles_per_block();
   return BT_OK;
 }

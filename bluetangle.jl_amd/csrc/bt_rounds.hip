@@ -40,7 +40,7 @@
 namespace bt {
 
 int tile_bits_for(int prec, int nbits);
-int coalesce_bits(int prec, bool deciding);
+int coalesce_bits(int prec, bool deciding, int nbits);
 int tiles_per_block();
 int item_tpb(int setting, uint64_t ntiles, int cap_div);
 
@@ -278,7 +278,7 @@ class RoundEngine {
     // density-matrix jobs (no norm folding): a superoperator spans up to
     // kMaxQK bits of vec(rho), so a smaller tile setting is raised to hold it
     const int T = j->fold ? tile_T(j->nbits) : dm_tile_bits_for(prec_, j->nbits);
-    j->ip->init(prog, j->slots.get(), T, coalesce_bits(prec_, btc::decides(*j->circ)));
+    j->ip->init(prog, j->slots.get(), T, coalesce_bits(prec_, btc::decides(*j->circ), j->nbits));
     j->ip->stream = 1;
     j->ip->seed = j->seed;
     j->ip->traj = j->traj;

@@ -290,9 +290,9 @@ int bt_set_tile_bits(int prec, int tile_bits);
 
 /* Tuning of the circuit executors (process-wide, per precision): tile bits,
  * low global bits every tile keeps for coalescing (a pass keeps one more when
- * its operators still fit; by default one fewer in circuits that decide
- * branches), tiles per workgroup of the rounds executor; 0 restores a
- * default. */
+ * its operators still fit; by default fewer in circuits that decide branches
+ * and for states that stay in the caches), tiles per workgroup of the rounds
+ * executor; 0 restores a default. */
 typedef struct {
   int32_t tile_bits;
   int32_t coalesce_bits;
