@@ -155,6 +155,12 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_grid_pass
   if (out) item_finish<NT>(sums, red, part, blockIdx.x, gridDim.x, count, out, nacc);
 }
 
+// Pass tables from pinned host memory to the device (16-byte words).
+__global__ void __launch_bounds__(256) k_stage(const uint4* src, uint4* dst, uint64_t words) {
+  const uint64_t step = (uint64_t)gridDim.x * 256;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < words; i += step) dst[i] = src[i];
+}
+
 // All passes of a state that is one tile in one launch (static plans: no
 // reductions): the launches between them, their cold tables and the trip of
 // the tile through memory cost more than a third of a 12-qubit circuit.
@@ -239,6 +245,24 @@ int coalesce_bits(int prec, bool deciding, int nbits) {
 int tile_bits_for(int prec, int nbits) {
   int T = g_tile_override[prec] ? g_tile_override[prec] : default_tile_bits(prec);
   return std::min(T, nbits);
+}
+
+// Enqueue the copy of `bytes` (rounded up to 16) from pinned host memory.  A
+// few KiB of tables in front of a pass: by a kernel the pass follows at once;
+// the runtime's copy took 4 us and left the device idle for 6 more (a kept
+// plan of a 12-qubit circuit 221 -> 192 us, of an 8-qubit density matrix 327
+// -> 312 us, a noisy 22-qubit trajectory 1182 -> 1157 us).  Past 1 MiB the
+// copy engine's rate matters more.
+int stage_copy(void* dst, const void* pinned, size_t bytes, hipStream_t stream) {
+  if (bytes > (1u << 20)) {
+    BT_HIP(hipMemcpyAsync(dst, pinned, bytes, hipMemcpyHostToDevice, stream));
+    return BT_OK;
+  }
+  const uint64_t words = (bytes + 15) / 16;
+  hipLaunchKernelGGL(k_stage, dim3((unsigned)std::max<uint64_t>(1, (words + 255) / 256)), dim3(256), 0, stream,
+                     (const uint4*)pinned, (uint4*)dst, words);
+  BT_HIP(hipGetLastError());
+  return BT_OK;
 }
 
 // Workgroups of a grid pass over ntiles tiles: eight per CU at most.
@@ -378,7 +402,7 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
       rc = fail(BT_ERR_STATE, "run_grid: pass limit exceeded");
       break;
     }
-    // the slot's previous table copy (this run's or an earlier one's) is done
+    // the pass that last used the slot (this run's or an earlier one's) is done
     const int slot = (int)(npass % kRing);
     if (hipEventSynchronize(ev[slot]) != hipSuccess) {
       rc = fail(BT_ERR_HIP, "run_grid: event sync");
@@ -394,11 +418,8 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
       break;
     }
     red_swap = head.red_swap;
-    if (hipMemcpyAsync(dslot, hslot, bytes, hipMemcpyHostToDevice, s->stream) != hipSuccess) {
-      rc = fail(BT_ERR_HIP, "run_grid: table copy");
-      break;
-    }
-    (void)hipEventRecord(ev[slot], s->stream);
+    rc = stage_copy(dslot, hslot, bytes, s->stream);
+    if (rc) break;
     // the host waits for a pass's sums only when a decision needs them or
     // the norm is folded into the next pass (fold = 0, a density matrix:
     // passes follow one another without a round trip)
@@ -414,12 +435,15 @@ static int run_grid(bt_state_s* s, const btc::CircuitHost& ch, uint64_t seed, ui
       to_result(plan, red_swap, h_acc, &res);
     } else {
       res.norm2 = 0.0;  // not used for an intermediate pass
+      (void)hipEventRecord(ev[slot], s->stream);  // a waited-for pass needs none
     }
   }
   if (rc == BT_OK && ip->err) rc = fail(ip->err, "interpreter error (" + std::to_string(ip->err) + ")");
   if (rc == BT_OK) {
     (void)hipEventRecord(e1, s->stream);
     if (hipStreamSynchronize(s->stream) != hipSuccess) rc = fail(BT_ERR_HIP, "run_grid: final sync");
+  } else {
+    (void)hipStreamSynchronize(s->stream);  // nothing reads the ring's slots any more
   }
   if (stats) {
     memset(stats, 0, sizeof *stats);
@@ -570,8 +594,8 @@ static int enqueue_static(bt_state_s* s, const std::vector<unsigned char>& table
     gr->tab_bytes = want;
   }
   memcpy(gr->h_tab, tables.data(), tables.size());
-  BT_HIP(hipMemcpyAsync(gr->d_tab, gr->h_tab, tables.size(), hipMemcpyHostToDevice, s->stream));
-  int rc = BT_OK;
+  int rc = stage_copy(gr->d_tab, gr->h_tab, tables.size(), s->stream);
+  if (rc) return rc;
   const int Tn = std::min(T, s->nbits);
   if (one_launch) {
     const int lds = (int)(((size_t)1 << Tn) * s->elem());

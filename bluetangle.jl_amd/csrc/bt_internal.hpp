@@ -122,6 +122,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
                        std::vector<uint8_t>* narrow, size_t* tabsz, bool* phases);
 int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part = nullptr,
                      unsigned* d_count = nullptr, double* out = nullptr, int nacc = 0);
+int stage_copy(void* dst, const void* pinned, size_t bytes, hipStream_t stream);
 void grid_pass_lds_attr(int prec, int T);
 int dm_tile_bits(bt_state_s* rho);              // tile bits of a density matrix's passes
 int dm_tile_bits_for(int prec, int nbits);      // the same for vec(rho) of nbits index bits

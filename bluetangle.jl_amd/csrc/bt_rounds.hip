@@ -389,7 +389,8 @@ class RoundEngine {
       blocks += it.nblocks;
       narrow = narrow && (prec_ == BT_C64 ? narrow_state<float>(j->nbits) : narrow_state<double>(j->nbits));
     }
-    BT_HIP(hipMemcpyAsync(d_blob_, h_blob_, used.load(), hipMemcpyHostToDevice, stream_));
+    rc = stage_copy(d_blob_, h_blob_, used.load(), stream_);
+    if (rc) return rc;
     // 3. launch
     const size_t lds = (size_t)(1ull << maxT) * elem();
     BT_HIP(hipEventRecord(ev_a_, stream_));
