@@ -193,7 +193,8 @@ int bt_state_create(int nqubits, int kind, int prec, bt_state* out) {
     }
   }
   const size_t part = sizeof(double) * kRedBlocks * kRedMax;
-  if (hipMalloc(&s->d_part, part + 16) != hipSuccess || hipMemset((char*)s->d_part + part, 0, 16) != hipSuccess ||
+  if (hipMalloc(&s->d_part, part + 4 * kCountWords) != hipSuccess ||
+      hipMemset((char*)s->d_part + part, 0, 4 * kCountWords) != hipSuccess ||
       hipHostMalloc(&s->h_out, sizeof(double) * kRedMax) != hipSuccess ||
       hipStreamCreate(&s->stream) != hipSuccess) {
     bt_state_destroy(s);

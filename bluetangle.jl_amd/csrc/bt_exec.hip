@@ -341,9 +341,9 @@ static int grid_res(bt_state_s* s, bool ring, GridRes** out) {
     const int cus = ctx().cus > 0 ? ctx().cus : 256;
     bool ok = hipHostMalloc(&g->h_ring, tabsz * kRing) == hipSuccess &&
               hipMalloc(&g->d_ring, tabsz * kRing) == hipSuccess &&
-              hipMalloc((void**)&g->d_part, sizeof(double) * kAcc * (size_t)cus * 8 + 16) == hipSuccess;
+              hipMalloc((void**)&g->d_part, sizeof(double) * kAcc * (size_t)cus * 8 + 4 * kCountWords) == hipSuccess;
     g->d_count = (unsigned*)(g->d_part + (size_t)kAcc * cus * 8);
-    ok = ok && hipMemset(g->d_count, 0, 16) == hipSuccess;
+    ok = ok && hipMemset(g->d_count, 0, 4 * kCountWords) == hipSuccess;
     for (int i = 0; i < kRing && ok; i++) ok = hipEventCreateWithFlags(&g->ev[i], hipEventDisableTiming) == hipSuccess;
     ok = ok && hipHostMalloc((void**)&g->h_acc, sizeof(double) * kAcc) == hipSuccess;
     if (!ok) {
@@ -508,7 +508,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
 
 // Enqueue one grid pass of state s (tile bits T) with its table at dtab;
 // out (pinned host memory, null: no sums are wanted) gets the pass's first
-// nacc sums; d_part: kAcc x grid doubles of partials, d_count: a zero.
+// nacc sums; d_part: kAcc x grid doubles of partials, d_count: kCountWords.
 int launch_grid_pass(bt_state_s* s, const void* dtab, bool narrow, int T, double* d_part, unsigned* d_count,
                      double* out, int nacc) {
   const int nbits = s->nbits;

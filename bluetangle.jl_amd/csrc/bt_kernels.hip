@@ -186,7 +186,7 @@ __device__ __forceinline__ void block_sums(const double (&acc)[M], double (*red)
 // 10 us of every call.
 struct ReduceOut {
   double* part;
-  unsigned* count;  // 0 between launches
+  unsigned* count;  // kCountWords, see count_last
   double* out;
 };
 
@@ -215,11 +215,9 @@ __device__ __forceinline__ bool reduce_finish(const double (*red)[M], const Redu
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials have reached the point of coherence
   __syncthreads();
-  if (threadIdx.x == 0)
-    last = __hip_atomic_fetch_add(o.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+  if (threadIdx.x == 0) last = count_last(o.count, blockIdx.x, nb);
   __syncthreads();
   if (!last) return false;
-  if (threadIdx.x == 0) __hip_atomic_store(o.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   double t = 0.0;
   if (j < M) {
     unsigned b = q;

@@ -63,7 +63,7 @@ struct RoundItem {
 // over its workgroups in a fixed order, do not depend on what else the
 // launch holds).  nb_uniform != 0: every item has that many workgroups (the
 // block -> item map is a division), else a binary search over the items'
-// first blocks.  Totals: count[item] (0 between launches), out + item * kAcc.
+// first blocks.  Totals: count + item * kCountWords, out + item * kAcc.
 template <typename R, typename O>
 __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_round(const RoundItem* items, int nitems, uint32_t nb_uniform,
                                                           double* part, unsigned* count, double* out) {
@@ -97,7 +97,8 @@ __global__ void __launch_bounds__(TileCfg<R>::NT, TileCfg<R>::WAVES) k_round(con
   const uint64_t t0 = (uint64_t)local * it.tpb;
   const uint64_t tend = std::min<uint64_t>((uint64_t)it.ntiles, t0 + it.tpb);
   tile_pass<R, O>((C<R>*)it.state, GeomConst(tab, sizeof(C<R>)), staged, tile, t0, 1, tend, red, sums, it.fresh);
-  item_finish<NT>(sums, red, part + (uint64_t)it.block0 * kAcc, local, it.nblocks, count + item,
+  item_finish<NT>(sums, red, part + (uint64_t)it.block0 * kAcc, local, it.nblocks,
+                  count + (uint64_t)item * kCountWords,
                   out + (uint64_t)item * kAcc, it.nacc);
 }
 
@@ -474,8 +475,8 @@ class RoundEngine {
       h_out_ = nullptr;
       const size_t cap = std::max(nitems, cap_items_ * 2);
       cap_items_ = 0;
-      BT_HIP(hipMalloc((void**)&d_count_, sizeof(unsigned) * cap));
-      BT_HIP(hipMemset(d_count_, 0, sizeof(unsigned) * cap));
+      BT_HIP(hipMalloc((void**)&d_count_, sizeof(unsigned) * kCountWords * cap));
+      BT_HIP(hipMemset(d_count_, 0, sizeof(unsigned) * kCountWords * cap));
       BT_HIP(hipHostMalloc((void**)&h_out_, sizeof(double) * kAcc * cap));
       cap_items_ = cap;
     }

@@ -1305,8 +1305,8 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
 // accumulator, each over every P-th workgroup, then a fixed tree) and writes
 // the totals to out (pinned host memory): no second launch and no copy.
 // The partials cross the XCDs' L2 caches: agent-scope stores, complete before
-// the state's count is raised, and agent-scope loads after it.  count is 0
-// between launches.  red: NT/64 doubles of LDS.  One noisy trajectory of 22
+// the state's count is raised, and agent-scope loads after it.  count:
+// kCountWords, see count_last.  red: NT/64 doubles of LDS.  One noisy trajectory of 22
 // qubits in 30 passes: 1.29 -> 1.25 ms against a totals launch and a copy.
 template <int NT>
 __device__ __forceinline__ void item_finish(const double* sums, double* red, double* part, uint32_t block,
@@ -1321,10 +1321,9 @@ __device__ __forceinline__ void item_finish(const double* sums, double* red, dou
     __hip_atomic_store(part + (uint64_t)tid * nb + block, sums[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials have reached the point of coherence
   __syncthreads();
-  if (tid == 0) last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+  if (tid == 0) last = count_last(count, block, nb);
   __syncthreads();
   if (!last) return;
-  if (tid == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // a power of two of threads per accumulator, 16 at least: a norm alone gets all
   const int P = nacc <= 1 ? NT : nacc <= 2 ? NT / 2 : nacc <= 5 ? NT / 8 : NT / 16;
   static_assert(NT == 256, "thread split of the totals");
