@@ -227,10 +227,10 @@ int default_tile_bits(int prec) {
 // wavefront access): 128 B for either precision.  deciding: a circuit whose
 // passes end where a branch is decided, with few operators each, keeps one
 // bit fewer: its tiles hold more of them and the fewer passes outweigh the
-// shorter runs (complex64 at 4 / 3 / 2 bits: 256 trajectories of 22 qubits,
-// a tenth measured after each of 32 layers, 339 / 325 / 335 ms in 72 / 58
-// passes each; one trajectory of 12 layers 1.24 / 1.18 / 1.24 ms; complex128
-// at 3 / 2: 1.84 / 1.67 ms).  Full passes prefer the longer runs (30 qubits,
+// shorter runs (complex64 at 4 / 3 bits: the passes of 512 trajectories of 22
+// qubits, a tenth measured after each of 32 layers, 620 / 584 ms, 72 / 58
+// each, 2 bits 3 % slower than 3; one trajectory of 12 layers 1.24 / 1.18 ms;
+// complex128 at 3 / 2: 1.84 / 1.67 ms).  Full passes prefer the longer runs (30 qubits,
 // 2 layers: 19.3 / 20.8 ms), except where the state stays in the caches: up
 // to 2^17 amplitudes at 2 bits (density matrices of 8 qubits, 16 layers,
 // complex64 at 4 / 2 bits 350 / 324 us, complex128 at 3 / 2 235 / 224 us, of
