@@ -488,6 +488,7 @@ int plan_static_passes(bt_state_s* s, const btc::CircuitHost& ch, int T, std::ve
   while (ip->step(&plan, &res)) {
     if (plan.red != bti::RED_NONE) return fail(BT_ERR_UNSUPPORTED, "plan_static_passes: a pass needs a reduction");
     if (++npass > max_passes) return fail(BT_ERR_STATE, "plan_static_passes: pass limit exceeded");
+    if (s->kind == BT_DM && s->prec == BT_C64) btc::settle_scales(plan, slots.data(), s->n);
     size_t bytes = 0;
     TableHead head;
     const int grc = pass_table(s->prec, plan, slots.data(), nbits, one.data(), &bytes, &head);
