@@ -76,44 +76,66 @@ __global__ void __launch_bounds__(256) k_chunk_sums(const C<R>* s, uint64_t n, u
   }
 }
 
-// Inclusive scan of x over the workgroup's 256 threads, fixed order; *total
-// gets the sum.
-__device__ __forceinline__ double block_scan(double x, double* total) {
-  __shared__ double wsum[4];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// Exclusive scan of x over the workgroup's 256 threads in two serial levels of
+// 16: *outer is the sum of the groups of 16 threads before this thread's,
+// *inner that of the threads before it in its group; returns the total.  With
+// serial sums, and prefixes added from the inside out (outer + (inner + own)),
+// the prefix after an entry is that before the next one, bit for bit: prefixes
+// never decrease, and an entry of 0 leaves them as they are.  A tree's prefixes
+// do not: an empty chunk's start could lie an ulp below the next chunk's, and
+// a target between the two found no probability in its chunk.  32 dependent
+// additions instead of a tree's 9: 8192 shots of 2^24 complex64 amplitudes
+// take 89.2 us a call (88.7 with the tree).
+__device__ __forceinline__ double block_scan(double x, double* outer, double* inner) {
+  __shared__ double v[16 * 17], g[16];
+  const int grp = threadIdx.x >> 4, at = grp * 17 + (threadIdx.x & 15);  // 17: off the same banks
+  __syncthreads();
+  v[at] = x;
+  __syncthreads();
+  if (threadIdx.x < 16) {
+    double t = 0.0;
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const double v = __shfl_up(x, o, 64);
-    if (lane >= o) x += v;
+    for (int i = 0; i < 16; i++) {
+      const double y = v[threadIdx.x * 17 + i];
+      v[threadIdx.x * 17 + i] = t;
+      t += y;
+    }
+    g[threadIdx.x] = t;
   }
   __syncthreads();
-  if (lane == 63) wsum[w] = x;
-  __syncthreads();
-  double before = 0.0;
-  for (int i = 0; i < w; i++) before += wsum[i];
-  *total = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
-  return before + x;
+  double total = 0.0, before = 0.0;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    if (i == grp) before = total;
+    total += g[i];
+  }
+  *outer = before;
+  *inner = v[at];
+  return total;
 }
 
 // pre[k]: sum of this workgroup's chunks before k (in place of the sums);
-// off[b]: sum of the workgroups before b, off[gridDim.x] = T.  One workgroup
-// over all chunks took 20 us at 8192 chunks and grew with them.
+// off[b]: sum of the workgroups before b, off[gridDim.x] = T.  The starts
+// off + pre never decrease and are equal up to the next chunk that holds
+// probability (see block_scan).  One workgroup over all chunks took 20 us at
+// 8192 chunks and grew with them.
 __global__ void __launch_bounds__(256) k_chunk_scan(double* pre, uint64_t nchunks, double* off, unsigned* count) {
   __shared__ int last;
   const uint64_t b0 = (uint64_t)blockIdx.x * kScanRun;
   constexpr int P = kScanRun / 256;  // consecutive chunks per thread
-  double x[P], mine = 0.0, total;
+  double x[P], mine = 0.0, outer, inner;
 #pragma unroll
   for (int i = 0; i < P; i++) {
     const uint64_t k = b0 + (uint64_t)threadIdx.x * P + i;
     x[i] = k < nchunks ? pre[k] : 0.0;
     mine += x[i];
   }
-  double run = block_scan(mine, &total) - mine;
+  const double total = block_scan(mine, &outer, &inner);
+  double run = 0.0;
 #pragma unroll
   for (int i = 0; i < P; i++) {
     const uint64_t k = b0 + (uint64_t)threadIdx.x * P + i;
-    if (k < nchunks) pre[k] = run;
+    if (k < nchunks) pre[k] = outer + (inner + run);
     run += x[i];
   }
   if (threadIdx.x == 0) {
@@ -124,18 +146,22 @@ __global__ void __launch_bounds__(256) k_chunk_scan(double* pre, uint64_t nchunk
   }
   __syncthreads();
   if (!last) return;
-  double base = 0.0;
-  for (unsigned b = 0; b < gridDim.x; b += 256) {
-    const unsigned k = b + threadIdx.x;
-    const double v =
-        k < gridDim.x ? __hip_atomic_load(off + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
-    double sum;
-    const double incl = block_scan(v, &sum);
-    __syncthreads();
-    if (k < gridDim.x) off[k] = base + (incl - v);
-    base += sum;
+  // the last workgroup scans the workgroups' totals the same way
+  const unsigned per = (gridDim.x + 255) / 256, r0 = threadIdx.x * per;
+  auto load = [&](unsigned k) {
+    return k < gridDim.x ? __hip_atomic_load(off + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+  };
+  mine = 0.0;
+  for (unsigned i = 0; i < per; i++) mine += load(r0 + i);
+  const double T = block_scan(mine, &outer, &inner);
+  run = 0.0;
+  for (unsigned i = 0; i < per; i++) {
+    const unsigned k = r0 + i;
+    const double y = load(k);
+    if (k < gridDim.x) off[k] = outer + (inner + run);
+    run += y;
   }
-  if (threadIdx.x == 0) off[gridDim.x] = base;
+  if (threadIdx.x == 0) off[gridDim.x] = T;
 }
 
 // Where a shot's uniform comes from: the caller's array, one value for all
@@ -383,9 +409,10 @@ static int sample_shots(bt_state_s* s, int64_t shots, const double* u, Uniforms 
 // ---------------------------------------------------------------------------
 // the no-allocation variant's scratch: one static device array per GPU
 // ---------------------------------------------------------------------------
-// Holds the chunk sums and prefix, the shots' uniforms, indices and boundary
-// flags, and the boundary count: 32 MiB covers a 2^30-amplitude state (8 MiB
-// of sums and prefix) with about 1.4 million shots.  In host code the array's
+// Holds the chunks' prefixes (in place of their sums), the runs' offsets and
+// the scan's counter, the shots' uniforms, indices and boundary flags, and the
+// boundary count: 32 MiB covers a 2^30-amplitude state (4 MiB of prefixes) with
+// about 1.7 million shots of 17 bytes.  In host code the array's
 // name is not a device address: kernels and copies take the address that
 // hipGetSymbolAddress returned for the current device (noalloc_setup).
 constexpr size_t kNoAllocScratch = 32ull << 20;

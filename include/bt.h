@@ -161,7 +161,7 @@ int bt_sample_stream(bt_state s, int64_t shots, uint64_t seed, uint64_t traj, ui
 /* bt_sample without any allocation: the same kernels, results and errors,
  * with every device buffer (chunk sums, prefix, uniforms, indices, flags) in
  * one static 32 MiB device array per GPU (a 2^30-amplitude state with about
- * 1.4 million shots fits; larger requests return BT_ERR_ARG).  No counterpart
+ * 1.7 million shots fits; larger requests return BT_ERR_ARG).  No counterpart
  * in the reference: for callers that cannot allocate (tight serving loops,
  * harnesses that forbid hipMalloc).  Calls on one GPU share the array: calls
  * that overlap on one GPU (states on different streams) race. */
