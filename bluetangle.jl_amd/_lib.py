@@ -15,11 +15,12 @@ LIB_PATH = os.path.join(_HERE, "libbt.so")
 BT_SV, BT_DM = 0, 1
 BT_C64, BT_C128 = 0, 1
 BT_BASIS_Z, BT_BASIS_X, BT_BASIS_Y, BT_BASIS_R = 0, 1, 2, 3
-BT_ERR_STATE = -6
+BT_ERR_NORM = -9
 BT_OP_GATE, BT_OP_CHANNEL, BT_OP_MEASURE, BT_OP_RESET, BT_OP_IF = 0, 1, 2, 3, 4
 
 ERRORS = {-1: "BT_ERR_ARG", -2: "BT_ERR_UNSUPPORTED", -3: "BT_ERR_HIP", -4: "BT_ERR_NOMEM", -5: "BT_ERR_DRAWS",
-          -6: "BT_ERR_STATE", -7: "BT_ERR_BUDGET", -8: "BT_ERR_NODEVICE"}
+          -6: "BT_ERR_STATE", -7: "BT_ERR_BUDGET", -8: "BT_ERR_NODEVICE",
+          -9: "BT_ERR_NORM"}
 
 # exported entry points of include/bt.h
 SYMBOLS = [

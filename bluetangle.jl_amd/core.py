@@ -392,7 +392,7 @@ def _apply_run(state, ops, noise, pars, rng, outs):
     n = ctypes.c_int64()
     rc = L.lib().bt_apply_ops(state.handle, arr, len(ir.ops), L.dptr(pool), pool.size // 2, L.dptr(u), draws,
                               L.iptr(got), got.size, ctypes.byref(n))
-    if rc == L.BT_ERR_STATE and draws:  # a state without a norm: op by op, on the draws already taken
+    if rc == L.BT_ERR_NORM:  # a state without a norm: op by op, on the draws already taken
         left = u.tolist()[::-1]
         for o in ops:
             _apply_one(state, o, noise, outs is not None, pars, lambda: left.pop() if left else rng(), outs)

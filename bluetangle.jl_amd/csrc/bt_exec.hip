@@ -770,8 +770,14 @@ int bt_apply_ops(bt_state s, const bt_ir_op* ops, int nops, const double* pool, 
     double n2 = 0;
     rc = launch_norm2(s, &n2);
     if (rc) return rc;
-    if (!(n2 > 0) || !std::isfinite(n2)) return fail(BT_ERR_STATE, "bt_apply_ops: the state has no norm");
-    return run_grid(s, ch, 0, 0, uniforms, nuni, outcomes, outcap, nout, nullptr, 1, T, n2);
+    if (!(n2 > 0) || !std::isfinite(n2)) return fail(BT_ERR_NORM, "bt_apply_ops: the state has no norm");
+    GridRes* gr = nullptr;
+    rc = grid_res(s, true, &gr);  // what run_grid allocates
+    if (rc) return rc;
+    rc = run_grid(s, ch, 0, 0, uniforms, nuni, outcomes, outcap, nout, nullptr, 1, T, n2);
+    // passes may have run: none of the codes that leave the state untouched
+    if (rc == BT_OK || rc == BT_ERR_HIP || rc == BT_ERR_STATE) return rc;
+    return fail(BT_ERR_STATE, "bt_apply_ops: stopped between operations: " + std::string(bt_last_error()));
   }
   std::vector<unsigned char> tables;
   std::vector<uint8_t> narrow;

@@ -40,6 +40,7 @@ extern "C" {
 #define BT_ERR_STATE (-6)
 #define BT_ERR_BUDGET (-7)
 #define BT_ERR_NODEVICE (-8)
+#define BT_ERR_NORM (-9) /* sampling asked of a state without a finite positive norm; the state is untouched */
 
 #define BT_SV 0
 #define BT_DM 1
@@ -94,8 +95,9 @@ int bt_apply_matrix(bt_state s, int k, const double* mat, const int* bits, uint6
  * Uniforms are consumed as the per-op entries consume theirs (one per channel
  * and measurement, two for BT_BASIS_R); probabilities are those of the state,
  * normalised or not.  Gates alone are enqueued on the state's stream like
- * bt_apply_matrix.  BT_ERR_STATE, with the state untouched, if sampling is
- * asked of a state without a finite positive norm. */
+ * bt_apply_matrix.  BT_ERR_ARG, BT_ERR_UNSUPPORTED, BT_ERR_NOMEM,
+ * BT_ERR_DRAWS and BT_ERR_NORM leave the state untouched; after any other
+ * error it may stand between two operations. */
 struct bt_ir_op_s;
 int bt_apply_ops(bt_state s, const struct bt_ir_op_s* ops, int nops, const double* pool, int64_t npool,
                  const double* uniforms, int64_t nuni, int* outcomes, int64_t outcap, int64_t* nout);
