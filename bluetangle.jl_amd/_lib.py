@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libbt.so")
 BT_SV, BT_DM = 0, 1
 BT_C64, BT_C128 = 0, 1
 BT_BASIS_Z, BT_BASIS_X, BT_BASIS_Y, BT_BASIS_R = 0, 1, 2, 3
-BT_ERR_NORM = -9
+BT_ERR_ARG, BT_ERR_UNSUPPORTED, BT_ERR_NOMEM, BT_ERR_NORM = -1, -2, -4, -9
 BT_OP_GATE, BT_OP_CHANNEL, BT_OP_MEASURE, BT_OP_RESET, BT_OP_IF = 0, 1, 2, 3, 4
 
 ERRORS = {-1: "BT_ERR_ARG", -2: "BT_ERR_UNSUPPORTED", -3: "BT_ERR_HIP", -4: "BT_ERR_NOMEM", -5: "BT_ERR_DRAWS",
@@ -27,7 +27,7 @@ SYMBOLS = [
     "bt_last_error", "bt_version", "bt_init", "bt_uniform",
     "bt_state_create", "bt_state_destroy", "bt_state_info", "bt_state_set_basis", "bt_state_copy",
     "bt_state_upload", "bt_state_download", "bt_state_device_ptr", "bt_state_sync", "bt_state_bytes",
-    "bt_apply_full", "bt_apply_ops", "bt_apply_fused5", "bt_run_fused", "bt_autotune_fused", "bt_inner", "bt_expect", "bt_expect_each", "bt_sample", "bt_sample_stream", "bt_sample_noalloc", "bt_run_batch_sample", "bt_graph_create_fused", "bt_graph_create_dm", "bt_graph_launch",
+    "bt_apply_full", "bt_apply_ops", "bt_apply_ops_drawn", "bt_apply_fused5", "bt_run_fused", "bt_autotune_fused", "bt_inner", "bt_expect", "bt_expect_each", "bt_sample", "bt_sample_stream", "bt_sample_noalloc", "bt_run_batch_sample", "bt_graph_create_fused", "bt_graph_create_dm", "bt_graph_launch",
     "bt_graph_passes", "bt_graph_destroy",
     "bt_apply_matrix", "bt_reduced_rho", "bt_apply_kraus_traj", "bt_apply_kraus_dm", "bt_measure", "bt_reset",
     "bt_probabilities", "bt_norm2", "bt_trace_purity", "bt_gather",
@@ -78,6 +78,8 @@ class Result(ctypes.Structure):
                 ("latency_ms", ctypes.c_double), ("queue_ms", ctypes.c_double)]
 
 
+DRAW = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.POINTER(ctypes.c_double))  # bt_draw
+
 _lib = None
 _lock = threading.Lock()
 
@@ -109,6 +111,8 @@ def lib():
             "bt_apply_full": (ctypes.c_int, [vp, dp]),
             "bt_apply_ops": (ctypes.c_int, [vp, ctypes.POINTER(IrOp), ctypes.c_int, dp, ctypes.c_int64, dp,
                                             ctypes.c_int64, ip, ctypes.c_int64, i64p]),
+            "bt_apply_ops_drawn": (ctypes.c_int, [vp, ctypes.POINTER(IrOp), ctypes.c_int, dp, ctypes.c_int64, DRAW, vp,
+                                                  ip, ctypes.c_int64, i64p]),
             "bt_apply_fused5": (ctypes.c_int, [vp, dp, ip]),
             "bt_inner": (ctypes.c_int, [vp, vp, dp, dp]),
             "bt_expect": (ctypes.c_int, [vp, ctypes.c_int, dp, ip, ctypes.c_uint64, ctypes.c_uint64, dp, dp]),

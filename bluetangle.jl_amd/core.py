@@ -376,27 +376,52 @@ def _run_op(x):
     return op if op.type == "🔬" or isinstance(op.mat, np.ndarray) else None
 
 
+# Errors of bt_apply_ops_drawn with nothing applied and nothing drawn: what a
+# run refuses (more than 64 Kraus operators, operations wider than a tile set by
+# hand, a state without a norm) the per-op entries may still take.
+_RUN_REFUSED = (L.BT_ERR_ARG, L.BT_ERR_UNSUPPORTED, L.BT_ERR_NOMEM, L.BT_ERR_NORM)
+
+
 def _apply_run(state, ops, noise, pars, rng, outs):
-    """`ops` in order by one bt_apply_ops call.  False, with the state and rng
-    untouched, if an op cannot be lowered (op by op then raises where it is)."""
+    """`ops` in order by one bt_apply_ops_drawn call.  False, with the state
+    and rng untouched, if the run is refused (op by op then raises where it is)."""
     from .circuit import compile_ir
     try:
         ir = compile_ir(ops, state.N, noise)
-    except (ValueError, TypeError):
+    except Exception:
         return False
-    draws = sum(0 if o.kind == L.BT_OP_GATE else 2 if o.basis == L.BT_BASIS_R and o.kind == L.BT_OP_MEASURE else 1
-                for o in ir.ops)
     arr, pool = ir.arrays()
-    u = np.array([rng() for _ in range(draws)] or [0.0], dtype=np.float64)
+    taken, stopped = [], []
+
+    def draw(_, n, u):
+        try:
+            for i in range(n):
+                taken.append(float(rng()))
+                u[i] = taken[i]
+        except BaseException as e:  # not through the C frames
+            stopped.append(e)
+            return 1
+        return 0
+
     got = np.zeros(max(len(ir.ops), 1), dtype=np.int32)
     n = ctypes.c_int64()
-    rc = L.lib().bt_apply_ops(state.handle, arr, len(ir.ops), L.dptr(pool), pool.size // 2, L.dptr(u), draws,
-                              L.iptr(got), got.size, ctypes.byref(n))
-    if rc == L.BT_ERR_NORM:  # a state without a norm: op by op, on the draws already taken
-        left = u.tolist()[::-1]
+    rc = L.lib().bt_apply_ops_drawn(state.handle, arr, len(ir.ops), L.dptr(pool), pool.size // 2, L.DRAW(draw), None,
+                                    L.iptr(got), got.size, ctypes.byref(n))
+    if stopped and not isinstance(stopped[0], Exception):
+        raise stopped[0]
+    if stopped:  # rng gave out: op by op up to where it did
+        left = taken[::-1]
+
+        def rest():
+            if not left:
+                raise stopped[0]
+            return left.pop()
+
         for o in ops:
-            _apply_one(state, o, noise, outs is not None, pars, lambda: left.pop() if left else rng(), outs)
+            _apply_one(state, o, noise, outs is not None, pars, rest, outs)
         return True
+    if rc in _RUN_REFUSED:
+        return False
     L.check(rc)
     if outs is not None:
         outs.extend(int(x) for x in got[: n.value])

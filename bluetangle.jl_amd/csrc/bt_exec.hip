@@ -748,8 +748,8 @@ int bt_run_circuit(bt_state s, bt_circuit c, uint64_t seed, uint64_t traj, const
   return run_static(s, tables, narrow, tabsz, phases, T, stats);
 }
 
-int bt_apply_ops(bt_state s, const bt_ir_op* ops, int nops, const double* pool, int64_t npool, const double* uniforms,
-                 int64_t nuni, int* outcomes, int64_t outcap, int64_t* nout) {
+int bt_apply_ops_drawn(bt_state s, const bt_ir_op* ops, int nops, const double* pool, int64_t npool, bt_draw draw,
+                       void* ctx, int* outcomes, int64_t outcap, int64_t* nout) {
   if (!s) return fail(BT_ERR_ARG, "null state");
   int rc = ensure_device();
   if (rc) return rc;
@@ -758,12 +758,14 @@ int bt_apply_ops(bt_state s, const bt_ir_op* ops, int nops, const double* pool, 
   std::string msg;
   rc = btc::analyze(s->n, ops, nops, nops, pool, npool, &ch, &msg);
   if (rc) return fail(rc, msg);
-  bool gates_only = true;
-  for (const bt_ir_op& op : ch.ops) gates_only = gates_only && op.kind == BT_OP_GATE;
-  if (nuni < ch.max_draws || (ch.max_draws > 0 && !uniforms))
-    return fail(BT_ERR_DRAWS, "too few uniforms for the operations");
-  if (nout) *nout = 0;
   const int T = tile_bits_for(s->prec, s->nbits);
+  bool gates_only = true;
+  for (const bt_ir_op& op : ch.ops) {
+    gates_only = gates_only && op.kind == BT_OP_GATE;
+    if (op.k > std::min(T, bti::kMaxQK))
+      return fail(BT_ERR_UNSUPPORTED, "bt_apply_ops: an operation is wider than a pass's tile or operators");
+  }
+  if (nout) *nout = 0;
   if (!gates_only) {
     // probabilities are those of the state as it is: the interpreter starts
     // from its norm
@@ -774,7 +776,10 @@ int bt_apply_ops(bt_state s, const bt_ir_op* ops, int nops, const double* pool, 
     GridRes* gr = nullptr;
     rc = grid_res(s, true, &gr);  // what run_grid allocates
     if (rc) return rc;
-    rc = run_grid(s, ch, 0, 0, uniforms, nuni, outcomes, outcap, nout, nullptr, 1, T, n2);
+    std::vector<double> u((size_t)ch.max_draws);
+    if (!u.empty() && (!draw || draw(ctx, (int64_t)u.size(), u.data())))
+      return fail(BT_ERR_DRAWS, "too few uniforms for the operations");
+    rc = run_grid(s, ch, 0, 0, u.data(), (int64_t)u.size(), outcomes, outcap, nout, nullptr, 1, T, n2);
     // passes may have run: none of the codes that leave the state untouched
     if (rc == BT_OK || rc == BT_ERR_HIP || rc == BT_ERR_STATE) return rc;
     return fail(BT_ERR_STATE, "bt_apply_ops: stopped between operations: " + std::string(bt_last_error()));
@@ -794,6 +799,21 @@ int bt_apply_ops(bt_state s, const bt_ir_op* ops, int nops, const double* pool, 
     trim_tables(gr);
   }
   return rc;
+}
+
+int bt_apply_ops(bt_state s, const bt_ir_op* ops, int nops, const double* pool, int64_t npool, const double* uniforms,
+                 int64_t nuni, int* outcomes, int64_t outcap, int64_t* nout) {
+  struct Given {
+    const double* u;
+    int64_t n;
+  } given{uniforms, nuni};
+  const bt_draw take = [](void* ctx, int64_t n, double* u) {
+    const Given* g = (const Given*)ctx;
+    if (!g->u || g->n < n) return 1;
+    memcpy(u, g->u, sizeof(double) * (size_t)n);
+    return 0;
+  };
+  return bt_apply_ops_drawn(s, ops, nops, pool, npool, take, &given, outcomes, outcap, nout);
 }
 
 int bt_run_circuit_dm(bt_state rho, bt_circuit c, bt_run_stats* stats) {

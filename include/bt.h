@@ -101,6 +101,12 @@ int bt_apply_matrix(bt_state s, int k, const double* mat, const int* bits, uint6
 struct bt_ir_op_s;
 int bt_apply_ops(bt_state s, const struct bt_ir_op_s* ops, int nops, const double* pool, int64_t npool,
                  const double* uniforms, int64_t nuni, int* outcomes, int64_t outcap, int64_t* nout);
+/* bt_apply_ops on uniforms that are taken once nothing can refuse the
+ * operations any more: draw(ctx, n, u) writes the next n uniforms to u.  If it
+ * returns nonzero nothing is applied (BT_ERR_DRAWS). */
+typedef int (*bt_draw)(void* ctx, int64_t n, double* u);
+int bt_apply_ops_drawn(bt_state s, const struct bt_ir_op_s* ops, int nops, const double* pool, int64_t npool,
+                       bt_draw draw, void* ctx, int* outcomes, int64_t outcap, int64_t* nout);
 /* OpF(name, mat) (struct.jl:716-720): psi <- M psi with a full 2^N x 2^N
  * matrix, column-major complex128; FP64 accumulation.  SV states only (the
  * reference's matrix OpF has no density-matrix method). */

@@ -56,3 +56,89 @@ def test_no_norm_has_a_code_of_its_own(bt, prec, value):
                               ctypes.byref(n))
     assert rc == -9 and n.value == 0
     assert np.array_equal(before, st.to_numpy(), equal_nan=True)
+
+
+class _Counted:
+    """A caller's own rng: the counter stream's draws, `most` of them."""
+
+    def __init__(self, bt, seed, most=10 ** 9):
+        self.stream, self.given, self.most = bt.UniformStream(seed), 0, most
+
+    def __call__(self):
+        if self.given == self.most:
+            raise StopIteration("no more draws")
+        self.given += 1
+        return self.stream()
+
+
+def _both_ways(bt, N, ops, prec, seed, most=10 ** 9):
+    """(error type, outcomes, draws, state) of the list and of its operations one by one."""
+    res = []
+    for one in (False, True):
+        st = bt.zero_state(N, prec)
+        rng, outs, err = _Counted(bt, seed, most), [], None
+        try:
+            if one:
+                for o in ops:
+                    outs += bt.apply(st, o, track_measurements=True, rng=rng)[1]
+            else:
+                outs = bt.apply(st, ops, track_measurements=True, rng=rng)[1]
+        except Exception as e:
+            err, outs = type(e), None
+        res.append((err, outs if err is None else None, rng.given, st.to_numpy()))
+    return res
+
+
+def _spread(bt, N):
+    return [bt.Op("RY(%g)" % (0.3 + 0.2 * i), 1 + i % N) for i in range(11)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["c64", "c128"])
+def test_channel_of_many_kraus_operators(bt, prec):
+    """65 Kraus operators are more than a circuit takes; the list goes op by op, on the same draws."""
+    N = 5
+    many = [np.eye(2) / np.sqrt(65)] * 65
+    ops = _spread(bt, N) + [bt.Op("MZ", 2), bt.OpQC("many", many, 3), bt.OpQC("amplitude_damping", 0.3, 1), bt.Op("MX", 3)]
+    for seed in range(4):
+        a, b = _both_ways(bt, N, ops, prec, seed)
+        assert a[:3] == b[:3] and a[0] is None and np.array_equal(a[3], b[3])
+
+
+@pytest.mark.gpu
+def test_operation_wider_than_the_tile(bt):
+    """Three-qubit channels under tiles of two bits: op by op, not half a run."""
+    N, L = 5, bt.core.L
+    k3 = [np.sqrt(0.9) * np.eye(8), np.sqrt(0.1) * np.kron(np.kron(bt.gate["X"], bt.gate["Z"]), bt.gate["Y"])]
+    ops = _spread(bt, N) + [bt.Op("MZ", 1), bt.OpQC("three", k3, 2), bt.Op("MZ", 4)]
+    L.check(L.lib().bt_set_tile_bits(1, 2))
+    try:
+        a, b = _both_ways(bt, N, ops, "c128", 3)
+    finally:
+        L.check(L.lib().bt_set_tile_bits(1, 0))
+    assert a[:3] == b[:3] and a[0] is None and np.array_equal(a[3], b[3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("most", [0, 1, 3])
+def test_rng_that_gives_out(bt, most):
+    """The operations before the draw that cannot be had are applied, and the rng's error is raised."""
+    N = 4
+    ops = _spread(bt, N) + [bt.OpQC("amplitude_damping", 0.2, 1), bt.Op("MZ", 2), bt.Op("H", 3), bt.OpQC("phase_damping", 0.3, 2),
+                            bt.Op("MY", 4)]
+    a, b = _both_ways(bt, N, ops, "c128", 1, most)
+    assert a[:3] == b[:3] and a[0] is StopIteration and np.array_equal(a[3], b[3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", ["qubit", "name", "model"])
+def test_draws_before_an_error(bt, bad):
+    """A list that raises at an operation has drawn for the ones before it only."""
+    N = 4
+    ops = _spread(bt, N) + [bt.Op("MZ", 2), bt.OpQC("amplitude_damping", 0.2, 1), bt.Op("H", 1)]
+    wrong = {"qubit": bt.Op("CNOT", 1, 9), "name": bt.Op("MZ", 3), "model": bt.OpQC("amplitude_damping", 0.1, 9)}[bad]
+    if bad == "name":
+        wrong.name = "MQ"
+    a, b = _both_ways(bt, N, ops + [wrong] + ops, "c128", 2)
+    assert a[:3] == b[:3] and a[0] is not None and a[2] == 2
+    assert np.abs(a[3] - b[3]).max() <= 1e-13
