@@ -359,6 +359,9 @@ def _apply_one(state, op, noise, track, pars, rng, outs):
 _RUN_MIN = 10
 _RUN_MIN_LARGE = 4
 _RUN_LARGE = 1 << 26
+# Most operations of a run: the tables of a gate-only run's passes (about 10 KB
+# for 24 operators) are held together, on the host and on the device.
+_RUN_MAX = 4096
 
 
 def _run_op(x):
@@ -436,7 +439,7 @@ def _apply_list(state, ops, noise, track, pars, rng, outs):
     i = 0
     while i < len(ops):
         run = []
-        while least <= len(ops) and i + len(run) < len(ops):
+        while least <= len(ops) and i + len(run) < len(ops) and len(run) < _RUN_MAX:
             op = _run_op(ops[i + len(run)])
             if op is None:
                 break

@@ -142,3 +142,16 @@ def test_draws_before_an_error(bt, bad):
     a, b = _both_ways(bt, N, ops + [wrong] + ops, "c128", 2)
     assert a[:3] == b[:3] and a[0] is not None and a[2] == 2
     assert np.abs(a[3] - b[3]).max() <= 1e-13
+
+
+def test_long_lists_are_several_runs(bt, monkeypatch):
+    """A run holds the tables of all its passes, so a list of any length is taken in pieces."""
+    from bluetangle_jl_amd import core
+    st = core.StateVector.__new__(core.StateVector)
+    st.N, st.prec, st.handle = 3, 1, None
+    seen = []
+    monkeypatch.setattr(core, "_apply_run", lambda state, run, *a: seen.extend([len(run)]) or True)
+    monkeypatch.setattr(core, "_apply_one", lambda state, op, *a: seen.append(op.name))
+    core._apply_list(st, [bt.Op("H", 1)] * 10000 + [bt.ifOp("MZ", 2, "X", "H")] + [bt.Op("H", 1)] * 4097, False, False,
+                     None, None, [])
+    assert seen == [4096, 4096, 1808, "MZ", 4096, "H"]
