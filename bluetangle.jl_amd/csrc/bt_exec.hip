@@ -999,7 +999,7 @@ int bt_set_tuning(int prec, int tile_bits, int coalesce, int tiles_per_blk) {
 int bt_get_tuning(int prec, int* tile_bits, int* coalesce, int* tiles_per_blk) {
   if (prec != BT_C64 && prec != BT_C128) return fail(BT_ERR_ARG, "bad precision");
   if (tile_bits) *tile_bits = g_tile_override[prec] ? g_tile_override[prec] : default_tile_bits(prec);
-  if (coalesce) *coalesce = coalesce_bits(prec, false, 64);
+  if (coalesce) *coalesce = coalesce_bits(prec, true, 64);
   if (tiles_per_blk) *tiles_per_blk = tiles_per_block();
   return BT_OK;
 }
@@ -1012,9 +1012,11 @@ int bt_get_tuning(int prec, int* tile_bits, int* coalesce, int* tiles_per_blk) {
 // weigh: pass tables staged into LDS, one partial sum each; a sample smaller
 // than the run underweights them).  Stage 2 times each distinct effective
 // value once (item_tpb: candidates the cap turns into the same launch are
-// one candidate) and installs and reports the effective value.  The first
-// failing run ends the search with its error and the previous tuning
-// restored.
+// one candidate) and installs and reports the effective value.  The reserve
+// that coalesce_bits gives the circuit is a candidate; where it wins the rule
+// stays in force, for this circuit and for others, instead of its value being
+// set for all of them.  The first failing run ends the search with its error
+// and the previous tuning restored.
 int bt_autotune_batch(bt_circuit c, int prec, int64_t sample, uint64_t seed, bt_tuning* best) {
   if (!c || !best) return fail(BT_ERR_ARG, "null circuit or result");
   if (prec != BT_C64 && prec != BT_C128) return fail(BT_ERR_ARG, "bad precision");
@@ -1033,19 +1035,25 @@ int bt_autotune_batch(bt_circuit c, int prec, int64_t sample, uint64_t seed, bt_
   std::vector<int64_t> nouts(sample2);
   double best_ms = -1;
   bt_tuning b{};
+  g_coalesce_override[p] = 0;
+  const int rule = coalesce_bits(prec, btc::decides(c->h), nb);
+  auto set = [&](int cb) { return cb == rule ? 0 : cb; };  // the override that gives cb
+  std::vector<int> cbs{rule};
+  for (int cb : {3, 4, 5})
+    if (cb != rule) cbs.push_back(cb);
   int rc = BT_OK;
   // rc keeps the first error: no candidate runs after it
   auto time_one = [&](int T, int cb, int tpb, int64_t n) -> double {
     if (rc) return -1.0;
     g_tile_override[p] = T;
-    g_coalesce_override[p] = cb;
+    g_coalesce_override[p] = set(cb);
     g_tpb_override = tpb;
     bt_run_stats st;
     rc = bt_run_batch(c, prec, seed, 0, n, outs.data(), outcap, nouts.data(), nullptr, &st);
     return rc ? -1.0 : st.kernel_ms / (double)n;
   };
   for (int T : Ts)
-    for (int cb : {3, 4, 5}) {
+    for (int cb : cbs) {
       if (rc) break;
       if (cb >= T) continue;
       const double ms = time_one(T, cb, 8, sample);
@@ -1086,7 +1094,7 @@ int bt_autotune_batch(bt_circuit c, int prec, int64_t sample, uint64_t seed, bt_
     return rc ? rc : fail(BT_ERR_STATE, "autotune: no candidate ran");
   }
   g_tile_override[p] = b.tile_bits;
-  g_coalesce_override[p] = b.coalesce_bits;
+  g_coalesce_override[p] = set(b.coalesce_bits);
   g_tpb_override = b.tiles_per_block;
   *best = b;
   return BT_OK;

@@ -307,11 +307,14 @@ typedef struct {
   int32_t tiles_per_block;
   double ms_per_traj;  /* autotune: device time per trajectory of the winner */
 } bt_tuning;
+/* bt_get_tuning's coalesce_bits: what was set, or else what circuits that
+ * decide branches (noisy trajectories) keep. */
 int bt_set_tuning(int prec, int tile_bits, int coalesce_bits, int tiles_per_block);
 int bt_get_tuning(int prec, int* tile_bits, int* coalesce_bits, int* tiles_per_block);
 /* Autotuner: runs `sample` trajectories of the circuit through bt_run_batch
- * for each candidate tile-bits / coalescing setting, then 4 x `sample` for
- * each tiles-per-workgroup candidate of the winner; keeps (and returns) the
+ * for each candidate tile-bits / coalescing setting (the circuit's default
+ * among them, which then stays a default), then 4 x `sample` for each
+ * tiles-per-workgroup candidate of the winner; keeps (and returns) the
  * fastest. */
 int bt_autotune_batch(bt_circuit c, int prec, int64_t sample, uint64_t seed, bt_tuning* best);
 
