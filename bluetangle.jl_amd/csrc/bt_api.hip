@@ -130,6 +130,10 @@ __global__ void k_clear_counts(unsigned* c, unsigned n) {
   for (unsigned i = threadIdx.x; i < n; i += blockDim.x) c[i] = 0;
 }
 
+void clear_counts(unsigned* count, hipStream_t stream) {
+  hipLaunchKernelGGL(k_clear_counts, dim3(1), dim3(256), 0, stream, count, (unsigned)kCountWords);
+}
+
 // y = M x, one thread per row; M column-major complex128 (a wavefront reads a
 // contiguous piece of each column), FP64 accumulation
 template <typename R>
@@ -205,8 +209,7 @@ int bt_state_create(int nqubits, int kind, int prec, bt_state* out) {
     return fail(BT_ERR_NOMEM, "allocation of state scratch failed");
   }
   s->d_count = (unsigned*)((char*)s->d_part + part);
-  // by a kernel in front of the first one: a synchronous clear cost 25 us per state
-  hipLaunchKernelGGL(k_clear_counts, dim3(1), dim3(256), 0, s->stream, s->d_count, (unsigned)kCountWords);
+  clear_counts(s->d_count, s->stream);
   rc = launch_set_basis(s, 0);
   if (rc) {
     bt_state_destroy(s);

@@ -282,9 +282,9 @@ constexpr size_t kTabKeep = 16ull << 20;
 struct GridRes {
   void* h_ring = nullptr;
   void* d_ring = nullptr;
-  double* d_part = nullptr;
+  double* d_part = nullptr;     // behind d_ring
   unsigned* d_count = nullptr;  // behind the partials
-  double* h_acc = nullptr;      // the finished sums (pinned, written by the pass)
+  double* h_acc = nullptr;      // the finished sums (pinned, written by the pass), behind h_ring
   // a static plan's tables: pinned and device, reused once the copy / the
   // launches that read them are done; at most kTabKeep bytes are kept
   void* h_tab = nullptr;
@@ -305,9 +305,7 @@ void free_grid_res(GridRes* g) {
   if (g->h_tab) (void)hipHostFree(g->h_tab);
   if (g->d_tab) (void)hipFree(g->d_tab);
   if (g->h_ring) (void)hipHostFree(g->h_ring);
-  if (g->h_acc) (void)hipHostFree(g->h_acc);
   if (g->d_ring) (void)hipFree(g->d_ring);
-  if (g->d_part) (void)hipFree(g->d_part);
   delete g;
 }
 
@@ -323,7 +321,9 @@ static bool pass_narrow(int prec, const TableHead& h) {
   return prec == BT_C64 ? narrow_io<float>(h) : narrow_io<double>(h);
 }
 
-// ring: also the rings and reduction buffers of run_grid
+// ring: also the rings and reduction buffers of run_grid, in one pinned and one
+// device allocation: a state's first run with decisions takes 45 us longer than
+// the next one (95 with four allocations and a synchronous clear)
 static int grid_res(bt_state_s* s, bool ring, GridRes** out) {
   if (!s->grid) {
     auto* g = new GridRes();
@@ -337,21 +337,23 @@ static int grid_res(bt_state_s* s, bool ring, GridRes** out) {
   }
   GridRes* g = s->grid;
   if (ring && !g->h_acc) {
-    const size_t tabsz = table_max(s->prec);
+    const size_t ring_bytes = (table_max(s->prec) * kRing + 255) / 256 * 256;
     const int cus = ctx().cus > 0 ? ctx().cus : 256;
-    bool ok = hipHostMalloc(&g->h_ring, tabsz * kRing) == hipSuccess &&
-              hipMalloc(&g->d_ring, tabsz * kRing) == hipSuccess &&
-              hipMalloc((void**)&g->d_part, sizeof(double) * kAcc * (size_t)cus * 8 + 4 * kCountWords) == hipSuccess;
-    g->d_count = (unsigned*)(g->d_part + (size_t)kAcc * cus * 8);
-    ok = ok && hipMemset(g->d_count, 0, 4 * kCountWords) == hipSuccess;
+    const size_t part = (size_t)kAcc * cus * 8;
+    bool ok = hipHostMalloc(&g->h_ring, ring_bytes + sizeof(double) * kAcc) == hipSuccess &&
+              hipMalloc(&g->d_ring, ring_bytes + sizeof(double) * part + sizeof(unsigned) * kCountWords) == hipSuccess;
     for (int i = 0; i < kRing && ok; i++) ok = hipEventCreateWithFlags(&g->ev[i], hipEventDisableTiming) == hipSuccess;
-    ok = ok && hipHostMalloc((void**)&g->h_acc, sizeof(double) * kAcc) == hipSuccess;
     if (!ok) {
       (void)hipGetLastError();
+      (void)hipStreamSynchronize(s->stream);  // an earlier run's tables may still be read
       free_grid_res(g);
       s->grid = nullptr;
       return fail(BT_ERR_NOMEM, "run_grid: allocation failed");
     }
+    g->d_part = (double*)((char*)g->d_ring + ring_bytes);
+    g->d_count = (unsigned*)(g->d_part + part);
+    clear_counts(g->d_count, s->stream);
+    g->h_acc = (double*)((char*)g->h_ring + ring_bytes);
   }
   *out = g;
   return BT_OK;

@@ -118,6 +118,9 @@ size_t release_cached_memory();
 // expectation of a 2^20-amplitude state 33 -> 23 us).
 constexpr unsigned kCountGroups = 32;
 constexpr size_t kCountWords = 16 * (1 + kCountGroups);  // unsigned, 0 between launches
+// Clear new counters by a kernel in front of the first launch that uses them:
+// a synchronous clear cost 25 us per state.
+void clear_counts(unsigned* count, hipStream_t stream);
 #if defined(__HIPCC__)
 // One thread of workgroup `block` of nb (1 or more), its results stored:
 // whether it is the last.
