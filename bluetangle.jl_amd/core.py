@@ -351,14 +351,23 @@ def _apply_one(state, op, noise, track, pars, rng, outs):
 
 
 # Runs of a list that go through bt_apply_ops (fused passes) instead of one
-# call per operation: of at least _RUN_MIN operations, or _RUN_MIN_LARGE where
-# the state is at least _RUN_LARGE bytes.  Measured, one call per gate against a
-# run: 8 gates 66 and 36 us on 2^12 complex128 amplitudes (a state's first run
-# adds 85 us: level from 10 gates on), 4 gates 155 and 64 us on 2^23, 94 gates
-# 35.8 and 1.4 ms on 2^27 complex64.
+# call per operation: of at least _RUN_MIN gates and channels, or _RUN_MIN_LARGE
+# where the state is at least _RUN_LARGE bytes.  Measurements and resets do not
+# count, and a run with any of them has to have _RUN_DECIDES more: it starts
+# with the state's norm, and each group of them ends a pass and is waited for
+# as the per-op calls are.  Measured, one call per operation / a run / a state's
+# first run, us:
+#   gates, 2^12 complex128          8: 95 / 52 / 88      10: 110 / 61 / 99
+#   a third of them channels        8: 130 / 93 / 150    10: 166 / 103 / 154
+#   gates with depolarizing noise   8: 348 / 145 / 183   10: 435 / 151 / 206
+#   gates and one MZ, 2^16 complex64   12: 134 / 149 / 205   17: 174 / 169 / 222
+#   gates, 2^23 complex64           4: 93 / 63 / 103     10: 209 / 112 / 157
+#   gates and one MZ, 2^23          4: 121 / 183 / 238   11: 255 / 242 / 296
+# and 94 gates on 2^27 complex64 35.8 ms / 1.4 ms.
 _RUN_MIN = 10
 _RUN_MIN_LARGE = 4
 _RUN_LARGE = 1 << 26
+_RUN_DECIDES = 6
 # Most operations of a run: the tables of a gate-only run's passes (about 10 KB
 # for 24 operators) are held together, on the host and on the device.
 _RUN_MAX = 4096
@@ -431,6 +440,12 @@ def _apply_run(state, ops, noise, pars, rng, outs):
     return True
 
 
+def _run_worth(run):
+    """Operations of a run that count towards its least length."""
+    n = sum(1 for o in run if o.type != "🔬" and o.name.upper() not in ("RES", "RESET"))
+    return n if n == len(run) else n - _RUN_DECIDES
+
+
 def _apply_list(state, ops, noise, track, pars, rng, outs):
     least = 1 << 62
     if isinstance(state, StateVector):
@@ -444,7 +459,7 @@ def _apply_list(state, ops, noise, track, pars, rng, outs):
             if op is None:
                 break
             run.append(op)
-        if len(run) >= least and _apply_run(state, run, noise, pars, rng, outs if track else None):
+        if len(run) >= least and _run_worth(run) >= least and _apply_run(state, run, noise, pars, rng, outs if track else None):
             i += len(run)
             continue
         for o in ops[i:i + max(len(run), 1)]:

@@ -155,3 +155,44 @@ def test_long_lists_are_several_runs(bt, monkeypatch):
     core._apply_list(st, [bt.Op("H", 1)] * 10000 + [bt.ifOp("MZ", 2, "X", "H")] + [bt.Op("H", 1)] * 4097, False, False,
                      None, None, [])
     assert seen == [4096, 4096, 1808, "MZ", 4096, "H"]
+
+
+def test_measurements_do_not_make_a_run(bt, monkeypatch):
+    """Short lists with measurements or resets are as fast op by op; gates and channels alone make a run of ten."""
+    from bluetangle_jl_amd import core
+    seen = []
+    monkeypatch.setattr(core, "_apply_run", lambda state, run, *a: seen.append(len(run)) or True)
+    monkeypatch.setattr(core, "_apply_one", lambda state, op, *a: seen.append(op.name))
+
+    def routes(N, ops):
+        st = core.StateVector.__new__(core.StateVector)
+        st.N, st.prec, st.handle = N, 0, None
+        seen.clear()
+        core._apply_list(st, ops, False, False, None, None, [])
+        return list(seen)
+
+    h, mz, res, damp = bt.Op("H", 1), bt.Op("MZ", 1), bt.Op("RES", 2), bt.OpQC("amplitude_damping", 0.1, 1)
+    assert routes(12, [h] * 10) == [10] and routes(12, [h] * 9) == ["H"] * 9
+    assert routes(12, [h] * 5 + [damp] * 5) == [10]
+    assert routes(12, [h] * 15 + [mz]) == ["H"] * 15 + ["MZ"] and routes(12, [h] * 16 + [mz] * 3) == [19]
+    assert routes(12, [res] + [h] * 15)[1:] == ["H"] * 15 and routes(12, [res] + [h] * 16) == [17]
+    assert routes(23, [h] * 4) == [4] and routes(23, [h] * 3) == ["H"] * 3
+    assert routes(23, [h] * 9 + [mz]) == ["H"] * 9 + ["MZ"] and routes(23, [h] * 10 + [mz]) == [11]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["c64", "c128"])
+def test_list_on_a_state_without_a_norm(bt, prec):
+    """A list long enough for a run, on a zero state: op by op, on the same draws."""
+    ops = [bt.Op("H", 1 + i % 3) for i in range(20)] + [bt.Op("MZ", 1), bt.Op("MR", 2), bt.OpQC("depolarizing", 0.1, 3)]
+    res = []
+    for one in (False, True):
+        st, rng, outs = bt.zero_state(3, prec), _Counted(bt, 3), []
+        st.upload(np.zeros(8))
+        if one:
+            for o in ops:
+                outs += bt.apply(st, o, track_measurements=True, rng=rng)[1]
+        else:
+            outs = bt.apply(st, ops, track_measurements=True, rng=rng)[1]
+        res.append((outs, rng.given, st.to_numpy()))
+    assert res[0][:2] == res[1][:2] and np.array_equal(res[0][2], res[1][2], equal_nan=True)
