@@ -301,9 +301,9 @@ inline bool split_superoperator(const std::vector<cd>& s16, std::vector<cd>* sa,
   // act on every qubit, so what they are off adds up over a circuit: with one
   // row and one column, A with the product's magnitude and B's largest entry 1,
   // the relative error of a density matrix against FP64 was (depolarizing
-  // noise and amplitude damping, 16 layers of 8 qubits) 5.6e-7 in complex64 and
-  // 9.1e-15 in complex128, the purity's up to 4.1e-7; this way 5.5e-7, 7.1e-15
-  // and 2.3e-7; with one 16 x 16 operator 6.7e-7, 7.6e-15 and 2.8e-7.
+  // noise and amplitude damping, 16 layers of 8 qubits, 32 circuits) 5.7e-7 in
+  // complex64, its purity's 3.3e-7, and 9.0e-15 in complex128; this way 5.5e-7,
+  // 1.9e-7 and 6.7e-15; with one 16 x 16 operator 6.7e-7, 1.1e-7 and 7.5e-15.
   using cl = std::complex<long double>;
   auto refine = [&](const std::vector<cl>& Y, bool rows) {
     std::vector<cl> X(16);
@@ -333,51 +333,71 @@ inline bool split_superoperator(const std::vector<cd>& s16, std::vector<cd>* sa,
   return true;
 }
 
+// What becomes of a one-qubit superoperator over [row, column] (16 complex
+// entries, column-major) that is held in FP32 at scale c.
+struct Held {
+  double off;    // how far its entries are from a multiple of the operator, squared and relative
+  double scale;  // which multiple: what it does to the size of a density matrix
+};
+inline Held held_in_single(const double* m, double size2, double trace, double c) {
+  // four sums each, so that they are not one chain of additions
+  double e[4] = {0, 0, 0, 0}, p[4] = {0, 0, 0, 0}, t = 0;
+  for (int j = 0; j < 32; j += 4) {
+    double d[4];
+    for (int i = 0; i < 4; i++) {
+      const double y = m[j + i] * c;
+      d[i] = (double)(float)y - y;
+      e[i] += d[i] * d[i];
+      p[i] += d[i] * m[j + i];
+    }
+    if (j == 0 || j == 24) t += d[0];  // rows 0 and 3 of columns 0 and 3: the trace of a diagonal input
+    if (j == 4 || j == 28) t += d[2];
+  }
+  const double s = ((p[0] + p[1]) + (p[2] + p[3])) / size2;  // the error along the operator
+  t -= s * trace;
+  return {((((e[0] + e[1]) + (e[2] + e[3])) - s * s * size2) + 8.0 * t * t) / (c * c), c + s};
+}
+
 // Complex64 passes over density matrices round their operators to FP32.  The
 // scale of an operator is free as long as a pass's scales multiply to one: of
 // the one-qubit superoperators (bits b and b + N) that FP32 does not hold as
 // they are, each but the last takes the scale, among a few next to the value
-// that undoes the others, at which its entries are nearest to FP32 numbers;
-// the sum of rows 0 and 3, which carries the trace, counts twice.  Two 4 x 4
-// operators per channel are more roundings than one 16 x 16; relative error against
-// FP64 with these scales / at scale 1 / with the 16 x 16 operators: 8 qubits, 16
-// layers 5.3e-7 / 5.5e-7 / 6.7e-7, 10 qubits, 4 layers 3.1e-7 / 3.3e-7 / 3.2e-7,
-// 12 qubits 3.5e-7 / 3.7e-7 / 3.7e-7; the trace's up to 2.0e-7 / 2.8e-7 / 1.2e-7,
-// 1.2e-7 / 3.1e-7 / 1.2e-7 and 1.0e-7 / 3.6e-7 / 0.9e-7.  16 scales cost a
-// circuit's first run 40 of 750 us (64: 190 us for another 2 to 3 % of the error).
+// that undoes the others, at which its entries are nearest to a multiple of
+// it, the trace above all; which multiple they are of is what the later ones
+// undo.  Two 4 x 4 operators per channel are more roundings than one 16 x 16, and an
+// error common to a circuit's operators adds up in the trace and the purity.
+// Against FP64, the 16 x 16 operators / the factors at scale 1 / this, 32 noisy
+// circuits each (means of the state's relative error, root mean squares of the
+// trace's and the purity's):
+//   8 qubits, 16 layers   6.7e-7 / 5.5e-7 / 5.3e-7   1.3e-7 / 1.8e-7 / 0.9e-7   1.1e-7 / 1.9e-7 / 1.1e-7
+//   10 qubits, 4 layers   3.3e-7 / 3.3e-7 / 3.1e-7   0.8e-7 / 1.3e-7 / 0.7e-7   0.8e-7 / 1.7e-7 / 1.2e-7
+//   12 qubits, 4 layers   3.6e-7 / 3.6e-7 / 3.5e-7   0.6e-7 / 1.3e-7 / 0.9e-7   0.9e-7 / 1.8e-7 / 1.0e-7
+// A circuit's first run takes up to 20 of 750 us longer for it.
 inline void settle_scales(const bti::Plan& plan, bti::QOp* slots, int N) {
-  constexpr int kScales = 16;
-  // squared error of q's entries at scale c, relative to them; at least `most` once it reaches that
-  auto error = [](const bti::QOp& q, double c, double most) {
-    double e = 0;
-    for (int col = 0; col < 4 && e < most * c * c; col++) {
-      double d[8];
-      for (int j = 0; j < 8; j++) {
-        const double y = q.m[8 * col + j] * c;
-        d[j] = (double)(float)y - y;
-        e += d[j] * d[j];
-      }
-      e += (d[0] + d[6]) * (d[0] + d[6]) + (d[1] + d[7]) * (d[1] + d[7]);
-    }
-    return e / (c * c);
-  };
+  constexpr int kScales = 8;
   bti::QOp* last = nullptr;
   double carry = 1.0;  // product of the scales taken
   for (int o = 0; o < plan.nops; o++) {
     bti::QOp& q = slots[plan.qidx[o]];
-    if (q.k != 2 || q.ctrl || std::abs(q.bits[0] - q.bits[1]) != N || !(error(q, 1.0, 1e300) > 0)) continue;
+    if (q.k != 2 || q.ctrl || std::abs(q.bits[0] - q.bits[1]) != N) continue;
+    if (std::all_of(q.m, q.m + 32, [](double x) { return (double)(float)x == x; })) continue;
     if (last) {
-      double least = 1e300, at = 1.0;
+      double* m = last->m;
+      double size2 = 0;
+      for (int j = 0; j < 32; j++) size2 += m[j] * m[j];
+      const double trace = (m[0] + m[6]) + (m[24] + m[30]);
+      Held best{1e300, 1.0};
+      double at = 1.0;
       for (int i = 0; i < kScales; i++) {
         const double c = (1.0 + ((i & 1) ? -1 : 1) * ((i + 1) / 2) * 0x1p-14) / carry;
-        const double e = error(*last, c, least);
-        if (e < least) {
-          least = e;
+        const Held h = held_in_single(m, size2, trace, c);
+        if (h.off < best.off) {
+          best = h;
           at = c;
         }
       }
-      for (int j = 0; j < 32; j++) last->m[j] *= at;
-      carry *= at;
+      for (int j = 0; j < 32; j++) m[j] *= at;
+      carry *= best.scale;
     }
     last = &q;
   }
