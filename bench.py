@@ -55,12 +55,12 @@ HBM_PEAK_GBS = 8000.0
 # k_round's measured HBM traffic / algorithmic bytes on this circuit, by the
 # tiling's coalescing bits (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated,
 # tilings 13,3,16 and 13,4,16); a tiling not in the table reports no traffic
-TRAFFIC_RATIO = {3: 1.125, 4: 1.000}
-# k_round's operator flops per algorithmic byte on this circuit at 3 coalescing
+TRAFFIC_RATIO = {3: 1.201, 4: 1.066}
+# k_round's operator flops per algorithmic byte on this circuit, by coalescing
 # bits: the register operators run as v_mfma_f32_4x4x1f32 (512 flop each;
 # rocprofv3 SQ_INSTS_VALU_MFMA_MOPS_F32 x 512 over the same launches'
 # algorithmic bytes), against the FP32 matrix-core peak
-MFMA_FLOP_PER_BYTE = {3: 11.505}
+MFMA_FLOP_PER_BYTE = {3: 11.461, 4: 9.195}
 MFMA_FP32_PEAK_TFLOPS = 157.3
 
 
@@ -325,7 +325,8 @@ def small_configs_leg(bt, args):
     gdiff = float(np.abs(rg.to_numpy() - r64.to_numpy()).max())
     out["c2"] = dict(N=c2["N"], dtype="complex64 (FP64 trace/purity)", layers=16, ms_per_circuit=round(dt * 1e3, 3),
                      max_entry_err_vs_fp64=err, trace=tr, purity=pu,
-                     note="bt_run_circuit_dm: gates as E rho E^dagger, channels as one superoperator pass each",
+                     note="bt_run_circuit_dm: gates as E rho E^dagger, channels as superoperators (a product two-qubit channel "
+                          "as one per qubit), many per pass",
                      graph_ms_per_circuit=round(dtg * 1e3, 3), graph_passes=graph.passes, graph_max_entry_diff=gdiff,
                      graph_note="the density-matrix passes captured once in a HIP graph (bt_graph_create_dm), "
                                 "replayed per circuit (reset + replay + FP64 trace and purity)")
@@ -681,7 +682,7 @@ def main():
                                 "flop_per_byte": fpb,
                                 "note": "the register operators' FP32 matrix-core work per algorithmic byte "
                                         "(rocprofv3 SQ_INSTS_VALU_MFMA_MOPS_F32 x 512, "
-                                        "profiles/k_round_c3_n22_4096traj.txt) against the FP32 MFMA peak"}},
+                                        "profiles/k_round_traffic_pmc.txt) against the FP32 MFMA peak"}},
     }
     out["precision"] = precision_leg(bt, c, args)
     log("precision", out["precision"])

@@ -990,8 +990,10 @@ namespace bt {
 
 // Up to this many probabilities k_probs writes to pinned host memory and the
 // caller's thread copies them; more go through the device buffer and the
-// runtime's copy to pageable memory, which cost 16 fetches of 2^6 to 2^17
-// probabilities 700 us instead of 520.
+// runtime's copy to pageable memory.  16 fetches of 2^6 to 2^17 probabilities
+// take 520 us this way, 700 the other; one of 2^19 293 and 323, 2^20 545 and
+// 625, 2^22 2978 and 3159: what is gained above the line is not worth pinning
+// 8 bytes per probability of the largest request.
 constexpr uint64_t kFetchPinned = 1u << 18;
 
 static size_t state_bytes(int kind, int prec, int nq) {
