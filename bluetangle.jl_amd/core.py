@@ -407,9 +407,9 @@ def _apply_run(state, ops, noise, pars, rng, outs):
 
     def draw(_, n, u):
         try:
-            for i in range(n):
+            for _ in range(n):
                 taken.append(float(rng()))
-                u[i] = taken[i]
+            ctypes.memmove(u, (ctypes.c_double * n)(*taken), 8 * n)
         except BaseException as e:  # not through the C frames
             stopped.append(e)
             return 1
@@ -442,7 +442,7 @@ def _apply_run(state, ops, noise, pars, rng, outs):
 
 def _run_worth(run):
     """Operations of a run that count towards its least length."""
-    n = sum(1 for o in run if o.type != "🔬" and o.name.upper() not in ("RES", "RESET"))
+    n = sum(1 for o in run if o.type != "🔬" and (type(o) is Op or o.name.upper() not in ("RES", "RESET")))
     return n if n == len(run) else n - _RUN_DECIDES
 
 
